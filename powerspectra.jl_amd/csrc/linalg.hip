@@ -52,25 +52,21 @@ void dgemm_dev(Ctx* c, int m, int n, int k, const double* dA, int64_t lda, const
 }
 
 // ---- LU with partial pivoting ---------------------------------------------
-// Right-looking blocked getrf.  Outer blocks of kLuPanel columns end with a
-// trailing update by rocBLAS (dtrsm + dgemm of depth kLuPanel).  Inside a
-// block, leaves of kLuLeaf columns are factored one column per launch: the
-// kernel picks the pivot from the candidates the previous launch published
-// (each with the candidate row's remaining leaf entries, so the pivot row
-// needs no dependent read), eliminates it from every other unflagged row of
-// the leaf and publishes the next column's candidates.  The rest of the
-// block is then updated by a dtrsm + dgemm of depth kLuLeaf.  Within a leaf
-// rows are not moved: the pivot row is flagged and left in place, so no
-// launch reads a row another workgroup writes.  After the leaf the pivot
-// sequence is turned into LAPACK's row interchanges (ipiv, 1-based) and
-// applied to every column, which leaves the matrix exactly as getrf's
-// physical swaps would.  Ties in |pivot| go to the smallest row index.  A
-// zero pivot column is skipped and reported (first one, 1-based), as getrf
-// does.  (A single cooperative launch per leaf with a grid barrier per
+// Right-looking blocked getrf.  Panels of kLuPanel columns end with a trailing
+// update by rocBLAS (dtrsm + dgemm of depth kLuPanel).  Inside a panel, leaves
+// of 8 to 32 columns are factored by one workgroup holding the leaf's rows in
+// registers (lu_leaf_wg), or, above kLuWgRowsMax rows, one column per launch
+// (lu_leaf_col).  Ties in |pivot| go to the smallest row index, NaN ranks
+// first, and a zero pivot column is skipped and reported (first one, 1-based),
+// as getrf does.  Within a leaf rows are not moved; after it the pivots become
+// LAPACK's row interchanges (ipiv, 1-based) and the leaf's net row movement,
+// applied to the panel's columns at once and to all others once per panel, as
+// the panel's net movement: the matrix ends exactly as getrf's physical swaps
+// leave it.  (A single cooperative launch per leaf with a grid barrier per
 // column measured slower: the cross-XCD barrier costs more than a launch.)
 constexpr int kLuLeaf = 32;
 constexpr int kLuPanel = 256;
-constexpr int kLuRows = 128;     // rows per workgroup in the leaf kernels (one per thread)
+constexpr int kLuRows = 128;     // rows per workgroup of the multi-workgroup leaf kernels
 
 struct LuWork {
   // per-workgroup pivot candidates, two buffers of cstride entries: the
@@ -86,11 +82,16 @@ struct LuWork {
   int* piv;           // the leaf's pivot rows (original positions)
   int* ipiv;          // LAPACK interchanges, 1-based, n entries
   int* info;          // first zero pivot column (1-based) or 0
-  // the leaf's net row movement: position mkey[k] receives the row at
-  // position mval[k], k < *nmove (at most 2 kLuLeaf)
+  // net row movements of the panel's leaves: position mkey[k] receives the row
+  // at position mval[k]; the leaf at panel column d with nc columns has the
+  // entries [2 d, 2 d + 2 nc), unused ones with key -1
   int* mkey;
   int* mval;
-  int* nmove;
+  // the panel's net movement as lu_panel_perm leaves it: entries [0, panel
+  // width) are the panel's own rows, in order, the others rows below it
+  int* pkey;
+  int* pval;
+  int* pcount;
 };
 
 // |x| for the pivot search; NaN ranks above everything, so a NaN column
@@ -245,96 +246,231 @@ __global__ void __launch_bounds__(kLuRows) lu_leaf_col(double* A, int64_t lda, i
   }
 }
 
-// The leaf factored by one workgroup when its rows fit in registers: 1024
-// threads, thread t holding rows c + t + 1024 k (k < NR) of the leaf's W
-// columns (kLuLeaf with one row per thread, kLuWgLeaf with more).  Per column: a workgroup argmax (ties to the lower row,
-// NaN first, as lu_better), the pivot row through LDS, and the elimination
-// of every other unpivoted row -- the arithmetic of lu_leaf_col, with two
-// barriers in place of a launch.  Rows stay in place; the pivots go to
-// w.piv for lu_leaf_ipiv and lu_leaf_move, as on the multi-workgroup path.
-constexpr int kLuWgLeaf = 16;
-constexpr int kLuWgThreads = 1024;
-constexpr int kLuWgRowsMax = 3 * kLuWgThreads;   // leaf rows one workgroup takes
+// The leaf factored by one workgroup that holds its rows in registers: thread
+// t has rows c + t + kLuWgThreads k (k < NR) of the leaf's W columns, NR x W
+// <= 96 doubles.  Per column: every wave takes its own maximum (DPP), its
+// winner copies its row to the wave's LDS slot, one barrier, and all waves
+// pick the best slot, whose row is already the pivot row.  The slots alternate
+// by column, so that barrier is the only one.  Eight waves of many rows rather
+// than sixteen of few: the search and the pivot choice cost a wave the same
+// whatever its rows, and two waves per SIMD already cover their latencies.
+//   The column at hand is always register 0: the update of column q + 1 writes
+// register q, so that one loop body serves eight columns and the code stays in
+// the instruction cache.  (Every column unrolled with static register indices
+// executes each instruction once a launch and is bound by fetching them.)
+// Multipliers are stored in place as they are made; pivot rows are kept in LDS
+// from their column on.  After the columns, wave 0 turns the pivots into
+// LAPACK's interchanges and the leaf's own columns are reordered.
+//   Measured: 42, 54 and 60 us a 32-column leaf of 512, 1024 and 1536 rows, 32
+// to 40 us a 16-column one of 2048 to 3072, 22 to 29 us an 8-column one of 4096
+// to 6144: 1.3 to 3.6 us a column, against 2.6 to 3.7 with 1024 threads and all
+// columns unrolled, and 5.7 for a launch per column above 3072 rows.  Device
+// solves: n = 2509 13.7 -> 7.5 ms, n = 6144 45.9 -> 28.3 ms.
+constexpr int kLuWgThreads = 512;
+constexpr int kLuWgWaves = kLuWgThreads / 64;
+constexpr int kLuWgRowsMax = 12 * kLuWgThreads;  // leaf rows one workgroup takes
+constexpr int kLuStage = 8;                       // columns per loop
 
-// LAPACK interchanges and net row movement of a leaf from its pivot rows, by
-// one wavefront (defined below).
-__device__ __forceinline__ void lu_leaf_ipiv_wave(int c, int nc, const int* piv, const LuWork& w);
+// x of another lane of the row (or x itself where the pattern has no source)
+template <int CTRL>
+__device__ __forceinline__ double lu_dpp(double x) {
+  const long long v = __double_as_longlong(x);
+  const int lo = (int)(v & 0xffffffffLL), hi = (int)(v >> 32);
+  const int l2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false);
+  const int h2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false);
+  return __longlong_as_double(((long long)h2 << 32) | (unsigned int)l2);
+}
 
-// One column step of lu_leaf_wg (J static, so every register index is).
-template <int NR, int W, int J>
-__device__ __forceinline__ void lu_wg_step(double (&vals)[NR][W], bool (&live)[NR],
-                                           int t, int c, int n, int nc, double* sv, int* sr,
-                                           double* u, int* spiv, const LuWork& w) {
-  if (J >= nc) return;  // uniform
-  const int lane = t & 63, wv = t >> 6;
-  double v = -1.0;
-  int r = 0x7fffffff;
+__device__ __forceinline__ double lu_lane(double x, int lane) {
+  const long long v = __double_as_longlong(x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(v & 0xffffffffLL), lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// max without the canonicalising moves fmax adds for values from lane moves
+__device__ __forceinline__ double lu_max(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// maximum over the wave (no NaN): four steps inside the 16-lane rows, two
+// across them, the result read from lane 63
+__device__ __forceinline__ double lu_wave_max(double v) {
+  v = lu_max(v, lu_dpp<0xB1>(v));    // quad_perm [1,0,3,2]
+  v = lu_max(v, lu_dpp<0x4E>(v));    // quad_perm [2,3,0,1]
+  v = lu_max(v, lu_dpp<0x124>(v));   // row_ror 4
+  v = lu_max(v, lu_dpp<0x128>(v));   // row_ror 8
+  v = lu_max(v, lu_dpp<0x142>(v));   // row_bcast 15
+  v = lu_max(v, lu_dpp<0x143>(v));   // row_bcast 31
+  return lu_lane(v, 63);
+}
+
+// Pivot slots of a column: each wave's winning row (from the column on) and
+// its value.
+template <int W>
+struct LuSlots {
+  double row[2][kLuWgWaves][W];
+  double mag[2][kLuWgWaves];
+  int pos[2][kLuWgWaves];
+};
+
+// Up to kLuStage columns from column j0 of the leaf on, WD columns still live
+// at its start (register q holds column j + q at step j).
+template <int NR, int W, int WD>
+__device__ __forceinline__ void lu_wg_stage(double (&vals)[NR][W], bool (&live)[NR], int t, int c,
+                                            int j0, int nc, double* A, int64_t lda,
+                                            LuSlots<W>& s, double (*P)[W], int* spiv,
+                                            const LuWork& w) {
+  const int lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int j1 = min(j0 + kLuStage, nc);
+#pragma unroll 1
+  for (int j = j0; j < j1; ++j) {
+    const int B = j & 1;
+    {
+      double v = -1.0;
+      bool nan = false;
 #pragma unroll
-  for (int k = 0; k < NR; ++k)
-    if (live[k]) lu_better(v, r, lu_mag(vals[k][J]), c + t + kLuWgThreads * k);
-  for (int o = 32; o >= 1; o >>= 1) lu_better(v, r, __shfl_xor(v, o), __shfl_xor(r, o));
-  if (lane == 0) {
-    sv[wv] = v;
-    sr[wv] = r;
-  }
-  __syncthreads();
-  // every wave combines the 16 wave winners: one LDS read per lane, then a
-  // 16-lane butterfly, and lane 0's result to all lanes
-  {
-    constexpr int kW = kLuWgThreads / 64;
-    v = lane < kW ? sv[lane] : -1.0;
-    r = lane < kW ? sr[lane] : 0x7fffffff;
-    for (int o = kW / 2; o >= 1; o >>= 1) lu_better(v, r, __shfl_xor(v, o), __shfl_xor(r, o));
-    r = __shfl(r, 0);
-  }
-  // a candidate always exists; the clamp keeps accesses in bounds regardless
-  const int p = r < n ? r : c + J;
-  // the pivot row's owner publishes its entries and drops out
+      for (int k = 0; k < NR; ++k) {
+        const double x = vals[k][0];
+        nan |= live[k] & (x != x);
+        v = lu_max(v, live[k] ? fabs(x) : -1.0);
+      }
+      double mx = lu_wave_max(v);
+      if (__builtin_amdgcn_ballot_w64(nan)) mx = INFINITY;
+      // the lowest row that reaches it: rows ascend with k, then with the lane
+      int kw = -1, lw = 0;
 #pragma unroll
-  for (int k = 0; k < NR; ++k) {
-    if (live[k] && c + t + kLuWgThreads * k == p) {
+      for (int k = NR - 1; k >= 0; --k) {
+        const unsigned long long m =
+            __builtin_amdgcn_ballot_w64(live[k] & !(fabs(vals[k][0]) < mx));
+        kw = m ? k : kw;
+        lw = m ? __builtin_ctzll(m) : lw;
+      }
 #pragma unroll
-      for (int jj = J; jj < W; ++jj)
-        if (jj < nc) u[jj] = vals[k][jj];
-      live[k] = false;
+      for (int k = 0; k < NR; ++k)
+        if (kw == k) {
+          if (lane == lw) {
+#pragma unroll
+            for (int q = 0; q < WD; ++q) s.row[B][wv][q] = vals[k][q];
+          }
+        }
+      if (lane == 0) {
+        s.mag[B][wv] = mx;
+        s.pos[B][wv] = kw < 0 ? 0x7fffffff : c + 64 * wv + lw + kLuWgThreads * kw;
+      }
+    }
+    __syncthreads();
+    const int sl = lane & (kLuWgWaves - 1);
+    const double mine = s.mag[B][sl];
+    const int pos = s.pos[B][sl];
+    double v = lu_max(mine, lu_dpp<0xB1>(mine));
+    v = lu_max(v, lu_dpp<0x4E>(v));
+    v = lu_max(v, lu_dpp<0x124>(v));     // 8 slots, repeated along the row
+    unsigned m = (unsigned)__builtin_amdgcn_ballot_w64(mine == v) & ((1u << kLuWgWaves) - 1);
+    int g = __builtin_ctz(m);
+    int p = __builtin_amdgcn_readlane(pos, g);
+    for (m &= m - 1; m; m &= m - 1) {    // equal magnitudes: the lower row
+      const int h = __builtin_ctz(m);
+      const int q = __builtin_amdgcn_readlane(pos, h);
+      if (q < p) {
+        p = q;
+        g = h;
+      }
+    }
+    // the pivot row: one entry per lane, then into scalar registers (a
+    // broadcast read of each would take the LDS a wave's whole return)
+    const double ul = s.row[B][g][lane & (W - 1)];
+    const double piv = lu_lane(ul, 0);
+    if (t < WD && j + t < W) P[j][j + t] = ul;
+    if (t == 0) {
+      spiv[j] = p;
+      if (piv == 0.0 && *w.info == 0) *w.info = c + j + 1;
+    }
+#pragma unroll
+    for (int k = 0; k < NR; ++k) live[k] &= c + t + kLuWgThreads * k != p;
+    double* a = A + (int64_t)(c + j) * lda + c + t;
+    // quotients by the rounded reciprocal with one residual correction: the
+    // correctly rounded quotient (|value| <= |pivot|); pivots whose reciprocal
+    // could leave the normal range are divided by, and under a zero pivot the
+    // column (all zeros) is left as it is
+    double l[NR];
+    if (__builtin_amdgcn_ballot_w64(fabs(piv) > 0x1p-1000 && fabs(piv) < 0x1p1000)) {
+      const double rp = 1.0 / piv;
+#pragma unroll
+      for (int k = 0; k < NR; ++k) {
+        const double q = vals[k][0] * rp;
+        l[k] = fma(fma(-q, piv, vals[k][0]), rp, q);
+      }
+    } else {
+      const double by = piv == 0.0 ? 1.0 : piv;
+#pragma unroll
+      for (int k = 0; k < NR; ++k) l[k] = vals[k][0] / by;
+    }
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+      if (live[k]) a[kLuWgThreads * k] = l[k];
+#pragma unroll
+    for (int q = 1; q < WD; ++q) {
+      const double u = lu_lane(ul, q);
+#pragma unroll
+      for (int k = 0; k < NR; ++k) vals[k][q - 1] = fma(-l[k], u, vals[k][q]);
     }
   }
-  __syncthreads();
-  const double piv = u[J];
-  if (t == 0) {
-    w.piv[J] = p;
-    spiv[J] = p;
-    if (piv == 0.0 && *w.info == 0) *w.info = c + J + 1;
-  }
-  if (piv != 0.0) {
-#pragma unroll
-    for (int k = 0; k < NR; ++k) {
-      if (live[k]) {  // the pivot rows are no longer live
-        const double l = vals[k][J] / piv;
-        vals[k][J] = l;
-#pragma unroll
-        for (int jj = J + 1; jj < W; ++jj)
-          if (jj < nc) vals[k][jj] = fma(-l, u[jj], vals[k][jj]);
+}
+
+// LAPACK interchanges and net row movement of a leaf from its pivot rows, by
+// one wavefront: at step j the row chosen (original position piv[j]) is
+// swapped with whatever row is at position c + j.  Only positions touched by
+// this leaf's swaps differ from the identity; they are kept as (position,
+// row) pairs, one pair per lane, found by ballot.  Returns the pair of this
+// lane (key -1: none).
+__device__ __forceinline__ int2 lu_leaf_ipiv_wave(int c, int nc, const int* piv, int* ipiv) {
+  const int lane = (int)(threadIdx.x & 63);
+  int key = -1, val = -1, m = 0;
+  for (int j = 0; j < nc; ++j) {
+    const int want = __builtin_amdgcn_readfirstlane(piv[j]);
+    const int pj = c + j;
+    const unsigned long long hv = __builtin_amdgcn_ballot_w64(key >= 0 && val == want);
+    const int q = hv ? __builtin_amdgcn_readlane(key, __builtin_ctzll(hv)) : want;
+    const unsigned long long hp = __builtin_amdgcn_ballot_w64(key == pj);
+    const int at_pj = hp ? __builtin_amdgcn_readlane(val, __builtin_ctzll(hp)) : pj;
+    if (lane == 0) ipiv[pj] = q + 1;
+    // position pj now holds `want`, position q the row that was at pj
+    if (hp) {
+      if (key == pj) val = want;
+    } else {
+      if (lane == m) {
+        key = pj;
+        val = want;
+      }
+      ++m;
+    }
+    if (q != pj) {
+      const unsigned long long hq = __builtin_amdgcn_ballot_w64(key == q);
+      if (hq) {
+        if (key == q) val = at_pj;
+      } else {
+        if (lane == m) {
+          key = q;
+          val = at_pj;
+        }
+        ++m;
       }
     }
   }
+  return make_int2(key, val);
 }
 
-template <int NR, int W, int... J>
-__device__ __forceinline__ void lu_wg_steps(double (&vals)[NR][W], bool (&live)[NR],
-                                            int t, int c, int n, int nc, double* sv, int* sr,
-                                            double* u, int* spiv, const LuWork& w,
-                                            std::integer_sequence<int, J...>) {
-  (lu_wg_step<NR, W, J>(vals, live, t, c, n, nc, sv, sr, u, spiv, w), ...);
-}
-
+// Leaf [c, cend) of the panel that starts at k0: see above.
 template <int NR, int W>
 __global__ void __launch_bounds__(kLuWgThreads) lu_leaf_wg(double* A, int64_t lda, int n, int c,
-                                                           int cend, LuWork w) {
-  __shared__ double sv[kLuWgThreads / 64];
-  __shared__ int sr[kLuWgThreads / 64];
-  __shared__ double u[W];
+                                                           int cend, int k0, LuWork w) {
+  __shared__ LuSlots<W> slots;
+  __shared__ double P[W][W];      // pivot row j from column j on
   __shared__ int spiv[W];
+  __shared__ int dest[W];         // where row c + i goes, or -1 for a pivot row
   const int t = threadIdx.x;
   const int nc = cend - c;
   double vals[NR][W];
@@ -347,105 +483,231 @@ __global__ void __launch_bounds__(kLuWgThreads) lu_leaf_wg(double* A, int64_t ld
     for (int jj = 0; jj < W; ++jj)
       vals[k][jj] = (live[k] && jj < nc) ? A[r + (int64_t)(c + jj) * lda] : 0.0;
   }
-  lu_wg_steps<NR, W>(vals, live, t, c, n, nc, sv, sr, u, spiv, w,
-                     std::make_integer_sequence<int, W>{});
-  // the leaf's interchanges and row movement (what lu_leaf_ipiv does on the
-  // other path), by wave 0 from the pivots in LDS
+  lu_wg_stage<NR, W, W>(vals, live, t, c, 0, nc, A, lda, slots, P, spiv, w);
+  if constexpr (W > kLuStage)
+    lu_wg_stage<NR, W, W - kLuStage>(vals, live, t, c, kLuStage, nc, A, lda, slots, P, spiv, w);
+  if constexpr (W > 2 * kLuStage) {
+    lu_wg_stage<NR, W, W - 2 * kLuStage>(vals, live, t, c, 2 * kLuStage, nc, A, lda, slots, P,
+                                         spiv, w);
+    lu_wg_stage<NR, W, W - 3 * kLuStage>(vals, live, t, c, 3 * kLuStage, nc, A, lda, slots, P,
+                                         spiv, w);
+  }
+  if (t < W) dest[t] = -1;
   __syncthreads();
-  if (t < 64) lu_leaf_ipiv_wave(c, nc, spiv, w);
-  // pivot rows keep the values they had when chosen
+  if (t < 64) {
+    const int2 mv = lu_leaf_ipiv_wave(c, nc, spiv, w.ipiv);
+    // rows that leave [c, cend): the positions below it that changed
+    if (mv.x >= cend) dest[mv.y - c] = mv.x;
+  }
+  __syncthreads();
+  int* const mkey = w.mkey + 2 * (c - k0);
+  int* const mval = w.mval + 2 * (c - k0);
+  if (t < nc) {
+    mkey[t] = c + t;
+    mval[t] = spiv[t];
+    mkey[nc + t] = dest[t];
+    mval[nc + t] = c + t;
+  }
+  // the leaf's own columns: multipliers of the pivot rows and of the rows they
+  // displace move, the pivot rows' upper part comes from LDS
+  constexpr int kPer = (W * W + kLuWgThreads - 1) / kLuWgThreads;
+  double up[kPer], down[kPer];
 #pragma unroll
-  for (int k = 0; k < NR; ++k) {
-    const int r = c + t + kLuWgThreads * k;
-    if (r < n) {
+  for (int e = 0; e < kPer; ++e) {
+    const int i = (t + e * kLuWgThreads) % W, jj = (t + e * kLuWgThreads) / W;
+    up[e] = down[e] = 0.0;
+    if (i < nc && jj < nc) {
+      const double* a = A + (int64_t)(c + jj) * lda;
+      up[e] = jj < i ? a[spiv[i]] : P[i][jj];
+      if (dest[i] >= 0) down[e] = a[c + i];
+    }
+  }
+  __syncthreads();
 #pragma unroll
-      for (int jj = 0; jj < W; ++jj)
-        if (jj < nc) A[r + (int64_t)(c + jj) * lda] = vals[k][jj];
+  for (int e = 0; e < kPer; ++e) {
+    const int i = (t + e * kLuWgThreads) % W, jj = (t + e * kLuWgThreads) / W;
+    if (i < nc && jj < nc) {
+      double* a = A + (int64_t)(c + jj) * lda;
+      a[c + i] = up[e];
+      if (dest[i] >= 0) a[dest[i]] = down[e];
     }
   }
 }
 
-// LAPACK interchanges of the leaf: at step j the row chosen (original
-// position piv[j]) is swapped with whatever row is at position c + j.  Only
-// positions touched by this leaf's swaps differ from the identity; one
-// wavefront keeps them as (position, row) pairs, one pair per lane, and finds
-// entries by ballot.
-__device__ __forceinline__ void lu_leaf_ipiv_wave(int c, int nc, const int* piv, const LuWork& w) {
-  const int lane = (int)(threadIdx.x & 63);
-  int key = -1, val = -1, m = 0;
-  for (int j = 0; j < nc; ++j) {
-    const int want = piv[j];
-    const int pj = c + j;
-    const unsigned long long hv = __ballot(key >= 0 && val == want);
-    const int q = hv ? __shfl(key, __ffsll((long long)hv) - 1) : want;
-    const unsigned long long hp = __ballot(key == pj);
-    const int at_pj = hp ? __shfl(val, __ffsll((long long)hp) - 1) : pj;
-    if (lane == 0) w.ipiv[pj] = q + 1;
-    // position pj now holds `want`, position q the row that was at pj
-    if (hp) {
-      if (key == pj) val = want;
-    } else {
-      if (lane == m) {
-        key = pj;
-        val = want;
-      }
-      ++m;
-    }
-    if (q != pj) {
-      const unsigned long long hq = __ballot(key == q);
-      if (hq) {
-        if (key == q) val = at_pj;
-      } else {
-        if (lane == m) {
-          key = q;
-          val = at_pj;
-        }
-        ++m;
-      }
-    }
+// The panel's other columns after lu_leaf_wg, one wave for each: the leaf's row
+// movement and, right of the leaf, the pivot rows' solve against its unit
+// lower triangle, lane i holding row i of both.  (The update of the rows below
+// it is a GEMM of its own: with a workgroup doing its columns' update too, one
+// CU's bandwidth bounds it, 17-19 us against 3 + 6.)
+constexpr int kLuApplyCols = 4;                   // columns (waves) per workgroup
+template <int W>
+__global__ void __launch_bounds__(64 * kLuApplyCols) lu_leaf_apply(double* A, int64_t lda, int c,
+                                                                   int cend, int k0, int kend,
+                                                                   LuWork w) {
+  const int t = threadIdx.x, i = t & 63, nc = cend - c;
+  // columns k0 .. c-1, then cend .. kend-1
+  const int at = k0 + (int)blockIdx.x * kLuApplyCols + (t >> 6);
+  const int col = at < c ? at : at + nc;
+  if (col >= kend) return;
+  double* a = A + (int64_t)col * lda;
+  const bool on = i < nc;
+  double x = 0.0, d = 0.0, l[W];
+  int to = -1;
+  const double* l11 = A + c + (int64_t)c * lda;
+  // nc == W right of the leaf: a shorter one ends its panel
+#pragma unroll
+  for (int j = 0; j < W; ++j)
+    l[j] = col >= cend && i < W && j < i ? l11[i + (int64_t)j * lda] : 0.0;
+  if (on) {
+    to = w.mkey[2 * (c - k0) + nc + i];
+    x = a[w.mval[2 * (c - k0) + i]];
+    d = a[c + i];
   }
-  // publish the positions whose row changed, compacted
-  const bool moved = lane < m && key != val;
-  const unsigned long long hm = __ballot(moved);
-  const int slot = __popcll(hm & ((1ull << lane) - 1ull));
-  if (moved) {
-    w.mkey[slot] = key;
-    w.mval[slot] = val;
-  }
-  if (lane == 0) *w.nmove = __popcll(hm);
+  if (on && to >= 0) a[to] = d;
+#pragma unroll
+  for (int j = 0; j + 1 < W; ++j) x = fma(-l[j], lu_lane(x, j), x);
+  if (on) a[c + i] = x;
 }
 
-__global__ void __launch_bounds__(64) lu_leaf_ipiv(int c, int nc, LuWork w) {
-  lu_leaf_ipiv_wave(c, nc, w.piv, w);
+// Interchanges and row movement of a leaf of the multi-workgroup path.
+__global__ void __launch_bounds__(64) lu_leaf_ipiv(int c, int nc, int k0, LuWork w) {
+  const int lane = (int)threadIdx.x;
+  const int2 mv = lu_leaf_ipiv_wave(c, nc, w.piv, w.ipiv);
+  if (lane < 2 * nc) {
+    w.mkey[2 * (c - k0) + lane] = mv.x;
+    w.mval[2 * (c - k0) + lane] = mv.y;
+  }
 }
 
-// Apply the leaf's row movement to every column, one thread per column: the
-// moved rows' values are all loaded, then all stored (the same result as the
-// leaf's interchanges applied one after another).
-__global__ void __launch_bounds__(256) lu_leaf_move(double* A, int64_t lda, int ncols, LuWork w) {
+// Apply the movement of the leaf [c, c + nc) to ncols columns from A on, one
+// thread per column: the moved rows' values are all loaded, then all stored
+// (the same result as the leaf's interchanges applied one after another).
+__global__ void __launch_bounds__(256) lu_leaf_move(double* A, int64_t lda, int ncols, int c,
+                                                    int nc, int k0, LuWork w) {
   __shared__ int sk[2 * kLuLeaf], sv[2 * kLuLeaf];
-  __shared__ int sn;
   const int t = threadIdx.x;
-  if (t == 0) sn = *w.nmove;
-  __syncthreads();
-  const int nm = sn;
-  if (t < nm) {
-    sk[t] = w.mkey[t];
-    sv[t] = w.mval[t];
+  if (t < 2 * kLuLeaf) {
+    sk[t] = t < 2 * nc ? w.mkey[2 * (c - k0) + t] : -1;
+    sv[t] = t < 2 * nc ? w.mval[2 * (c - k0) + t] : 0;
   }
   __syncthreads();
   const int col = (int)blockIdx.x * 256 + t;
-  if (col >= ncols || nm == 0) return;
+  if (col >= ncols) return;
   double* a = A + (int64_t)col * lda;
   double v[2 * kLuLeaf];
 #pragma unroll
   for (int k = 0; k < 2 * kLuLeaf; ++k)
-    if (k < nm) v[k] = a[sv[k]];
+    if (sk[k] >= 0) v[k] = a[sv[k]];
 #pragma unroll
   for (int k = 0; k < 2 * kLuLeaf; ++k)
-    if (k < nm) a[sk[k]] = v[k];
+    if (sk[k] >= 0) a[sk[k]] = v[k];
 }
 
+// The panel's net row movement from its leaves' (columns cut[0] < cut[1] < ..
+// relative to the panel, cut[nleaf] its width), over the rows [k0, n): the
+// rows are replayed leaf by leaf in an LDS table, as offsets from k0.
+constexpr int kLuPermRows = 65536;               // rows the table holds
+constexpr int kLuMaxLeaves = kLuPanel / 8;
+struct LuCuts {
+  short n;
+  short cut[kLuMaxLeaves + 1];
+};
+__global__ void __launch_bounds__(256) lu_panel_perm(int k0, int nb, int n, LuCuts cuts,
+                                                     LuWork w) {
+  __shared__ unsigned short pr[kLuPermRows];
+  __shared__ int count;
+  const int t = threadIdx.x, rows = n - k0;
+  for (int i = t; i < rows; i += 256) pr[i] = (unsigned short)i;
+  if (t == 0) count = nb;
+  __syncthreads();
+  for (int f = 0; f < cuts.n; ++f) {
+    const int e0 = 2 * cuts.cut[f], e1 = 2 * cuts.cut[f + 1];   // at most 2 kLuLeaf entries
+    const bool on = e0 + t < e1;
+    const int key = on ? w.mkey[e0 + t] : -1;
+    const unsigned short v = key >= 0 ? pr[w.mval[e0 + t] - k0] : 0;
+    __syncthreads();
+    if (key >= 0) pr[key - k0] = v;
+    __syncthreads();
+  }
+  for (int i = t; i < rows; i += 256) {
+    const int from = pr[i];
+    if (i < nb) {
+      w.pkey[i] = k0 + i;
+      w.pval[i] = k0 + from;
+    } else if (from != i) {
+      const int e = atomicAdd(&count, 1);        // at most nb rows below the panel change
+      w.pkey[e] = k0 + i;
+      w.pval[e] = k0 + from;
+    }
+  }
+  __syncthreads();
+  if (t == 0) *w.pcount = count;
+}
+
+// Apply the panel's movement to the columns outside [k0, k0 + nb) and to the
+// right-hand sides: kLuMoveCols columns per workgroup, a thread per entry, so
+// that the panel's own rows are read and written as contiguous runs.
+constexpr int kLuMoveCols = 8;
+__global__ void __launch_bounds__(512) lu_panel_move(double* A, int64_t lda, int n, int k0, int nb,
+                                                     double* B, int64_t ldb, int nrhs, LuWork w) {
+  static_assert(2 * kLuPanel <= 512, "one thread per entry");
+  const int t = threadIdx.x;
+  const bool on = t < *w.pcount;
+  const int key = on ? w.pkey[t] : 0, val = on ? w.pval[t] : 0;
+  const bool moves = on && key != val;
+  double v[kLuMoveCols];
+  double* at[kLuMoveCols];
+#pragma unroll
+  for (int q = 0; q < kLuMoveCols; ++q) {
+    const int i = (int)blockIdx.x * kLuMoveCols + q;
+    at[q] = nullptr;
+    if (i < n - nb) at[q] = A + (int64_t)(i < k0 ? i : i + nb) * lda;
+    else if (i < n - nb + nrhs) at[q] = B + (int64_t)(i - (n - nb)) * ldb;
+    if (moves && at[q]) v[q] = at[q][val];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kLuMoveCols; ++q)
+    if (moves && at[q]) at[q][key] = v[q];
+}
+
+// The leaf [c, cend) of the panel [k0, kend) and its movement and solve in the
+// panel's other columns; its width is lu_leaf_width(n - c).
+template <int NR, int W>
+void launch_leaf_wg(hipStream_t s, double* dA, int64_t lda, int n, int c, int cend, int k0,
+                    int kend, const LuWork& w) {
+  hipLaunchKernelGGL((lu_leaf_wg<NR, W>), dim3(1), dim3(kLuWgThreads), 0, s, dA, lda, n, c, cend,
+                     k0, w);
+  const int other = kend - k0 - (cend - c);
+  if (other > 0)
+    hipLaunchKernelGGL(lu_leaf_apply<W>, dim3((other + kLuApplyCols - 1) / kLuApplyCols),
+                       dim3(64 * kLuApplyCols), 0, s, dA, lda, c, cend, k0, kend, w);
+}
+
+void launch_leaf(hipStream_t s, double* dA, int64_t lda, int n, int c, int cend, int k0, int kend,
+                 const LuWork& w) {
+#define PSX_LEAF(NR, W) launch_leaf_wg<NR, W>(s, dA, lda, n, c, cend, k0, kend, w)
+  switch ((n - c + kLuWgThreads - 1) / kLuWgThreads) {
+    case 1: return PSX_LEAF(1, 32);
+    case 2: return PSX_LEAF(2, 32);
+    case 3: return PSX_LEAF(3, 32);
+    case 4: return PSX_LEAF(4, 16);
+    case 5: return PSX_LEAF(5, 16);
+    case 6: return PSX_LEAF(6, 16);
+    case 7:
+    case 8: return PSX_LEAF(8, 8);
+    case 9:
+    case 10: return PSX_LEAF(10, 8);
+    default: return PSX_LEAF(12, 8);
+  }
+#undef PSX_LEAF
+}
+
+// Columns of the leaf that starts with `rows` rows to factor.
+int lu_leaf_width(int rows) {
+  const int nr = (rows + kLuWgThreads - 1) / kLuWgThreads;
+  return nr > 12 ? kLuLeaf : nr > 6 ? 8 : nr > 3 ? 16 : 32;
+}
 // Where an LU runs: a stream, the rocBLAS handle bound to it and a device work
 // area of lu_work_bytes(n) bytes (pivot candidates, flags, the leaf's row
 // movement).  Factorizations on different lanes may run at the same time.
@@ -460,10 +722,13 @@ size_t lu_work_bytes(int n) {
   const size_t rows_bytes = 2 * (size_t)Gmax * kLuLeaf * sizeof(double);
   const size_t move_off = (rows_bytes + 24 * (size_t)Gmax + 4 * kLuLeaf + (size_t)n + 255) &
                           ~size_t(255);
-  return move_off + sizeof(int) * (4 * kLuLeaf + 1) + 256;
+  return move_off + sizeof(int) * (8 * kLuPanel + 1) + 256;
 }
 
-void lu_factor_on(const LuLane& L, int n, double* dA, int64_t lda, int* dipiv, int* dinfo) {
+// dA (n x n) becomes its LU factors; the interchanges are applied to the nrhs
+// columns of dB on the way.
+void lu_factor_on(const LuLane& L, int n, double* dA, int64_t lda, int* dipiv, int* dinfo,
+                  double* dB = nullptr, int64_t ldb = 0, int nrhs = 0) {
   rocblas_handle h = L.h;
   hipStream_t s = L.s;
   const int Gmax = (n + kLuRows - 1) / kLuRows;
@@ -478,67 +743,78 @@ void lu_factor_on(const LuLane& L, int n, double* dA, int64_t lda, int* dipiv, i
   w.candi = (int*)(base + rows_bytes + 16 * (size_t)Gmax);    // 2 Gmax ints
   w.piv = (int*)(base + rows_bytes + 24 * (size_t)Gmax);      // kLuLeaf ints
   w.done = (unsigned char*)(base + rows_bytes + 24 * (size_t)Gmax + 4 * kLuLeaf);  // n flags
-  w.mkey = (int*)(base + move_off);                           // 2 kLuLeaf ints
-  w.mval = w.mkey + 2 * kLuLeaf;                              // 2 kLuLeaf ints
-  w.nmove = w.mval + 2 * kLuLeaf;                             // 1 int
+  w.mkey = (int*)(base + move_off);                           // 2 kLuPanel ints each
+  w.mval = w.mkey + 2 * kLuPanel;
+  w.pkey = w.mval + 2 * kLuPanel;
+  w.pval = w.pkey + 2 * kLuPanel;
+  w.pcount = w.pval + 2 * kLuPanel;                           // 1 int
   w.ipiv = dipiv;
   w.info = dinfo;
   PSX_HIP(hipMemsetAsync(dinfo, 0, sizeof(int), s));
   const double one = 1.0, mone = -1.0;
   for (int k = 0; k < n; k += kLuPanel) {
-    const int kend = std::min(n, k + kLuPanel);
+    const int kend = std::min(n, k + kLuPanel), nb = kend - k;
+    // the panel's net movement is replayed in LDS, which bounds its rows
+    const bool deferred = n - k <= kLuPermRows;
+    LuCuts cuts{};
     for (int cl = k; cl < kend;) {
-      // the trailing leaves, once their rows fit one workgroup, in one launch each
       const int rows = n - cl;
       const bool one_wg = rows <= kLuWgRowsMax;
-      const int nr = (rows + kLuWgThreads - 1) / kLuWgThreads;
-      // one row per thread leaves room for kLuLeaf columns, more rows for kLuWgLeaf
-      const int width = !one_wg || nr == 1 ? kLuLeaf : kLuWgLeaf;
-      const int cend = std::min(kend, cl + width);
+      const int cend = std::min(kend, cl + lu_leaf_width(rows));
       const int nc = cend - cl;
       if (one_wg) {
-        if (nr == 1)
-          hipLaunchKernelGGL((lu_leaf_wg<1, kLuLeaf>), dim3(1), dim3(kLuWgThreads), 0, s, dA, lda,
-                             n, cl, cend, w);
-        else if (nr == 2)
-          hipLaunchKernelGGL((lu_leaf_wg<2, kLuWgLeaf>), dim3(1), dim3(kLuWgThreads), 0, s, dA,
-                             lda, n, cl, cend, w);
-        else
-          hipLaunchKernelGGL((lu_leaf_wg<3, kLuWgLeaf>), dim3(1), dim3(kLuWgThreads), 0, s, dA,
-                             lda, n, cl, cend, w);
-        // (the kernel converts its pivots itself)
+        launch_leaf(s, dA, lda, n, cl, cend, k, kend, w);
       } else {
-        const int G = (n - cl + kLuRows - 1) / kLuRows;
+        const int G = (rows + kLuRows - 1) / kLuRows;
         hipLaunchKernelGGL(lu_leaf_init, dim3(G), dim3(kLuRows), 0, s, dA, lda, n, cl, cend, w);
         for (int j = 0; j < nc; ++j)
           hipLaunchKernelGGL(lu_leaf_col, dim3(G), dim3(kLuRows), 0, s, dA, lda, n, cl, j, cend,
                              G, w);
+        hipLaunchKernelGGL(lu_leaf_ipiv, dim3(1), dim3(64), 0, s, cl, nc, k, w);
+        hipLaunchKernelGGL(lu_leaf_move, dim3((nb + 255) / 256), dim3(256), 0, s,
+                           dA + (int64_t)k * lda, lda, nb, cl, nc, k, w);
+        if (cend < kend)   // rest of the panel: U = L11^-1 A
+          PSX_ROC(rocblas_dtrsm(h, rocblas_side_left, rocblas_fill_lower,
+                                rocblas_operation_none, rocblas_diagonal_unit, nc, kend - cend,
+                                &one, dA + cl + (int64_t)cl * lda, (rocblas_int)lda,
+                                dA + cl + (int64_t)cend * lda, (rocblas_int)lda));
       }
-      if (!one_wg) hipLaunchKernelGGL(lu_leaf_ipiv, dim3(1), dim3(64), 0, s, cl, nc, w);
-      hipLaunchKernelGGL(lu_leaf_move, dim3((n + 255) / 256), dim3(256), 0, s, dA, lda, n, w);
+      if (!deferred) {
+        if (k > 0)
+          hipLaunchKernelGGL(lu_leaf_move, dim3((k + 255) / 256), dim3(256), 0, s, dA, lda, k, cl,
+                             nc, k, w);
+        if (kend < n)
+          hipLaunchKernelGGL(lu_leaf_move, dim3((n - kend + 255) / 256), dim3(256), 0, s,
+                             dA + (int64_t)kend * lda, lda, n - kend, cl, nc, k, w);
+        if (nrhs > 0)
+          hipLaunchKernelGGL(lu_leaf_move, dim3((nrhs + 255) / 256), dim3(256), 0, s, dB, ldb,
+                             nrhs, cl, nc, k, w);
+      }
       PSX_HIP(hipGetLastError());
-      if (cend < kend) {   // rest of the block: U = L11^-1 A, then the update
-        double* L11 = dA + cl + (int64_t)cl * lda;
-        double* A12 = dA + cl + (int64_t)cend * lda;
-        PSX_ROC(rocblas_dtrsm(h, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none,
-                              rocblas_diagonal_unit, nc, kend - cend, &one, L11, (rocblas_int)lda,
-                              A12, (rocblas_int)lda));
-        if (cend < n)
-          PSX_ROC(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, n - cend,
-                                kend - cend, nc, &mone, dA + cend + (int64_t)cl * lda,
-                                (rocblas_int)lda, A12, (rocblas_int)lda, &one,
-                                dA + cend + (int64_t)cend * lda, (rocblas_int)lda));
-      }
+      if (cend < kend)     // the rows below it
+        PSX_ROC(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, n - cend,
+                              kend - cend, nc, &mone, dA + cend + (int64_t)cl * lda,
+                              (rocblas_int)lda, dA + cl + (int64_t)cend * lda, (rocblas_int)lda,
+                              &one, dA + cend + (int64_t)cend * lda, (rocblas_int)lda));
+      cuts.cut[cuts.n++] = (short)(cl - k);
       cl = cend;
+    }
+    cuts.cut[cuts.n] = (short)nb;
+    const int others = n - nb + nrhs;
+    if (deferred && others > 0) {
+      hipLaunchKernelGGL(lu_panel_perm, dim3(1), dim3(256), 0, s, k, nb, n, cuts, w);
+      hipLaunchKernelGGL(lu_panel_move, dim3((others + kLuMoveCols - 1) / kLuMoveCols), dim3(512),
+                         0, s, dA, lda, n, k, nb, dB, ldb, nrhs, w);
+      PSX_HIP(hipGetLastError());
     }
     if (kend < n) {        // trailing matrix
       double* L11 = dA + k + (int64_t)k * lda;
       double* A12 = dA + k + (int64_t)kend * lda;
       PSX_ROC(rocblas_dtrsm(h, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none,
-                            rocblas_diagonal_unit, kend - k, n - kend, &one, L11, (rocblas_int)lda,
+                            rocblas_diagonal_unit, nb, n - kend, &one, L11, (rocblas_int)lda,
                             A12, (rocblas_int)lda));
       PSX_ROC(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, n - kend, n - kend,
-                            kend - k, &mone, dA + kend + (int64_t)k * lda, (rocblas_int)lda, A12,
+                            nb, &mone, dA + kend + (int64_t)k * lda, (rocblas_int)lda, A12,
                             (rocblas_int)lda, &one, dA + kend + (int64_t)kend * lda,
                             (rocblas_int)lda));
     }
@@ -708,113 +984,133 @@ void lu_trs_dev(Ctx* c, int n, const double* dA, int64_t lda, double* dx) {
 
 // ---- triangular solves with many right-hand sides ---------------------------
 // Blocked left substitution X = T^{-1} B for the LU factors (T = unit lower L
-// or upper U) and m right-hand sides, in kTrsRows-row blocks: the diagonal
-// block is solved by substitution (trsm_diag, one thread per right-hand side,
-// the block staged in LDS), and the rows still to come are updated by a
-// rocBLAS GEMM.  Substitution keeps LAPACK's backward error on ill-conditioned
-// U, which a trsm built on inverted diagonal blocks does not.
-constexpr int kTsmRows = 64;               // diagonal block of the many-column solve
-constexpr int kTsmLd = kTsmRows + 1;        // its LDS column stride
-constexpr int kTsmCols = 192;               // right-hand sides per workgroup (one per thread)
+// or upper U) and m right-hand sides, in kTsmRows-row blocks: the diagonal
+// block is solved by substitution (trsm_block), and the rows still to come are
+// updated by a rocBLAS GEMM of depth kTsmRows.  Substitution keeps LAPACK's
+// backward error on ill-conditioned U, which a trsm built on inverted diagonal
+// blocks does not.
+//   A wave takes kTsmCols right-hand sides, lane i holding rows i, i + 64, ..
+// of the block; the value solved at a step goes through scalar registers to
+// all lanes.  The triangle passes through LDS, kTsmAhead columns at a time,
+// one set ahead of the steps, so that a workgroup's waves read it from L2
+// once: with each wave reading it for itself the L2 bounds the kernel (103 and
+// 169 us at m = 2509; 34 and 58 us with LDS).  Issue-bound on the broadcasts,
+// the quotients and the updates.  64-row blocks, one right-hand side a thread,
+// ran 45 us each (180 for 256 rows) on 14 workgroups, and their depth-64 GEMMs
+// were bound by the traffic of B.
+constexpr int kTsmRows = 256;
+constexpr int kTsmSub = kTsmRows / 64;
+constexpr int kTsmCols = 2;
+constexpr int kTsmWaves = 8;
+constexpr int kTsmAhead = 16;
+constexpr int kTsmStage = kTsmAhead * kTsmRows / (64 * kTsmWaves);  // values a thread stages
 
 template <bool UPPER>
-__global__ void __launch_bounds__(kTsmCols) trsm_diag(const double* __restrict__ A, int64_t lda,
-                                                      int n, int k, double* __restrict__ B,
-                                                      int64_t ldb, int m) {
-  __shared__ double D[kTsmRows * kTsmLd];         // the diagonal block, column-major
-  __shared__ double Bs[kTsmRows][kTsmCols];       // this workgroup's rows of B
-  const int t = threadIdx.x;
-  const int R0 = k * kTsmRows, cn = min(kTsmRows, n - R0);
-  const int c0 = (int)blockIdx.x * kTsmCols, cm = min(kTsmCols, m - c0);
-  // stage D and B: 64 consecutive rows per wave, one column per wave and pass
-  const int lane = t & 63, wv = t >> 6;
-  {
-    const bool rin = lane < cn;
-    const double* a = A + (R0 + (rin ? lane : 0)) + (int64_t)R0 * lda;
-    constexpr int kW = kTsmCols / 64;                       // waves
-    constexpr int kPer = (kTsmRows + kW - 1) / kW;          // columns per wave, rounded up
-    double v[kPer];
+__global__ void __launch_bounds__(64 * kTsmWaves) trsm_block(const double* __restrict__ A,
+                                                             int64_t lda, int n, int R0,
+                                                             double* __restrict__ B, int64_t ldb,
+                                                             int m) {
+  __shared__ double Ts[2][kTsmAhead][kTsmRows];
+  const int t = threadIdx.x, lane = t & 63;
+  const int col0 = __builtin_amdgcn_readfirstlane(
+      ((int)blockIdx.x * kTsmWaves + (t >> 6)) * kTsmCols);
+  const int cn = min(kTsmRows, n - R0);
+  const double* T = A + R0 + (int64_t)R0 * lda;     // T[row + column lda]
+  double* b = B + R0 + (int64_t)col0 * ldb;
+  // acc: what the sub-blocks already solved take from one still to come,
+  // summed by itself and subtracted once, as the GEMM between blocks does
+  double x[kTsmSub][kTsmCols], acc[kTsmSub][kTsmCols], d[kTsmSub], rd[kTsmSub];
+  bool plain = true;
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int ic = q * kW + wv;
-      v[q] = (rin && ic < cn) ? a[(int64_t)ic * lda] : 0.0;
-    }
+  for (int s = 0; s < kTsmSub; ++s) {
+    const int r = 64 * s + lane;
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int ic = q * kW + wv;
-      if (ic < kTsmRows) D[ic * kTsmLd + lane] = v[q];
+    for (int q = 0; q < kTsmCols; ++q) {
+      x[s][q] = r < cn && col0 + q < m ? b[r + (int64_t)q * ldb] : 0.0;
+      acc[s][q] = 0.0;
     }
+    d[s] = UPPER && r < cn ? T[r + (int64_t)r * lda] : 1.0;
+    rd[s] = 1.0 / d[s];
+    plain &= fabs(d[s]) > 0x1p-1000 && fabs(d[s]) < 0x1p1000;
   }
-  {
-    const bool rin = lane < cn;
-    const double* b = B + (R0 + (rin ? lane : 0)) + (int64_t)c0 * ldb;
-    constexpr int kPer = kTsmCols / (kTsmCols / 64);  // 64 columns per wave
-#pragma unroll 16
-    for (int q = 0; q < kPer; ++q) {
-      const int jc = q * (kTsmCols / 64) + wv;
-      Bs[lane][jc] = (rin && jc < cm) ? b[(int64_t)jc * ldb] : 0.0;
+  // every pivot's reciprocal in the normal range: quotients by it, with one
+  // residual correction (the correctly rounded quotient)
+  const bool fast = __builtin_amdgcn_ballot_w64(!plain) == 0;
+  // sets of kTsmAhead columns, from the first (lower) or last (upper) that
+  // holds one of the block; a thread stages kTsmStage of a set's entries in
+  // its row, zero beyond the block
+  const int row = t % kTsmRows, part = (t / kTsmRows) * kTsmStage;
+  double ahead[kTsmStage];
+  auto load = [&](int f) {
+#pragma unroll
+    for (int e = 0; e < kTsmStage; ++e) {
+      const int j = f * kTsmAhead + part + e;
+      ahead[e] = row < cn && j < cn ? T[row + (int64_t)j * lda] : 0.0;
     }
-  }
-  __syncthreads();
-  if (t < cm) {
-    // two 32-row sub-blocks; the one being solved sits in registers
-    constexpr int S = 32;
-    const int nsub = (cn + S - 1) / S;
+  };
+  constexpr int kSets = 64 / kTsmAhead;             // of a 64-row sub-block
+  const int last = (cn - 1) / kTsmAhead;
+  load(UPPER ? last : 0);
+#pragma unroll
+  for (int ss = 0; ss < kTsmSub; ++ss) {
+    const int s = UPPER ? kTsmSub - 1 - ss : ss;
+    const int f0 = s * kSets, f1 = min(f0 + kSets - 1, last);
+#pragma unroll
+    for (int c = 0; c < kTsmCols; ++c) x[s][c] -= acc[s][c];
 #pragma unroll 1
-    for (int q = 0; q < nsub; ++q) {
-      const int sb = UPPER ? nsub - 1 - q : q;
-      const int s0 = sb * S, sn = min(S, cn - s0);
-      double x[S];
+    for (int i = f0; i <= f1; ++i) {
+      const int f = UPPER ? f1 - (i - f0) : i, buf = f & 1;
 #pragma unroll
-      for (int i = 0; i < S; ++i) x[i] = Bs[(s0 + i) & (kTsmRows - 1)][t];
-      if (!UPPER) {
+      for (int e = 0; e < kTsmStage; ++e) Ts[buf][part + e][row] = ahead[e];
+      __syncthreads();                              // also ends the reads of set f -+ 1
+      const int nf = UPPER ? f - 1 : f + 1;
+      if (nf >= 0 && nf <= last) load(nf);
+      const int j0 = (f - f0) * kTsmAhead;
 #pragma unroll
-        for (int j = 0; j < S; ++j) {
-          if (j < sn) {
+      for (int u = 0; u < kTsmAhead; ++u) {
+        const int e = UPPER ? kTsmAhead - 1 - u : u, j = j0 + e;
+        const bool off = UPPER ? lane < j : lane > j;
+        double tv[kTsmSub];
 #pragma unroll
-            for (int i = j + 1; i < S; ++i)
-              x[i] = fma(-D[(s0 + j) * kTsmLd + s0 + i], x[j], x[i]);
+        for (int q = 0; q < kTsmSub; ++q)
+          if (UPPER ? q <= s : q >= s) tv[q] = Ts[buf][e][64 * q + lane];
+#pragma unroll
+        for (int c = 0; c < kTsmCols; ++c) {
+          double y = x[s][c], xj;
+          if (UPPER) {
+            if (fast) {
+              const double z = y * rd[s];
+              const double w = fma(fma(-z, d[s], y), rd[s], z);
+              xj = lu_lane(w, j);
+              // an overflow, whose correction is NaN, or a NaN: divide
+              if ((__double2hiint(xj) & 0x7ff00000) != 0x7ff00000) {
+                y = w;
+              } else {
+                y = y / d[s];
+                xj = lu_lane(y, j);
+              }
+            } else {
+              y = y / d[s];
+              xj = lu_lane(y, j);
+            }
+          } else {
+            xj = lu_lane(y, j);
           }
-          __builtin_amdgcn_sched_barrier(0);
+          const double own = fma(-tv[s], xj, x[s][c]);
+          x[s][c] = off ? own : (UPPER && lane == j) ? y : x[s][c];
+#pragma unroll
+          for (int q = 0; q < kTsmSub; ++q)
+            if (UPPER ? q < s : q > s) acc[q][c] = fma(tv[q], xj, acc[q][c]);
         }
-      } else {
-#pragma unroll
-        for (int j = S - 1; j >= 0; --j) {
-          if (j < sn) {
-            x[j] = x[j] / D[(s0 + j) * kTsmLd + s0 + j];
-#pragma unroll
-            for (int i = 0; i < j; ++i) x[i] = fma(-D[(s0 + j) * kTsmLd + s0 + i], x[j], x[i]);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < S; ++i)
-        if (i < sn) Bs[s0 + i][t] = x[i];
-      // the other sub-block's rows take this one's contribution
-      const int r0 = UPPER ? 0 : s0 + sn, r1 = UPPER ? s0 : cn;
-#pragma unroll 4
-      for (int i = r0; i < r1; ++i) {
-        double p0 = 0.0, p1 = 0.0;
-#pragma unroll
-        for (int j = 0; j < S; j += 2) {
-          p0 = fma(D[(s0 + j) * kTsmLd + i], x[j], p0);
-          p1 = fma(D[(s0 + j + 1) * kTsmLd + i], x[j + 1], p1);
-        }
-        Bs[i][t] -= p0 + p1;
       }
     }
   }
-  __syncthreads();
-  {
-    const bool rin = lane < cn;
-    double* b = B + (R0 + (rin ? lane : 0)) + (int64_t)c0 * ldb;
-    constexpr int kPer = kTsmCols / (kTsmCols / 64);
-#pragma unroll 16
-    for (int q = 0; q < kPer; ++q) {
-      const int jc = q * (kTsmCols / 64) + wv;
-      if (rin && jc < cm) b[(int64_t)jc * ldb] = Bs[lane][jc];
-    }
+#pragma unroll
+  for (int s = 0; s < kTsmSub; ++s) {
+    const int r = 64 * s + lane;
+#pragma unroll
+    for (int q = 0; q < kTsmCols; ++q)
+      if (r < cn && col0 + q < m) b[r + (int64_t)q * ldb] = x[s][q];
   }
 }
 
@@ -825,17 +1121,16 @@ static void trsm_left_dev(Ctx* c, bool upper, int n, const double* dA, int64_t l
   rocblas_handle h = blas(c);
   hipStream_t s = c->stream;
   const int nb = (n + kTsmRows - 1) / kTsmRows;
-  const unsigned g = (unsigned)((m + kTsmCols - 1) / kTsmCols);
+  const unsigned g = (unsigned)((m + kTsmWaves * kTsmCols - 1) / (kTsmWaves * kTsmCols));
   const double one = 1.0, mone = -1.0;
   for (int q = 0; q < nb; ++q) {
-    const int k = upper ? nb - 1 - q : q;
-    const int R0 = k * kTsmRows, cn = std::min(kTsmRows, n - R0);
+    const int R0 = (upper ? nb - 1 - q : q) * kTsmRows, cn = std::min(kTsmRows, n - R0);
     if (upper)
-      hipLaunchKernelGGL(trsm_diag<true>, dim3(g), dim3(kTsmCols), 0, s, dA, lda, n, k, dB, ldb,
-                         m);
+      hipLaunchKernelGGL(trsm_block<true>, dim3(g), dim3(64 * kTsmWaves), 0, s, dA, lda, n, R0, dB,
+                         ldb, m);
     else
-      hipLaunchKernelGGL(trsm_diag<false>, dim3(g), dim3(kTsmCols), 0, s, dA, lda, n, k, dB, ldb,
-                         m);
+      hipLaunchKernelGGL(trsm_block<false>, dim3(g), dim3(64 * kTsmWaves), 0, s, dA, lda, n, R0, dB,
+                         ldb, m);
     PSX_HIP(hipGetLastError());
     if (!upper && R0 + cn < n)  // rows below: B2 -= L21 X1
       PSX_ROC(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, n - R0 - cn, m, cn,
@@ -847,36 +1142,6 @@ static void trsm_left_dev(Ctx* c, bool upper, int n, const double* dA, int64_t l
                             &one, dB, (rocblas_int)ldb));
   }
 }
-
-// dA (n x n, lda) is overwritten by its LU factors; dB (n x nrhs) by X.
-// Factor dA in place; ipiv (device, n + 64 ints) receives the LAPACK
-// interchanges.  Raises SingularException on a zero pivot.
-static void lu_factor_checked(Ctx* c, int n, double* dA, int64_t lda, int* ipiv) {
-  int* info = ipiv + n + 32;
-  lu_factor_dev(c, n, dA, lda, ipiv, info);
-  int hinfo = 0;
-  PSX_HIP(hipMemcpyAsync(&hinfo, info, sizeof(hinfo), hipMemcpyDeviceToHost, c->stream));
-  PSX_HIP(hipStreamSynchronize(c->stream));
-  PSX_REQUIRE(hinfo == 0, PSX_ERR_SINGULAR,
-              "LU: zero pivot at position " + std::to_string(hinfo) +
-                  " (Julia SingularException)");
-}
-
-// A device int array of n + 64 entries (LAPACK interchanges and their info
-// slot, or a row permutation), freed on scope exit after the stream has
-// drained.
-struct Pivots {
-  Ctx* c;
-  int* p;
-  Pivots(Ctx* cc, int n) : c(cc), p((int*)ctx_alloc(cc, sizeof(int) * ((size_t)n + 64))) {}
-  ~Pivots() {
-    (void)hipStreamSynchronize(c->stream);
-    try {
-      ctx_free(c, p);
-    } catch (...) {
-    }
-  }
-};
 
 // The row order LAPACK's interchanges produce, perm[i] = the original row
 // that ends at position i, built by one thread in LDS (the interchanges are
@@ -915,38 +1180,36 @@ __global__ void __launch_bounds__(256) lu_permute_cols(const int* __restrict__ p
   for (int i = threadIdx.x; i < n; i += 256) b[i] = col[perm[i]];
 }
 
-// B = A^{-1} B from the factors of A in dA and its interchanges ipiv.
-static void lu_getrs_dev(Ctx* c, int n, const double* dA, int64_t lda, const int* ipiv,
-                         double* dB, int64_t ldb, int nrhs) {
-  if (nrhs <= 0) return;
-  // P b by the LAPACK interchanges, then the two substitutions.  Many
-  // columns share one permutation, built once and applied as a gather;
-  // a few columns take rocSOLVER's laswp (the sequential chain is the same).
-  if (nrhs > kTrsMaxRhs && n <= kPermMax) {
-    Pivots perm(c, n);
-    hipLaunchKernelGGL(lu_perm, dim3(1), dim3(256), 0, c->stream, ipiv, n, perm.p);
-    hipLaunchKernelGGL(lu_permute_cols, dim3((unsigned)nrhs), dim3(256), 0, c->stream,
-                       (const int*)perm.p, n, dB, ldb);
-    PSX_HIP(hipGetLastError());
-  } else {
-    PSX_ROC(rocsolver_dlaswp(blas(c), nrhs, dB, (rocblas_int)ldb, 1, n,
-                             (const rocblas_int*)ipiv, 1));
-  }
+// A device array for LAPACK's interchanges: n entries, the info slot at n + 32.
+static size_t pivot_bytes(int n) {
+  return (sizeof(int) * ((size_t)n + 64) + 255) & ~size_t(255);
+}
+
+// SingularException for a zero pivot in a finished factorisation; waits for
+// the context stream.
+static void check_pivots(Ctx* c, int n, const int* ipiv) {
+  int hinfo = 0;
+  PSX_HIP(hipMemcpyAsync(&hinfo, ipiv + n + 32, sizeof(hinfo), hipMemcpyDeviceToHost, c->stream));
+  PSX_HIP(hipStreamSynchronize(c->stream));
+  PSX_REQUIRE(hinfo == 0, PSX_ERR_SINGULAR,
+              "LU: zero pivot at position " + std::to_string(hinfo) +
+                  " (Julia SingularException)");
+}
+
+// dA (n x n, lda) becomes its LU factors, dB (n x nrhs) A^{-1} dB.
+void lu_solve_dev(Ctx* c, int n, double* dA, int64_t lda, double* dB, int64_t ldb,
+                  int nrhs) {
+  const size_t wb = (lu_work_bytes(n) + 255) & ~size_t(255);
+  char* work = (char*)ctx_scratch(c, wb + pivot_bytes(n));
+  int* ipiv = (int*)(work + wb);
+  lu_factor_on(LuLane{c->stream, blas(c), work}, n, dA, lda, ipiv, ipiv + n + 32, dB, ldb, nrhs);
   if (nrhs <= kTrsMaxRhs) {
     for (int j = 0; j < nrhs; ++j) lu_trs_dev(c, n, dA, lda, dB + (int64_t)j * ldb);
   } else {
     trsm_left_dev(c, false, n, dA, lda, dB, ldb, nrhs);
     trsm_left_dev(c, true, n, dA, lda, dB, ldb, nrhs);
   }
-}
-
-
-void lu_solve_dev(Ctx* c, int n, double* dA, int64_t lda, double* dB, int64_t ldb,
-                  int nrhs) {
-  Pivots pv(c, n);
-  lu_factor_checked(c, n, dA, lda, pv.p);
-  lu_getrs_dev(c, n, dA, lda, pv.p, dB, ldb, nrhs);
-  PSX_HIP(hipStreamSynchronize(c->stream));
+  check_pivots(c, n, ipiv);
 }
 
 // Independent systems side by side.  System i runs on lane i: lane 0 is the
@@ -990,9 +1253,7 @@ void lu_solve_concurrent(Ctx* c, const LuSystem* sys, int count) {
                               : LuLane{c->lstream[i - 1], (rocblas_handle)c->lblas[i - 1],
                                        work + off[i]};
       if (i > 0) PSX_HIP(hipStreamWaitEvent(L.s, c->lane_ev[0], 0));
-      lu_factor_on(L, q.n, q.dA, q.lda, q.ipiv, q.ipiv + q.n + 32);
-      PSX_ROC(rocsolver_dlaswp(L.h, q.nrhs, q.dB, (rocblas_int)q.ldb, 1, q.n,
-                               (const rocblas_int*)q.ipiv, 1));
+      lu_factor_on(L, q.n, q.dA, q.lda, q.ipiv, q.ipiv + q.n + 32, q.dB, q.ldb, q.nrhs);
       for (int j = 0; j < q.nrhs; ++j)
         lu_trs_on(L.s, q.n, q.dA, q.lda, q.dB + (int64_t)j * q.ldb);
       PSX_HIP(hipGetLastError());
@@ -1049,23 +1310,58 @@ static void transpose(Ctx* c, int n, const double* dIn, double* dOut) {
                         &one, dIn, n, &zero, dOut, n, dOut, n));
 }
 
-// dOut = B1^{-1} Y B2^{-T}; dB1, dB2 are overwritten by their LU factors.
-// dB2 == dB1 (one matrix on both sides) is factored once.
-void decouple_dev(Ctx* c, int n, const double* dY, double* dB1, double* dB2,
-                  double* dOut) {
-  const size_t nn = (size_t)n * n;
-  WorkBuf wk(c, sizeof(double) * nn);
-  double* tmp = (double*)wk.base();
-  PSX_HIP(hipMemcpyAsync(tmp, dY, sizeof(double) * nn, hipMemcpyDeviceToDevice, c->stream));
-  Pivots pv(c, n);
-  lu_factor_checked(c, n, dB1, n, pv.p);
-  lu_getrs_dev(c, n, dB1, n, pv.p, tmp, n, n);   // tmp = B1^{-1} Y
-  transpose(c, n, tmp, dOut);                     // dOut = tmp^T
-  if (dB2 != dB1) lu_factor_checked(c, n, dB2, n, pv.p);
-  lu_getrs_dev(c, n, dB2, n, pv.p, dOut, n, n);  // dOut = B2^{-1} tmp^T
-  transpose(c, n, dOut, tmp);                     // tmp = (B2^{-1} tmp^T)^T
-  PSX_HIP(hipMemcpyAsync(dOut, tmp, sizeof(double) * nn, hipMemcpyDeviceToDevice, c->stream));
-  PSX_HIP(hipStreamSynchronize(c->stream));
+// dY = B1^{-1} Y B2^{-T}, with dT scratch of the same size; dB1, dB2 are
+// overwritten by their LU factors.  dB2 == dB1 (one matrix on both sides) is
+// factored once; otherwise B2 is factored on a stream of its own, beside B1's
+// factorisation and solve (both are bound by the latency of one workgroup's
+// leaves), once `b2` has put it on the device.
+void decouple_dev(Ctx* c, int n, double* dY, double* dB1, double* dB2, double* dT,
+                  const std::function<void()>& b2) {
+  const bool same = dB2 == dB1;
+  ensure_lanes(c, 1);
+  const size_t wb = (lu_work_bytes(n) + 255) & ~size_t(255), pb = pivot_bytes(n);
+  char* work = (char*)ctx_scratch(c, 2 * wb + 3 * pb);
+  int* const p1 = (int*)(work + 2 * wb);
+  int* const p2 = (int*)(work + 2 * wb + pb);
+  int* const perm = (int*)(work + 2 * wb + 2 * pb);
+  const LuLane L1{c->stream, blas(c), work};
+  const LuLane L2 = same ? L1 : LuLane{c->lstream[0], (rocblas_handle)c->lblas[0], work + wb};
+  const int* ip2 = same ? p1 : p2;
+  PSX_HIP(hipEventRecord(c->lane_ev[0], c->stream));
+  try {
+    lu_factor_on(L1, n, dB1, n, p1, p1 + n + 32, dY, n, n);
+    trsm_left_dev(c, false, n, dB1, n, dY, n, n);   // dY = B1^{-1} Y
+    trsm_left_dev(c, true, n, dB1, n, dY, n, n);
+    transpose(c, n, dY, dT);                        // dT = dY^T
+    if (!same) {
+      b2();
+      PSX_HIP(hipStreamWaitEvent(L2.s, c->lane_ev[0], 0));
+      lu_factor_on(L2, n, dB2, n, p2, p2 + n + 32);
+    }
+    if (n <= kPermMax)
+      hipLaunchKernelGGL(lu_perm, dim3(1), dim3(256), 0, L2.s, ip2, n, perm);
+    PSX_HIP(hipGetLastError());
+    if (!same) {
+      PSX_HIP(hipEventRecord(c->lane_ev[1], L2.s));
+      PSX_HIP(hipStreamWaitEvent(c->stream, c->lane_ev[1], 0));
+    }
+    if (n <= kPermMax)
+      hipLaunchKernelGGL(lu_permute_cols, dim3((unsigned)n), dim3(256), 0, c->stream,
+                         (const int*)perm, n, dT, (int64_t)n);
+    else
+      PSX_ROC(rocsolver_dlaswp(blas(c), n, dT, n, 1, n, (const rocblas_int*)ip2, 1));
+    PSX_HIP(hipGetLastError());
+    trsm_left_dev(c, false, n, dB2, n, dT, n, n);   // dT = B2^{-1} dT
+    trsm_left_dev(c, true, n, dB2, n, dT, n, n);
+    transpose(c, n, dT, dY);
+  } catch (...) {
+    // nothing may still run on the caller's buffers once the error is out
+    (void)hipStreamSynchronize(L2.s);
+    (void)hipStreamSynchronize(c->stream);
+    throw;
+  }
+  check_pivots(c, n, p1);
+  if (!same) check_pivots(c, n, p2);
 }
 
 }  // namespace psx
@@ -1181,17 +1477,18 @@ int psx_decouple_covmat(psx_ctx* hctx, int n, const double* Y, const double* B1,
     PSX_REQUIRE(n >= 1, PSX_ERR_ARGUMENT, "n must be positive");
     PSX_REQUIRE(Y && B1 && B2 && out, PSX_ERR_ARGUMENT, "null pointer");
     PSX_HIP(hipSetDevice(c->device));
-    // one matrix passed for both B1 and B2 is copied and factored once
+    // one matrix passed for both B1 and B2 is copied and factored once; B2 is
+    // copied in while B1 is being factored
     const bool same = B1 == B2;
     const size_t nn = (size_t)n * n, b = sizeof(double) * nn;
     XferBuf x(c, xfer_bytes({4 * b}));
     double* d = x.take(4 * b);
     double* dB2 = same ? d + nn : d + 2 * nn;
-    h2d_matrix(c, d, n, Y, n, n, n);
     h2d_matrix(c, d + nn, n, B1, n, n, n);
-    if (!same) h2d_matrix(c, dB2, n, B2, n, n, n);
-    decouple_dev(c, n, d, d + nn, dB2, d + 3 * nn);
-    d2h_matrix(c, out, n, d + 3 * nn, n, n, n);
+    h2d_matrix(c, d, n, Y, n, n, n);
+    decouple_dev(c, n, d, d + nn, dB2, d + 3 * nn,
+                 [&] { h2d_matrix_x(c, dB2, n, B2, n, n, n); });
+    d2h_matrix(c, out, n, d, n, n, n);
     PSX_HIP(hipStreamSynchronize(c->stream));
   });
 }

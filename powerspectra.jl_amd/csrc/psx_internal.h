@@ -301,8 +301,8 @@ void dgemm_dev(Ctx* c, int m, int n, int k, const double* dA, int64_t lda, const
                int64_t ldb, double* dC, int64_t ldc);
 void lu_solve_dev(Ctx* c, int n, double* dA, int64_t lda, double* dB,
                   int64_t ldb, int nrhs);  // dA overwritten by LU
-void decouple_dev(Ctx* c, int n, const double* dY, double* dB1, double* dB2,
-                  double* dOut);
+void decouple_dev(Ctx* c, int n, double* dY, double* dB1, double* dB2, double* dT,
+                  const std::function<void()>& b2);
 // One of several independent systems A X = B on the device (A overwritten by
 // its LU factors, B by X), with 1 to 4 right-hand sides and ipiv a device
 // array of n + 64 ints (LAPACK interchanges, info slot at n + 32).

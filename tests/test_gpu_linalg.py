@@ -296,3 +296,85 @@ def test_lu_solve_pm_arguments(ctx, pkg):
         ctx.lu_solve_pm(A, A, np.ones(7))
     with pytest.raises(pkg.SingularException):
         ctx.lu_solve_pm(A, A, np.ones(8), 1)
+
+
+def _permuted(A, ipiv):
+    p = np.arange(A.shape[0])
+    for i, q in enumerate(np.asarray(ipiv) - 1):
+        p[i], p[q] = p[q], p[i]
+    return A[p]
+
+
+# either side of every change of the leaf kernel (512 rows a register row, 32,
+# 16 and 8 columns a leaf, the multi-workgroup path above 6144 rows) and of the
+# 256-column panel
+@pytest.mark.parametrize("n", [8, 9, 255, 256, 257, 511, 512, 513, 1024, 1025, 1536, 1537, 2049,
+                               2561, 3072, 3073, 4097, 5121, 6144, 6177])
+def test_lu_factor_at_leaf_edges(ctx, n):
+    A = np.random.default_rng(n).uniform(-1, 1, (n, n))
+    LU, ipiv = ctx.lu_factor(A)
+    L, U = np.tril(LU, -1) + np.eye(n), np.triu(LU)
+    assert np.abs(L).max() <= 1.0
+    # |P A - L U| <= gamma_n |L| |U| for any order of the updates, and as much
+    # again for the product formed here
+    err = np.abs(_permuted(A, ipiv) - L @ U)
+    bound = 2 * n * np.finfo(float).eps * (np.abs(L) @ np.abs(U))
+    assert (err <= bound).all()
+
+
+@pytest.mark.parametrize("n", [40, 300, 1600])
+def test_lu_pivot_ties_zero_columns_and_nan(ctx, n):
+    # every |entry| alike: ties go to the row that came first in the matrix
+    # the leaf started from (the first 8 columns are one leaf); exact arithmetic
+    from fractions import Fraction
+    A = np.where(np.random.default_rng(n).uniform(size=(n, n)) < 0.5, -1.0, 1.0)
+    _, ipiv = ctx.lu_factor(A)
+    M = [[Fraction(int(v)) for v in row[:8]] for row in A]
+    at, free = list(range(n)), set(range(n))     # row at each position
+    for j in range(7):       # (magnitudes 1, 2, 3, 4: exact in doubles too)
+        top = max(abs(M[i][j]) for i in free)
+        p = min(i for i in free if abs(M[i][j]) == top)
+        assert ipiv[j] - 1 == at.index(p)
+        q = at.index(p)
+        at[j], at[q] = at[q], at[j]
+        free.remove(p)
+        for i in free:
+            f = M[i][j] / M[p][j]
+            M[i] = [a - f * b for a, b in zip(M[i], M[p])]
+        if any(v.denominator & (v.denominator - 1) for i in free for v in M[i]):
+            break            # entries no longer doubles
+    # a zero column is reported where LAPACK reports it
+    B = np.random.default_rng(n + 1).uniform(-1, 1, (n, n))
+    B[:, n // 2] = 0.0
+    with pytest.raises(Exception, match=f"position {n // 2 + 1}"):
+        ctx.lu_solve(B, np.ones(n))
+    # a NaN is the pivot of its column and reaches the solution
+    B = np.random.default_rng(n + 2).uniform(-1, 1, (n, n))
+    B[n - 3, 0] = np.nan
+    LU, ipiv = ctx.lu_factor(B)
+    assert ipiv[0] == n - 2
+    assert np.isnan(ctx.lu_solve(B, np.ones(n))).all()
+    # pivots whose reciprocals leave the normal range
+    S = np.random.default_rng(n + 3).uniform(-1, 1, (n, n)) * 2.0 ** -1010
+    x = ctx.lu_solve(S, S @ np.ones(n))
+    ref = np.linalg.solve(S * 2.0 ** 1010, (S * 2.0 ** 1010) @ np.ones(n))
+    cond = np.linalg.cond(S * 2.0 ** 1010)
+    assert np.abs(x - 1).max() <= 1e3 * np.abs(ref - 1).max() + cond * 1e-13
+
+
+@pytest.mark.parametrize("n,m", [(1, 5), (15, 7), (16, 16), (17, 33), (63, 5), (64, 15), (65, 17),
+                                 (240, 16), (255, 31), (256, 5), (257, 18), (511, 6), (513, 65)])
+def test_solve_many_right_hand_sides_at_block_edges(ctx, n, m):
+    rng = np.random.default_rng(n)
+    A = rng.uniform(-1, 1, (n, n))
+    B = rng.uniform(-1, 1, (n, m))
+    X = ctx.lu_solve(A, B)
+    LU, ipiv = ctx.lu_factor(A)
+    L, U = np.tril(LU, -1) + np.eye(n), np.triu(LU)
+    # backward error of substitution with computed factors: |A X - B| <=
+    # 3 gamma_n |P^T L| |U| |X| (Higham, theorem 9.4); doubled for the product here
+    R = np.abs(_permuted(A @ X - B, ipiv))
+    assert (R <= 6 * n * np.finfo(float).eps * (np.abs(L) @ (np.abs(U) @ np.abs(X)))).all()
+    if n > 1 and m == n:
+        Y = rng.uniform(-1, 1, (n, n))
+        assert np.array_equal(ctx.decouple_covmat(Y, A, A), ctx.decouple_covmat(Y, A, A.copy()))
