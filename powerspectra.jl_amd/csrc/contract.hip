@@ -119,8 +119,12 @@ __device__ __forceinline__ double accum(double w, double t, double acc) {
 
 // EPI: EPI_MCM, EPI_COV or EPI_RMAX; COVK: covariance kind for EPI_COV; WPE: minimum
 // waves per SIMD the register allocation must allow; TPB: threads per
-// workgroup (64 per tile).
-template <int R, int N00, int N02, int NPE, int NPO, int EPI, int COVK, int WPE, int TPB>
+// workgroup (64 CS per tile).  CS > 1 splits the sum over c of a tile between CS
+// waves, whose sums are added through LDS: wave p takes the c of every chunk
+// floor(c / kSplitChunk) = p mod CS.  The chunks do not depend on the tile, so
+// every kernel adds the terms of a pair in the same order, whatever its R.
+constexpr int kSplitChunk = 32;
+template <int R, int N00, int N02, int NPE, int NPO, int EPI, int COVK, int WPE, int TPB, int CS>
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(WPE)))
 contract_kernel(KArgs A) {
   constexpr int NV = N00 + N02 + NPE + NPO;
@@ -134,10 +138,13 @@ contract_kernel(KArgs A) {
 
   const int lane = threadIdx.x & 63;
   const int wave = ufl(threadIdx.x >> 6);
+  static_assert(CS == 1 || (kSplitChunk % R == 0 && R % CS == 0), "");
+  constexpr int WG = TPB / 64 / CS;   // tiles per workgroup
   // tile lists come in whole workgroups (padded with empty tiles): every wave
   // of a launched workgroup has a tile and reaches the epilogue's barriers
-  const int tile = ufl(blockIdx.x * (TPB / 64) + wave);
-  if (ufl(blockIdx.x * (TPB / 64)) >= A.ntiles) return;
+  const int part = wave % CS, tw = wave / CS;
+  const int tile = ufl(blockIdx.x * WG + tw);
+  if (ufl(blockIdx.x * WG) >= A.ntiles) return;
   const int x0 = sload(&A.tiles[tile].x0, 0);
   const int S0 = sload(&A.tiles[tile].S0, 0);
   const int own_lo = sload(&A.tiles[tile].lo, 0);
@@ -169,7 +176,8 @@ contract_kernel(KArgs A) {
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[k][r] = 0.0;
 
-  // Walking pointers; step c = cbeg + blk R + u reads
+  // nblocks blocks of R steps from c0 (a multiple of R) on.
+  // Walking pointers; step c = c0 + blk R + u reads
   //   lane:    G[l1 - c] = gl[-u],  Z[l1 - c - 1] = zl[-u]
   //   uniform: gamma_c = sg[u],  z_c = sz[u]
   //   window refill (q = -c - 1): G[t + q] = gwp[-u], Z[t + q - 1] = zwp[-u],
@@ -177,82 +185,94 @@ contract_kernel(KArgs A) {
   //   records: l3 = S0 + r - 2c at rec[(r - 2u) RS]
   // with t = S0 - x0 - lane; every pointer advances once per block.
   const int t = S0 - x0 - lane;
-  const double* gl = A.G + kTabOff + (l1 - cbeg);
-  const double* zl = A.Z + kTabOff + (l1 - cbeg - 1);
-  const double* gwp = A.G + kTabOff + (t - cbeg - 1);
-  const double* zwp = A.Z + kTabOff + (t - cbeg - 2);
-  const double* sg = A.G + kTabOff + cbeg;
-  const double* sz = A.Z + kTabOff + cbeg;
-  const double* sdp = A.D + kTabOff + (S0 - cbeg - 1);
-  const double* sip = A.IG + kTabOff + (S0 - cbeg - 1);
-  const double* rec = A.rec + (int64_t)(kWOff + S0 - 2 * cbeg) * RS;
+  auto steps = [&](const int c0, const int nblocks) {
+    const double* gl = A.G + kTabOff + (l1 - c0);
+    const double* zl = A.Z + kTabOff + (l1 - c0 - 1);
+    const double* gwp = A.G + kTabOff + (t - c0 - 1);
+    const double* zwp = A.Z + kTabOff + (t - c0 - 2);
+    const double* sg = A.G + kTabOff + c0;
+    const double* sz = A.Z + kTabOff + c0;
+    const double* sdp = A.D + kTabOff + (S0 - c0 - 1);
+    const double* sip = A.IG + kTabOff + (S0 - c0 - 1);
+    const double* rec = A.rec + (int64_t)(kWOff + S0 - 2 * c0) * RS;
 
-  // sliding windows: slot r at step c needs (q = r - c)
-  //   gw: gamma_{t+q} delta_{S0+q},  zw: z_{t+q-1} igamma_{S0+q},
-  // held at index q mod R (cbeg % R == 0).
-  double gw[kG ? R : 1], zw[kZ ? R : 1];
+    // sliding windows: slot r at step c needs (q = r - c)
+    //   gw: gamma_{t+q} delta_{S0+q},  zw: z_{t+q-1} igamma_{S0+q},
+    // held at index q mod R (c0 % R == 0).
+    double gw[kG ? R : 1], zw[kZ ? R : 1];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if constexpr (kG) gw[r] = gwp[r + 1] * sload(sdp, r + 1);
-    if constexpr (kZ) zw[r] = zwp[r + 1] * sload(sip, r + 1);
-  }
-
-  for (int blk = 0; blk < nblk; ++blk) {
-#pragma unroll
-    for (int u = 0; u < R; ++u) {
-      double g1 = 0.0, z1 = 0.0;
-      if constexpr (kG) g1 = gl[-u] * sload(sg, u);
-      if constexpr (kZ) z1 = zl[-u] * sload(sz, u);
-      const double* ru = rec - 2 * u * RS;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int wi = ((r - u) % R + R) % R;
-        const double* rr = ru + r * RS;
-        double p = 0.0, Q = 0.0;
-        if constexpr (kG) p = g1 * gw[wi];
-        if constexpr (kE) {
-          const double E = sig[r] - sload(rr, FT);
-          Q = fma(E, E, -kap[r]);
-        }
-#pragma unroll
-        for (int k = 0; k < N00; ++k) acc[k][r] = accum<EPI>(sload(rr, k), p, acc[k][r]);
-        double pq = 0.0;
-        if constexpr (N02 > 0) {
-          pq = p * Q;
-#pragma unroll
-          for (int k = 0; k < N02; ++k)
-            acc[N00 + k][r] = accum<EPI>(sload(rr, N00 + k), pq, acc[N00 + k][r]);
-        }
-        if constexpr (NPE > 0) {
-          const double pqq = (N02 > 0 ? pq : p * Q) * Q;
-#pragma unroll
-          for (int k = 0; k < NPE; ++k)
-            acc[N00 + N02 + k][r] =
-                accum<EPI>(sload(rr, N00 + N02 + k), pqq, acc[N00 + N02 + k][r]);
-        }
-        if constexpr (NPO > 0) {
-          const double D1 = sig[r] - sload(rr, FT1);
-          const double pd = (z1 * zw[wi]) * (D1 * D1);
-#pragma unroll
-          for (int k = 0; k < NPO; ++k)
-            acc[NE + k][r] = accum<EPI>(sload(rr, NE + k), pd, acc[NE + k][r]);
-        }
-      }
-      // advance the windows to step c + 1: the slot that held r = R-1 now
-      // receives q = -c - 1
-      const int ni = (R - 1 - u) % R;
-      if constexpr (kG) gw[ni] = gwp[-u] * sload(sdp, -u);
-      if constexpr (kZ) zw[ni] = zwp[-u] * sload(sip, -u);
+    for (int r = 0; r < R; ++r) {
+      if constexpr (kG) gw[r] = gwp[r + 1] * sload(sdp, r + 1);
+      if constexpr (kZ) zw[r] = zwp[r + 1] * sload(sip, r + 1);
     }
-    gl -= R;
-    zl -= R;
-    gwp -= R;
-    zwp -= R;
-    sg += R;
-    sz += R;
-    sdp -= R;
-    sip -= R;
-    rec -= 2 * R * RS;
+
+    for (int blk = 0; blk < nblocks; ++blk) {
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        double g1 = 0.0, z1 = 0.0;
+        if constexpr (kG) g1 = gl[-u] * sload(sg, u);
+        if constexpr (kZ) z1 = zl[-u] * sload(sz, u);
+        const double* ru = rec - 2 * u * RS;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int wi = ((r - u) % R + R) % R;
+          const double* rr = ru + r * RS;
+          double p = 0.0, Q = 0.0;
+          if constexpr (kG) p = g1 * gw[wi];
+          if constexpr (kE) {
+            const double E = sig[r] - sload(rr, FT);
+            Q = fma(E, E, -kap[r]);
+          }
+#pragma unroll
+          for (int k = 0; k < N00; ++k) acc[k][r] = accum<EPI>(sload(rr, k), p, acc[k][r]);
+          double pq = 0.0;
+          if constexpr (N02 > 0) {
+            pq = p * Q;
+#pragma unroll
+            for (int k = 0; k < N02; ++k)
+              acc[N00 + k][r] = accum<EPI>(sload(rr, N00 + k), pq, acc[N00 + k][r]);
+          }
+          if constexpr (NPE > 0) {
+            const double pqq = (N02 > 0 ? pq : p * Q) * Q;
+#pragma unroll
+            for (int k = 0; k < NPE; ++k)
+              acc[N00 + N02 + k][r] =
+                  accum<EPI>(sload(rr, N00 + N02 + k), pqq, acc[N00 + N02 + k][r]);
+          }
+          if constexpr (NPO > 0) {
+            const double D1 = sig[r] - sload(rr, FT1);
+            const double pd = (z1 * zw[wi]) * (D1 * D1);
+#pragma unroll
+            for (int k = 0; k < NPO; ++k)
+              acc[NE + k][r] = accum<EPI>(sload(rr, NE + k), pd, acc[NE + k][r]);
+          }
+        }
+        // advance the windows to step c + 1: the slot that held r = R-1 now
+        // receives q = -c - 1
+        const int ni = (R - 1 - u) % R;
+        if constexpr (kG) gw[ni] = gwp[-u] * sload(sdp, -u);
+        if constexpr (kZ) zw[ni] = zwp[-u] * sload(sip, -u);
+      }
+      gl -= R;
+      zl -= R;
+      gwp -= R;
+      zwp -= R;
+      sg += R;
+      sz += R;
+      sdp -= R;
+      sip -= R;
+      rec -= 2 * R * RS;
+    }
+  };
+  if constexpr (CS == 1) {
+    steps(cbeg, nblk);
+  } else {
+    const int cend = cbeg + nblk * R;
+    for (int ch = cbeg / kSplitChunk; ch * kSplitChunk < cend; ++ch) {
+      if (ch % CS != part) continue;
+      const int c0 = ufl(max(cbeg, ch * kSplitChunk));
+      steps(c0, ufl((min(cend, (ch + 1) * kSplitChunk) - c0) / R));
+    }
   }
 
   // ---- epilogue ----
@@ -268,51 +288,89 @@ contract_kernel(KArgs A) {
     return;
   }
   // The workgroup's tiles are one row chunk over WG R consecutive
-  // anti-diagonals: S0 of wave w = S0 of wave 0 + w R, empty tiles (hi < lo)
+  // anti-diagonals: S0 of tile w = S0 of tile 0 + w R, empty tiles (hi < lo)
   // last (checked on the host).  Each output matrix goes through LDS and
   // leaves as column segments: column l1 takes rows l2 = S - l1 (the mirrored
   // element) and column l2 rows l1 = S - l2 (the direct one) over the span of
   // anti-diagonals, consecutive threads on consecutive rows, instead of one
   // scattered 8-byte store per lane.
-  constexpr int WG = TPB / 64, SPAN = WG * R, CPP = TPB / SPAN;
+  constexpr int SPAN = WG * R, CPP = TPB / SPAN;
   static_assert(TPB % SPAN == 0, "anti-diagonal span must divide the workgroup");
-  __shared__ double xs[WG][R][64];
+  constexpr int KC = CS == 1 ? 1 : NV < 4 ? NV : 4;  // outputs through LDS at a time
+  __shared__ double xs[WG][CS][KC][R][64];
   __shared__ int tinfo[WG][4];
   const int lmin = A.lmin;
-  if (lane == 0) {
-    tinfo[wave][0] = x0;
-    tinfo[wave][1] = S0;
-    tinfo[wave][2] = own_lo;
-    tinfo[wave][3] = own_hi;
+  if (lane == 0 && part == 0) {
+    tinfo[tw][0] = x0;
+    tinfo[tw][1] = S0;
+    tinfo[tw][2] = own_lo;
+    tinfo[tw][3] = own_hi;
+  }
+  // from here on a wave holds the RO slots r = part + CS rr
+  constexpr int RO = R / CS;
+  double fin[NV][RO];
+  if constexpr (CS == 1) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+      for (int r = 0; r < R; ++r) fin[k][r] = acc[k][r];
+  } else {
+#pragma unroll
+    for (int k0 = 0; k0 < NV; k0 += KC) {
+#pragma unroll
+      for (int k = k0; k < NV && k < k0 + KC; ++k)
+#pragma unroll
+        for (int r = 0; r < R; ++r) xs[tw][part][k - k0][r][lane] = acc[k][r];
+      __syncthreads();
+#pragma unroll
+      for (int k = k0; k < NV && k < k0 + KC; ++k)
+#pragma unroll
+        for (int rr = 0; rr < RO; ++rr) {
+          // the parts added with their rounding errors kept: one rounding
+          // more than the parts' own sums have (against long double at lmax
+          // 400 the largest element error falls from 9.5e-16 to 6.4e-16 for
+          // TT and from 1.4e-15 to 6.7e-16 for --)
+          double v = xs[tw][0][k - k0][part + CS * rr][lane], e = 0.0;
+#pragma unroll
+          for (int q = 1; q < CS; ++q) {
+            const double x = xs[tw][q][k - k0][part + CS * rr][lane];
+            const double sum = v + x, z = sum - v;
+            e += (v - (sum - z)) + (x - z);
+            v = sum;
+          }
+          v += e;
+          fin[k][rr] = v;
+        }
+      __syncthreads();
+    }
   }
   const double L1 = (double)l1;
   const double pi1 = (L1 - 1.0) * L1 * (L1 + 1.0) * (L1 + 2.0);
-  double k02r[kE ? R : 1], k22r[(NPE + NPO) > 0 ? R : 1];
+  double k02r[kE ? RO : 1], k22r[(NPE + NPO) > 0 ? RO : 1];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int l2 = S0 + r - l1;
+  for (int rr = 0; rr < RO; ++rr) {
+    const int l2 = S0 + part + CS * rr - l1;
     const double L2 = (double)l2;
     const double pi2 = (L2 - 1.0) * L2 * (L2 + 1.0) * (L2 + 2.0);
     const bool spin2 = (l1 >= 2) && (l2 >= 2);
-    if constexpr (kE) k02r[r] = spin2 ? 1.0 / (2.0 * sqrt(pi1 * pi2)) : 0.0;
-    if constexpr ((NPE + NPO) > 0) k22r[r] = spin2 ? 1.0 / (4.0 * pi1 * pi2) : 0.0;
+    if constexpr (kE) k02r[rr] = spin2 ? 1.0 / (2.0 * sqrt(pi1 * pi2)) : 0.0;
+    if constexpr ((NPE + NPO) > 0) k22r[rr] = spin2 ? 1.0 / (4.0 * pi1 * pi2) : 0.0;
   }
   bool bad = false;
   // the value of pair (l1, S - l1) if this workgroup computed and owns it
-  auto staged = [&](int S, int m1, double& v) -> bool {
+  auto staged = [&](int q, int S, int m1, double& v) -> bool {
     const int i = S - tinfo[0][1];
     if (i < 0 || i >= SPAN) return false;
     const int w = i / R, r = i - w * R;
     if (m1 < tinfo[w][2] || m1 > tinfo[w][3]) return false;
     const int m2 = S - m1;
     if (m1 < lmin || m1 > m2 || m2 > lmax) return false;
-    v = xs[w][r][m1 - tinfo[w][0]];
+    v = xs[w][0][q][r][m1 - tinfo[w][0]];
     return true;
   };
   // column segments of one output matrix; MCM weights (2 l2 + 1) on the
   // direct element, (2 l1 + 1) on the mirrored one, none for covariance
-  auto store = [&](double* o, bool weighted) {
-    __syncthreads();
+  auto store = [&](double* o, int q, bool weighted) {
     int l1lo = lmax + 1, l1hi = -1;
 #pragma unroll
     for (int w = 0; w < WG; ++w)
@@ -325,36 +383,40 @@ contract_kernel(KArgs A) {
     const int S = s0 + i;
     for (int m1 = l1lo + cs; m1 <= l1hi; m1 += CPP) {
       double v;
-      if (staged(S, m1, v))
+      if (staged(q, S, m1, v))
         o[(int64_t)(S - m1 - lmin) + (int64_t)(m1 - lmin) * A.ldo] =
             weighted ? (2.0 * (double)m1 + 1.0) * v : v;
     }
     for (int m2 = s0 - l1hi + cs; m2 <= s0 + SPAN - 1 - l1lo; m2 += CPP) {
       double v;
-      if (staged(S, S - m2, v))
+      if (staged(q, S, S - m2, v))
         o[(int64_t)(S - m2 - lmin) + (int64_t)(m2 - lmin) * A.ldo] =
             weighted ? (2.0 * (double)m2 + 1.0) * v : v;
     }
-    __syncthreads();
   };
   if constexpr (EPI == EPI_MCM) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
+    for (int k0 = 0; k0 < NV; k0 += KC) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        double kap_k = 1.0;
-        if constexpr (N02 > 0)
-          if (k >= N00 && k < N00 + N02) kap_k = k02r[r];
-        if constexpr ((NPE + NPO) > 0)
-          if (k >= N00 + N02) kap_k = k22r[r];
-        xs[wave][r][lane] = kap_k * acc[k][r];
-      }
-      store(A.out[k], true);
+      for (int k = k0; k < NV && k < k0 + KC; ++k)
+#pragma unroll
+        for (int rr = 0; rr < RO; ++rr) {
+          double kap_k = 1.0;
+          if constexpr (N02 > 0)
+            if (k >= N00 && k < N00 + N02) kap_k = k02r[rr];
+          if constexpr ((NPE + NPO) > 0)
+            if (k >= N00 + N02) kap_k = k22r[rr];
+          xs[tw][0][k - k0][part + CS * rr][lane] = kap_k * fin[k][rr];
+        }
+      __syncthreads();
+#pragma unroll 1
+      for (int k = k0; k < NV && k < k0 + KC; ++k) store(A.out[k], k - k0, true);
+      __syncthreads();
     }
   } else {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int l2 = S0 + r - l1;
+    for (int rr = 0; rr < RO; ++rr) {
+      const int r = part + CS * rr, l2 = S0 + r - l1;
       double v = 0.0;
       if (!(l1 < own_lo || l1 > own_hi || l1 < lmin || l1 > l2 || l2 > lmax)) {
         double xi[NV];
@@ -362,16 +424,17 @@ contract_kernel(KArgs A) {
         for (int k = 0; k < NV; ++k) {
           double kap_k = 1.0;
           if constexpr (N02 > 0)
-            if (k >= N00 && k < N00 + N02) kap_k = k02r[r];
+            if (k >= N00 && k < N00 + N02) kap_k = k02r[rr];
           if constexpr ((NPE + NPO) > 0)
-            if (k >= N00 + N02) kap_k = k22r[r];
-          xi[k] = kap_k * acc[k][r];
+            if (k >= N00 + N02) kap_k = k22r[rr];
+          xi[k] = kap_k * fin[k][rr];
         }
         v = cov_combine<COVK>(l1, l2, xi, A.spec, A.ratio, bad);
       }
-      xs[wave][r][lane] = v;
+      xs[tw][0][0][r][lane] = v;
     }
-    store(A.out[0], false);
+    __syncthreads();
+    store(A.out[0], 0, false);
     if (bad) atomicOr(A.err, 1);
   }
 }
@@ -498,6 +561,14 @@ std::vector<Tile> make_tiles(int lmin, int lmax, int LW, int R, int waves) {
     if (w < nwg) perm.push_back((int)w);
     if (b > 4 * nwg + 64 * kXcds * kRun) break;  // unreachable guard
   }
+  // A split block's workgroups are nearly all resident at once, a CU holding
+  // every kCus-th of the list: reverse every other run of that many, so that
+  // the CU with the longest of one run has the shortest of the next (3 % at
+  // lmax 767).
+  constexpr int kCus = 256;
+  if (waves == 1)
+    for (int r0 = kCus; r0 < nwg; r0 += 2 * kCus)
+      std::reverse(perm.begin() + r0, perm.begin() + std::min(nwg, r0 + kCus));
   // every workgroup occupies exactly `waves` slots; short groups are padded
   // with empty tiles (hi = -1 < lo: no lane owns anything, no c step runs)
   std::vector<Tile> out;
@@ -682,7 +753,8 @@ using KernelFn = void (*)(KArgs);
 
 struct Config {
   int R;
-  int waves;  // per workgroup
+  int waves;    // tiles per workgroup
+  int threads;  // per workgroup
   KernelFn fn;
   const char* name;
 };
@@ -690,8 +762,14 @@ struct Config {
 template <int R, int N00, int N02, int NPE, int NPO, int EPI, int COVK, int WPE = 1,
           int WAVES = 4>
 Config cfg(const char* name) {
-  return Config{R, WAVES, contract_kernel<R, N00, N02, NPE, NPO, EPI, COVK, WPE, 64 * WAVES>,
-                name};
+  return Config{R, WAVES, 64 * WAVES,
+                contract_kernel<R, N00, N02, NPE, NPO, EPI, COVK, WPE, 64 * WAVES, 1>, name};
+}
+
+// one tile a workgroup, its sum over c split between four waves
+template <int R, int N00, int N02, int NPE, int NPO, int EPI, int COVK, int WPE = 1>
+Config cfg_split(const char* name) {
+  return Config{R, 1, 256, contract_kernel<R, N00, N02, NPE, NPO, EPI, COVK, WPE, 256, 4>, name};
 }
 
 // Anti-diagonals per tile (R) and minimum waves per SIMD for each kernel,
@@ -736,6 +814,82 @@ Config cfg(const char* name) {
 #define PSX_WAVES_SET 4
 #endif
 
+// Blocks of up to kSplitRows rows split each tile's sum over c between the
+// four waves of a workgroup that has no other tile.  Unsplit, such a block has
+// too few workgroups to share out: at lmax 767 the set's 288 workgroups of
+// four tiles put 88 us of issue on the CU with the longest against 33 us on
+// average.  Split, every kernel is faster up to there (TT, TE, ++, --, fused
+// ++/--, set, TTTT in us, unsplit / split: lmax 191 15/8 28/9 30/9 28/9 42/16
+// 58/21 54/38, lmax 767 29/14 59/22 66/23 58/22 82/41 122/58 85/61, lmax 1535
+// 60/52 120/98 139/113 118/94 230/213 310/281 204/200) and at lmax 2047 the
+// large ones are 5 % slower.  The line depends on the block's size alone: what
+// is computed alone, in a set or in a batch adds its terms in one order.
+constexpr int kSplitRows = 1600;
+// The spin-2 single blocks take 4 anti-diagonals a tile up to kSplitNarrow rows
+// (lmax 511: 13 us against 16 with 8), 8 above (lmax 1535: 98 against 102);
+// TT takes 8 throughout (lmax 767: 14 against 16 with 4).
+constexpr int kSplitNarrow = 1024;
+
+bool split_sums(const ContractRequest& rq) {
+  return rq.epi != EPI_RMAX && rq.lmax - rq.lmin + 1 <= kSplitRows;
+}
+
+Config pick_split_config(const ContractRequest& rq) {
+  const int* f = rq.nfam;
+  const bool narrow = rq.lmax - rq.lmin + 1 <= kSplitNarrow;
+  if (rq.epi == EPI_MCM) {
+    if (f[0] == 1 && f[1] == 0 && f[2] == 0 && f[3] == 0)
+      return cfg_split<8, 1, 0, 0, 0, EPI_MCM, 0>("psx_mcm_00");
+    if (f[0] == 0 && f[1] == 1 && f[2] == 0 && f[3] == 0)
+      return narrow ? cfg_split<4, 0, 1, 0, 0, EPI_MCM, 0>("psx_mcm_02")
+                    : cfg_split<8, 0, 1, 0, 0, EPI_MCM, 0>("psx_mcm_02");
+    if (f[0] == 0 && f[1] == 0 && f[2] == 1 && f[3] == 0)
+      return narrow ? cfg_split<4, 0, 0, 1, 0, EPI_MCM, 0>("psx_mcm_pp")
+                    : cfg_split<8, 0, 0, 1, 0, EPI_MCM, 0>("psx_mcm_pp");
+    if (f[0] == 0 && f[1] == 0 && f[2] == 0 && f[3] == 1)
+      return narrow ? cfg_split<4, 0, 0, 0, 1, EPI_MCM, 0>("psx_mcm_mm")
+                    : cfg_split<8, 0, 0, 0, 1, EPI_MCM, 0>("psx_mcm_mm");
+    if (f[0] == 0 && f[1] == 0 && f[2] == 1 && f[3] == 1)
+      return cfg_split<4, 0, 0, 1, 1, EPI_MCM, 0>("psx_mcm_pm");
+    if (f[0] == 1 && f[1] == 2 && f[2] == 1 && f[3] == 1)
+      return cfg_split<4, 1, 2, 1, 1, EPI_MCM, 0, 4>("psx_mcm_set");
+    if (f[0] == 1 && f[1] == 1 && f[2] == 1 && f[3] == 1)
+      return cfg_split<4, 1, 1, 1, 1, EPI_MCM, 0, 4>("psx_mcm_set1");
+    if (f[1] == 0 && f[2] == 0 && f[3] == 0) {
+      if (f[0] == 2) return cfg_split<4, 2, 0, 0, 0, EPI_MCM, 0>("psx_mcm_group");
+      if (f[0] == 4) return cfg_split<4, 4, 0, 0, 0, EPI_MCM, 0>("psx_mcm_group");
+      if (f[0] == 8) return cfg_split<4, 8, 0, 0, 0, EPI_MCM, 0>("psx_mcm_group");
+    }
+    if (f[0] == 0 && f[2] == 0 && f[3] == 0) {
+      if (f[1] == 2) return cfg_split<4, 0, 2, 0, 0, EPI_MCM, 0>("psx_mcm_group");
+      if (f[1] == 4) return cfg_split<4, 0, 4, 0, 0, EPI_MCM, 0>("psx_mcm_group");
+      if (f[1] == 8) return cfg_split<4, 0, 8, 0, 0, EPI_MCM, 0>("psx_mcm_group");
+    }
+    if (f[0] == 0 && f[1] == 0 && f[3] == 0) {
+      if (f[2] == 2) return cfg_split<4, 0, 0, 2, 0, EPI_MCM, 0>("psx_mcm_group");
+      if (f[2] == 4) return cfg_split<4, 0, 0, 4, 0, EPI_MCM, 0>("psx_mcm_group");
+      if (f[2] == 8) return cfg_split<4, 0, 0, 8, 0, EPI_MCM, 0>("psx_mcm_group");
+    }
+    if (f[0] == 0 && f[1] == 0 && f[2] == 0) {
+      if (f[3] == 2) return cfg_split<4, 0, 0, 0, 2, EPI_MCM, 0>("psx_mcm_group");
+      if (f[3] == 4) return cfg_split<4, 0, 0, 0, 4, EPI_MCM, 0>("psx_mcm_group");
+      if (f[3] == 8) return cfg_split<4, 0, 0, 0, 8, EPI_MCM, 0>("psx_mcm_group");
+    }
+  } else {
+    switch (rq.cov_kind) {
+      case PSX_COV_TTTT: return cfg_split<4, 8, 0, 0, 0, EPI_COV, PSX_COV_TTTT>("psx_cov_tttt");
+      case PSX_COV_EEEE: return cfg_split<4, 0, 0, 8, 0, EPI_COV, PSX_COV_EEEE>("psx_cov_eeee");
+      case PSX_COV_TTTE: return cfg_split<4, 4, 0, 0, 0, EPI_COV, PSX_COV_TTTE>("psx_cov_ttte");
+      case PSX_COV_TETE: return cfg_split<4, 1, 4, 0, 0, EPI_COV, PSX_COV_TETE>("psx_cov_tete");
+      case PSX_COV_TEEE: return cfg_split<4, 0, 4, 0, 0, EPI_COV, PSX_COV_TEEE>("psx_cov_teee");
+      case PSX_COV_TEEE_PLANCK:
+        return cfg_split<4, 0, 0, 4, 0, EPI_COV, PSX_COV_TEEE_PLANCK>("psx_cov_teee_planck");
+      case PSX_COV_TTEE: return cfg_split<4, 2, 0, 0, 0, EPI_COV, PSX_COV_TTEE>("psx_cov_ttee");
+    }
+  }
+  throw Error{PSX_ERR_ARGUMENT, "unsupported contraction configuration"};
+}
+
 Config pick_config(const ContractRequest& rq) {
   const int* f = rq.nfam;
   if (rq.epi == EPI_RMAX) {
@@ -751,6 +905,7 @@ Config pick_config(const ContractRequest& rq) {
       return cfg<8, 0, 0, 0, 1, EPI_RMAX, 0>("psx_rowmax");
     throw Error{PSX_ERR_ARGUMENT, "row maxima of one family only"};
   }
+  if (split_sums(rq)) return pick_split_config(rq);
   if (rq.epi == EPI_MCM) {
     if (f[0] == 1 && f[1] == 0 && f[2] == 0 && f[3] == 0) {
       // TT: 8 anti-diagonals per tile up to 4096 rows (5 % faster at lmax 3071),
@@ -925,7 +1080,7 @@ static int* run_contraction_checked(Ctx* c, const ContractRequest& rq, hipStream
     }
   }
   ka.err = err;
-  const int threads = 64 * cf.waves;
+  const int threads = cf.threads;
   if (band_done) {
     // every band on s, an event after each (one timed region for all)
     PSX_REQUIRE(s == c->stream && tl.bands.size() <= kMaxBands, PSX_ERR_ARGUMENT,
@@ -1164,7 +1319,7 @@ void run_contraction_noalloc(Ctx* c, const ContractRequest& rq0) {
   ka.out[0] = rq.dout[0];
   ka.err = nullptr;
   const unsigned blocks = (unsigned)((ka.ntiles + cf.waves - 1) / cf.waves);
-  hipLaunchKernelGGL(cf.fn, dim3(blocks), dim3(64 * cf.waves), 0, c->stream, ka);
+  hipLaunchKernelGGL(cf.fn, dim3(blocks), dim3(cf.threads), 0, c->stream, ka);
   PSX_HIP(hipGetLastError());
 }
 

@@ -141,3 +141,47 @@ def test_reference_namaster_diagonals_gpu(ctx):
     assert np.max(np.abs(dtt - tt) / np.abs(tt)) < 1e-12
     assert np.max(np.abs(dee - ee) / np.abs(ee)) < 5e-7
     assert np.max(np.abs(dte - te) / np.abs(te)) < 5e-7
+
+
+# either side of the block sizes where the sum over c stops being split between
+# a workgroup's waves and where the spin-2 blocks change their tile height
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 1599, 1600, 1601])
+def test_rows_and_set_at_split_edges(ctx, oracle, n):
+    lmin = 3
+    lmax = lmin + n - 1
+    W = mask_like_W(lmax + 1, seed=n)
+    singles = [ctx.mcm(kind, lmin, lmax, W) for kind in KINDS]
+    for kind, M in zip(KINDS, singles):
+        for l1 in (lmin, lmin + n // 3, lmax - 40, lmax):
+            row = lambda k, w: oracle.mcm_rows(k, lmin, lmax, l1, l1, w, precision=1)[l1 - lmin]
+            # n terms, each good to a few ulp, summed in any order: (n + 20) eps
+            # times the sum of their magnitudes (Cauchy-Schwarz for the mixed family)
+            mag = (np.sqrt(row(0, np.abs(W)) * row(2, np.abs(W))) if kind == 1
+                   else row(kind, np.abs(W)))
+            R = row(kind, W)
+            ok = np.isfinite(R)
+            err = np.abs(M[l1 - lmin] - R)[ok]
+            assert (err <= (n + 20) * np.finfo(float).eps * mag[ok]).all(), (kind, n, l1)
+    # a block's terms are added in one order, alone, in a pair, a set or a batch
+    outs = ctx.mcm_set(lmin, lmax, W, W, W, W)
+    for o, k in zip(outs, (0, 1, 1, 2, 3)):
+        assert rel_err(o, singles[k]) <= 1e-15
+    for kind in KINDS:
+        for o in ctx.mcm_batch(kind, lmin, lmax, [W] * 3):
+            assert np.array_equal(o, singles[kind])
+
+
+@pytest.mark.parametrize("kind", range(7))
+@pytest.mark.parametrize("n", [31, 33, 65, 130, 1600, 1601])
+def test_cov_rows_at_split_edges(ctx, oracle, kind, n):
+    from helpers import spectra_set
+    nW, nS, nR = oracle.COV_ARITY[kind]
+    lmin = 2
+    lmax = lmin + n - 1
+    S, R = spectra_set(lmax, seed=kind)
+    W = [mask_like_W(lmax + 1, seed=k) for k in range(nW)]
+    C = ctx.cov(kind, lmin, lmax, S[:nS], R[:nR], W)
+    for l1 in (lmin, lmin + n // 2, lmax):
+        ref = oracle.cov(kind, lmin, lmax, S[:nS], R[:nR], W, rows=(l1, l1))[l1 - lmin]
+        e = rel_err(C[l1 - lmin], ref)
+        assert e <= RTOL_FP64, (kind, n, l1, e)
