@@ -58,9 +58,20 @@ void check_block(int lmin, int lmax, int64_t LW, int64_t ld) {
               "leading dimension smaller than lmax-lmin+1");
 }
 
-void h2d(Ctx* c, void* dst, const void* src, size_t bytes) {
-  PSX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
-}
+// Host arrays into pieces already carved from one device buffer, in one copy
+// where they are small.
+struct Upload {
+  Ctx* c;
+  char* base = nullptr;
+  std::vector<HostPiece> pieces;
+  void add(void* dst, const void* src, size_t bytes) {
+    if (!base) base = (char*)dst;
+    pieces.push_back({src, bytes, (size_t)((char*)dst - base)});
+  }
+  void send() {
+    if (base) h2d_pieces(c, base, pieces);
+  }
+};
 
 ContractRequest block_request(int lmin, int lmax, int64_t LW, int64_t ld) {
   ContractRequest rq;
@@ -291,7 +302,7 @@ int psx_mcm(psx_ctx* h, int kind, int lmin, int lmax, const double* W, int64_t L
     XferBuf x(c, xfer_bytes({wb, mb}));
     double* dW = x.take(wb);
     double* dM = x.take(mb);
-    h2d(c, dW, W, wb);
+    h2d_pieces(c, dW, {{W, wb, 0}});
     run_contraction_to_host(c, mcm_request(kind, lmin, lmax, dW, LW, dM, n), &M, ldM);
   });
 }
@@ -317,7 +328,7 @@ int psx_mcm_binned(psx_ctx* h, int kind, int lmin, int lmax, const double* W, in
     double* dQ = x.take(qb);
     double* dT = x.take(pb);
     double* dO = x.take(ob);
-    h2d(c, dW, W, wb);
+    h2d_pieces(c, dW, {{W, wb, 0}});
     h2d_matrix(c, dP, nbl, P, nbl, nbl, n);
     h2d_matrix(c, dQ, n, Q, n, n, nbr);
     run_contraction(c, mcm_request(kind, lmin, lmax, dW, LW, dM, n));
@@ -351,7 +362,7 @@ int psx_mcm_pm(psx_ctx* h, int lmin, int lmax, const double* W, int64_t LW,
     double* dW = x.take(wb);
     double* dP = x.take(mb);
     double* dQ = x.take(mb);
-    h2d(c, dW, W, wb);
+    h2d_pieces(c, dW, {{W, wb, 0}});
     double* const host[2] = {Mpp, Mmm};
     run_contraction_to_host(c, pm_request(lmin, lmax, dW, LW, dP, dQ, n), host, ldM);
   });
@@ -404,10 +415,12 @@ int psx_mcm_set(psx_ctx* h, int lmin, int lmax, int64_t LW, const double* W_TT,
     XferBuf x(c, xfer_bytes({wb, wb, wb, wb, mb, mb, mb, mb, mb}));
     double* dWp[4];
     double* dMp[5];
+    Upload up{c};
     for (int k = 0; k < 4; ++k) {
       dWp[k] = x.take(wb);
-      if (Wh[k]) h2d(c, dWp[k], Wh[k], wb);
+      if (Wh[k]) up.add(dWp[k], Wh[k], wb);
     }
+    up.send();
     for (int k = 0; k < 5; ++k) dMp[k] = x.take(mb);
     if (W_TT && W_TE && W_ET && W_PP) {
       run_contraction_to_host(c, set_request(lmin, lmax, LW, dWp, dMp, n), Mh, ldM);
@@ -446,10 +459,12 @@ int psx_master_decouple(psx_ctx* h, int lmin, int lmax, int64_t LW, const double
     XferBuf x(c, xfer_bytes({wb, wb, wb, wb, tb, tb, tb, ab, bb, pb, pb, pb, pb}));
     const double* Wh[4] = {W_TT, W_TE, W_ET, W_PP};
     double* dW[4];
+    Upload up{c};
     for (int k = 0; k < 4; ++k) {
       dW[k] = x.take(wb);
-      h2d(c, dW[k], Wh[k], wb);
+      up.add(dW[k], Wh[k], wb);
     }
+    up.send();
     double* dTT = x.take(tb);
     double* dTE = x.take(tb);
     double* dET = x.take(tb);
@@ -470,7 +485,7 @@ int psx_master_decouple(psx_ctx* h, int lmin, int lmax, int64_t LW, const double
     // solves [M++ -M--; -M-- M++] = D [M++ M--; M-- M++] D, D = diag(I, -I)
     std::vector<double> rhs(pcl, pcl + 9 * (size_t)n);
     for (int i = 0; i < n; ++i) rhs[8 * (size_t)n + i] = -rhs[8 * (size_t)n + i];
-    h2d(c, dB, rhs.data(), bb);
+    h2d_pieces(c, dB, {{rhs.data(), bb, 0}});
     const LuSystem sys[4] = {
         {N, dA, N, dB + 5 * (size_t)n, N, 2, piv[0]},   // EE, BB | EB, -BE
         {n, dTT, N, dB, n, 1, piv[1]},                  // TT
@@ -478,8 +493,7 @@ int psx_master_decouple(psx_ctx* h, int lmin, int lmax, int64_t LW, const double
         {n, dET, N, dB + 3 * (size_t)n, n, 2, piv[3]},  // ET | BT
     };
     lu_solve_concurrent(c, sys, 4);
-    PSX_HIP(hipMemcpyAsync(rhs.data(), dB, bb, hipMemcpyDeviceToHost, c->stream));
-    PSX_HIP(hipStreamSynchronize(c->stream));
+    d2h_matrix(c, rhs.data(), 9 * (int64_t)n, dB, 9 * (int64_t)n, 9 * (int64_t)n, 1);
     for (int i = 0; i < n; ++i) rhs[8 * (size_t)n + i] = -rhs[8 * (size_t)n + i];
     std::copy(rhs.begin(), rhs.end(), out);
   });
@@ -527,18 +541,20 @@ int psx_cov(psx_ctx* h, int kind, int lmin, int lmax, const double* const* spect
     const double* ds[4] = {nullptr, nullptr, nullptr, nullptr};
     const double* dr[4] = {nullptr, nullptr, nullptr, nullptr};
     const double* dw[8] = {nullptr};
+    Upload up{c};
     for (int i = 0; i < nS; ++i, p += sb) {
-      h2d(c, p, spectra[i], sb);
+      up.add(p, spectra[i], sb);
       ds[i] = (const double*)p;
     }
     for (int i = 0; i < nR; ++i, p += sb) {
-      h2d(c, p, ratios[i], sb);
+      up.add(p, ratios[i], sb);
       dr[i] = (const double*)p;
     }
     for (int i = 0; i < nW; ++i, p += wb) {
-      h2d(c, p, W[i], wb);
+      up.add(p, W[i], wb);
       dw[i] = (const double*)p;
     }
+    up.send();
     ContractRequest rq = cov_request(kind, lmin, lmax, ds, dr, dw, LW, precision, dC, n);
     if (precision != PSX_FP64) {
       double* const outs[1] = {dC};
@@ -584,11 +600,13 @@ int psx_mcm_batch(psx_ctx* h, int kind, int lmin, int lmax, int K, const double*
     XferBuf x(c, total);
     std::vector<const double*> dW(K);
     std::vector<double*> dM(K);
+    Upload up{c};
     for (int k = 0; k < K; ++k) {
       double* d = x.take(wb);
-      h2d(c, d, W[k], wb);
+      up.add(d, W[k], wb);
       dW[k] = d;
     }
+    up.send();
     for (int k = 0; k < K; ++k) dM[k] = x.take(mb);
     mcm_batch_dev(c, kind, lmin, lmax, K, dW.data(), LW, precision, dM.data(), n);
     std::vector<D2HMatrix> out;
@@ -639,21 +657,23 @@ int psx_cov_batch(psx_ctx* h, int kind, int lmin, int lmax, int nblk,
     std::vector<const double*> ds((size_t)nblk * nS), dr((size_t)nblk * nR),
         dw((size_t)nblk * nW);
     std::vector<double*> dc(nblk);
+    Upload up{c};
     for (size_t i = 0; i < ds.size(); ++i) {
       double* d = x.take(sb);
-      h2d(c, d, spectra[i], sb);
+      up.add(d, spectra[i], sb);
       ds[i] = d;
     }
     for (size_t i = 0; i < dr.size(); ++i) {
       double* d = x.take(sb);
-      h2d(c, d, ratios[i], sb);
+      up.add(d, ratios[i], sb);
       dr[i] = d;
     }
     for (size_t i = 0; i < dw.size(); ++i) {
       double* d = x.take(wb);
-      h2d(c, d, W[i], wb);
+      up.add(d, W[i], wb);
       dw[i] = d;
     }
+    up.send();
     for (int b = 0; b < nblk; ++b) dc[b] = x.take(cb);
     cov_batch_dev(c, kind, lmin, lmax, nblk, ds.data(), nR ? dr.data() : nullptr, dw.data(), LW,
                   precision, dc.data(), n);

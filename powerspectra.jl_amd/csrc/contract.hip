@@ -970,9 +970,21 @@ int nv_of(const ContractRequest& rq) {
 }  // namespace
 
 static int* run_contraction_checked(Ctx* c, const ContractRequest& rq, hipStream_t s,
-                                    void* scratch, size_t scratch_bytes, int nbands = 1,
+                                    void* scratch, size_t scratch_bytes, bool check = true,
+                                    int nbands = 1,
                                     std::vector<std::pair<int, hipEvent_t>>* band_done =
                                         nullptr);
+
+// The covariance flag at err into the context's pinned word, in stream order
+// on the context stream, and the check of it once that has been waited for.
+static void fetch_cov_flag(Ctx* c, const int* err) {
+  ensure_stage(c);
+  PSX_HIP(hipMemcpyAsync(c->flag, err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+}
+static void check_cov_flag(const Ctx* c) {
+  PSX_REQUIRE(*c->flag == 0, PSX_ERR_DOMAIN,
+              "sqrt of a negative spectrum product (Julia DomainError)");
+}
 
 struct RecLayout {
   int nv, ne, rs, ft, ft1;
@@ -998,7 +1010,7 @@ size_t contraction_scratch_bytes(const ContractRequest& rq) {
 }
 
 int* run_contraction_on(Ctx* c, const ContractRequest& rq, hipStream_t s,
-                        void* scratch, size_t scratch_bytes) {
+                        void* scratch, size_t scratch_bytes, bool check) {
   const int nv = nv_of(rq);
   PSX_REQUIRE(nv >= 1 && nv <= kMaxV, PSX_ERR_ARGUMENT, "bad number of W spectra");
   PSX_REQUIRE(rq.lmin >= 0 && rq.lmax >= rq.lmin, PSX_ERR_ARGUMENT, "bad lmin/lmax");
@@ -1007,14 +1019,15 @@ int* run_contraction_on(Ctx* c, const ContractRequest& rq, hipStream_t s,
   // l3 never exceeds l1 + l2 <= 2 lmax: longer W spectra are truncated
   ContractRequest rqe = rq;
   rqe.LW = std::min<int64_t>(rq.LW, 2 * (int64_t)rq.lmax + 1);
-  return run_contraction_checked(c, rqe, s, scratch, scratch_bytes);
+  return run_contraction_checked(c, rqe, s, scratch, scratch_bytes, check);
 }
 
 // With band_done, the tiles run as nbands launches in l1 bands and after each
-// one an event is recorded on s and listed with the band's done_l; the
-// covariance flag is then left to the caller.
+// one an event is recorded on s and listed with the band's done_l.  The
+// covariance flag is waited for and checked here on the context stream, unless
+// `check` is off or there are bands: then that is the caller's.
 static int* run_contraction_checked(Ctx* c, const ContractRequest& rq, hipStream_t s,
-                                    void* scratch, size_t scratch_bytes, int nbands,
+                                    void* scratch, size_t scratch_bytes, bool check, int nbands,
                                     std::vector<std::pair<int, hipEvent_t>>* band_done) {
   const int nv = nv_of(rq);
   const int n = rq.lmax - rq.lmin + 1;
@@ -1111,12 +1124,10 @@ static int* run_contraction_checked(Ctx* c, const ContractRequest& rq, hipStream
       PSX_HIP(hipGetLastError());
     }
   }
-  if (rq.epi == EPI_COV && s == c->stream) {
-    int h = 0;
-    PSX_HIP(hipMemcpyAsync(&h, err, sizeof(int), hipMemcpyDeviceToHost, s));
+  if (check && rq.epi == EPI_COV && s == c->stream) {
+    fetch_cov_flag(c, err);
     PSX_HIP(hipStreamSynchronize(s));
-    PSX_REQUIRE(h == 0, PSX_ERR_DOMAIN,
-                "sqrt of a negative spectrum product (Julia DomainError)");
+    check_cov_flag(c);
   }
   return rq.epi == EPI_COV ? err : nullptr;
 }
@@ -1132,8 +1143,8 @@ void run_contraction_to_host(Ctx* c, const ContractRequest& rq, double* const* h
   const int nout = rq.epi == EPI_MCM ? nv_of(rq) : 1;
   PSX_REQUIRE(rq.ldo == n, PSX_ERR_ARGUMENT, "device outputs must be packed (ld = n)");
   for (int k = 0; k < nout; ++k) PSX_REQUIRE(host[k], PSX_ERR_ARGUMENT, "null output pointer");
-  // bands only pay when the outputs outgrow one staging buffer
-  const bool banded = (size_t)nout * n * (size_t)n * sizeof(double) > kStageBytes;
+  // bands only pay when there is much to copy
+  const bool banded = (size_t)nout * n * (size_t)n * sizeof(double) > kBandBytes;
   void* scratch = ctx_scratch(c, contraction_scratch_bytes(rq));
   std::vector<std::pair<int, hipEvent_t>> done;
   int* err = nullptr;
@@ -1144,15 +1155,16 @@ void run_contraction_to_host(Ctx* c, const ContractRequest& rq, double* const* h
     PSX_REQUIRE(rq.lmax <= kLmaxCap, PSX_ERR_ARGUMENT, "lmax above 8191 is not supported");
     ContractRequest rqe = rq;
     rqe.LW = std::min<int64_t>(rq.LW, 2 * (int64_t)rq.lmax + 1);
-    err = run_contraction_checked(c, rqe, c->stream, scratch, c->scratch_bytes, kMaxBands,
-                                  &done);
+    err = run_contraction_checked(c, rqe, c->stream, scratch, c->scratch_bytes, false,
+                                  kMaxBands, &done);
   } else {
-    // one launch; it checks the covariance flag itself, and the copy follows
-    // it on the context stream
-    run_contraction_on(c, rq, c->stream, scratch, c->scratch_bytes);
+    // one launch, the covariance flag and the copy in stream order
+    err = run_contraction_on(c, rq, c->stream, scratch, c->scratch_bytes, false);
+    if (err) fetch_cov_flag(c, err);
     std::vector<D2HMatrix> whole;
     for (int k = 0; k < nout; ++k) whole.push_back({host[k], ldh, rq.dout[k], n, n, n});
     d2h_matrices(c, whole.data(), nout);
+    if (err) check_cov_flag(c);
     return;
   }
   // columns [j0, j1) of every output once the band completing them is done
@@ -1168,13 +1180,9 @@ void run_contraction_to_host(Ctx* c, const ContractRequest& rq, double* const* h
   }
   PSX_REQUIRE(j0 == n, PSX_ERR_ARGUMENT, "band bookkeeping left columns uncovered");
   d2h_matrices_overlapped(c, pieces.data(), (int)pieces.size());
+  if (err) fetch_cov_flag(c, err);
   PSX_HIP(hipStreamSynchronize(c->stream));
-  if (err) {
-    int h = 0;
-    PSX_HIP(hipMemcpy(&h, err, sizeof(int), hipMemcpyDeviceToHost));
-    PSX_REQUIRE(h == 0, PSX_ERR_DOMAIN,
-                "sqrt of a negative spectrum product (Julia DomainError)");
-  }
+  if (err) check_cov_flag(c);
 }
 
 // ---- allocation-free mode-coupling path -----------------------------------

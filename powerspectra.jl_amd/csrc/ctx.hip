@@ -316,62 +316,99 @@ int psx_memcpy_d2h(psx_ctx* h, void* dst, const void* src, size_t bytes) {
 
 // ---- staged host copies ---------------------------------------------------
 // Copies between device memory and pageable host memory run far below PCIe
-// speed; large ones go through two pinned buffers so that the DMA into (or
-// out of) one overlaps host threads copying the other.
+// speed (a 2-D one goes row by row: 660 us for a 96 x 96 block), so all go
+// through a ring of pinned slots: the DMA runs ahead in some while host threads
+// copy others, a chunk split between several threads, which also fault in a
+// fresh destination's pages.  Chunks are an eighth of the transfer, at most a
+// slot (8 MB, 147 us at 57 GB/s: 2 MB chunks lost 20 % of that rate between
+// DMAs on 400 MB) and at least kChunkBytes, so that short ones overlap too.
 namespace psx {
 
 namespace {
-constexpr size_t kDirectBytes = size_t(1) << 20;
-// A contiguous range longer than a stage buffer (one long column, or columns
-// packed on both sides: a map, a set of a_lm) is recut into columns of this
-// many doubles (512 KB), so that it goes through the staged pipeline and its
-// host copies spread over threads.
-constexpr int64_t kLineDoubles = int64_t(1) << 16;
+constexpr int kCopyThreads = 11;                    // and the calling thread
+constexpr size_t kChunkBytes = size_t(1) << 20;
+constexpr size_t kTaskBytes = size_t(768) << 10;    // of a chunk, per task
+constexpr size_t kInlineBytes = size_t(256) << 10;  // copied by the caller itself
+}  // namespace
+
+CopyPool::CopyPool(int threads) {
+  try {
+    for (int i = 0; i < threads; ++i) threads_.emplace_back([this] { work(); });
+  } catch (const std::system_error&) {
+    // (as many as the process may have; with none, submit runs the tasks)
+  }
+}
+
+CopyPool::~CopyPool() {
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    stop_ = true;
+  }
+  cv_.notify_all();
+  for (auto& t : threads_) t.join();
+}
+
+void CopyPool::submit(const std::function<void()>& task) {
+  if (threads_.empty()) return task();
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    tasks_.push_back(task);
+  }
+  cv_.notify_one();
+}
+
+void CopyPool::work() {
+  for (;;) {
+    std::function<void()> t;
+    {
+      std::unique_lock<std::mutex> lk(mu_);
+      cv_.wait(lk, [&] { return stop_ || !tasks_.empty(); });
+      if (tasks_.empty()) return;   // stopping
+      t = std::move(tasks_.front());
+      tasks_.pop_front();
+    }
+    t();
+  }
+}
+
+void Stage::grow(int n) {
+  n = std::min(n, kSlots);
+  while (have < n) {
+    Slot& sl = slot[have];
+    if (!sl.ev) PSX_HIP(hipEventCreateWithFlags(&sl.ev, hipEventDisableTiming));
+    void* p = nullptr;
+    PSX_HIP(hipHostMalloc(&p, kSlotBytes, hipHostMallocDefault));
+    sl.p = (char*)p;
+    ++have;
+  }
+}
+
+void Stage::release() {
+  for (Slot& sl : slot) {
+    if (sl.ev) (void)hipEventDestroy(sl.ev);
+    if (sl.p) (void)hipHostFree(sl.p);
+    sl.ev = nullptr;
+    sl.p = nullptr;
+  }
+  have = next = 0;
+}
 
 void ensure_stage(Ctx* c) {
-  if (c->stage[0]) return;
-  for (int i = 0; i < 2; ++i) {
-    PSX_HIP(hipHostMalloc(&c->stage[i], kStageBytes, hipHostMallocDefault));
-    PSX_HIP(hipEventCreateWithFlags(&c->stage_ev[i], hipEventDisableTiming));
+  if (c->xstream) return;
+  if (!c->pool) {
+    const int hw = (int)std::max(2u, std::thread::hardware_concurrency());
+    c->pool = std::make_unique<CopyPool>(std::min(kCopyThreads, hw - 1));
   }
+  if (!c->flag) PSX_HIP(hipHostMalloc((void**)&c->flag, kFlags * sizeof(int), hipHostMallocDefault));
   PSX_HIP(hipStreamCreateWithFlags(&c->xstream, hipStreamNonBlocking));
 }
 
-// dst(:, j) = src(:, j) for j < cols, column-major, split over host threads
-void copy_cols(double* dst, int64_t ldd, const double* src, int64_t lds, int64_t rows,
-               int64_t cols) {
-  const size_t bytes = sizeof(double) * (size_t)rows * (size_t)cols;
-  const int nt = (int)std::min<int64_t>(
-      {8, (int64_t)std::max(1u, std::thread::hardware_concurrency()), cols,
-       (int64_t)(bytes >> 22) + 1});
-  auto work = [&](int t) {
-    const int64_t j0 = cols * t / nt, j1 = cols * (t + 1) / nt;
-    if (ldd == rows && lds == rows) {
-      std::memcpy(dst + j0 * rows, src + j0 * rows, sizeof(double) * rows * (j1 - j0));
-    } else {
-      for (int64_t j = j0; j < j1; ++j)
-        std::memcpy(dst + j * ldd, src + j * lds, sizeof(double) * rows);
-    }
-  };
-  if (nt <= 1) {
-    work(0);
-    return;
-  }
-  std::vector<std::thread> th;
-  for (int t = 1; t < nt; ++t) th.emplace_back(work, t);
-  work(0);
-  for (auto& x : th) x.join();
-}
-}  // namespace
-
 void release_stage(Ctx* c) {
   if (c->xstream) (void)hipStreamSynchronize(c->xstream);
-  for (int i = 0; i < 2; ++i) {
-    if (c->stage_ev[i]) (void)hipEventDestroy(c->stage_ev[i]);
-    if (c->stage[i]) (void)hipHostFree(c->stage[i]);
-    c->stage_ev[i] = nullptr;
-    c->stage[i] = nullptr;
-  }
+  c->pool.reset();
+  c->stage.release();
+  if (c->flag) (void)hipHostFree(c->flag);
+  c->flag = nullptr;
   if (c->xstream) (void)hipStreamDestroy(c->xstream);
   c->xstream = nullptr;
   for (hipEvent_t& e : c->band_ev) {
@@ -386,84 +423,201 @@ void ensure_band_events(Ctx* c) {
 }
 
 namespace {
-// one column block of a staged copy: nc columns of `rows` doubles
+// one piece of a staged copy: nc columns of `rows` doubles, at most a slot
 struct Chunk {
   double* host;
   int64_t ldh;
-  const double* dev;
+  double* dev;
   int64_t ldd;
   int64_t rows, nc;
   hipEvent_t after;
+  size_t bytes() const { return sizeof(double) * (size_t)rows * (size_t)nc; }
 };
 
-void chunk_to_stage(hipStream_t s, void* stage, const Chunk& k) {
-  const size_t colb = sizeof(double) * (size_t)k.rows;
-  if (k.ldd == k.rows)
-    PSX_HIP(hipMemcpyAsync(stage, k.dev, colb * (size_t)k.nc, hipMemcpyDeviceToHost, s));
-  else
-    PSX_HIP(hipMemcpy2DAsync(stage, colb, k.dev, k.ldd * sizeof(double), colb, (size_t)k.nc,
-                             hipMemcpyDeviceToHost, s));
+// Cut a matrix into chunks of at most `most` doubles; packed ranges and columns
+// longer than that are cut along the rows.
+void cut(std::vector<Chunk>& ch, int64_t most, double* host, int64_t ldh, double* dev,
+         int64_t ldd, int64_t rows, int64_t cols, hipEvent_t after) {
+  if (rows <= 0 || cols <= 0) return;
+  if (cols > 1 && ldh == rows && ldd == rows) {
+    rows *= cols;
+    cols = 1;
+  }
+  if (cols == 1 || rows > most) {
+    for (int64_t j = 0; j < cols; ++j)
+      for (int64_t i = 0; i < rows; i += most) {
+        const int64_t m = std::min(most, rows - i);
+        ch.push_back({host + j * ldh + i, m, dev + j * ldd + i, m, m, 1, after});
+      }
+    return;
+  }
+  const int64_t cpc = most / rows;
+  for (int64_t j = 0; j < cols; j += cpc)
+    ch.push_back({host + j * ldh, ldh, dev + j * ldd, ldd, rows, std::min(cpc, cols - j), after});
+}
+
+// doubles a chunk holds in a transfer of `total`
+int64_t chunk_doubles(int64_t total) {
+  const int64_t lo = kChunkBytes / sizeof(double), hi = Stage::kSlotBytes / sizeof(double);
+  return std::min(hi, std::max(lo, (total / 8 + 511) & ~int64_t(511)));
+}
+
+void copy_cols(double* dst, int64_t ldd, const double* src, int64_t lds, int64_t rows,
+               int64_t cols) {
+  if (ldd == rows && lds == rows) {
+    std::memcpy(dst, src, sizeof(double) * rows * cols);
+    return;
+  }
+  for (int64_t j = 0; j < cols; ++j)
+    std::memcpy(dst + j * ldd, src + j * lds, sizeof(double) * rows);
+}
+
+// (the waiting thread takes no task itself: it has the next DMA to issue)
+void wait_copied(const Stage::Slot& sl) {
+  while (sl.copying.load(std::memory_order_acquire)) std::this_thread::yield();
+}
+
+// waits for every host copy of the stage, also when an error unwinds: they use
+// the caller's memory
+struct CopiesDone {
+  Stage& st;
+  ~CopiesDone() {
+    for (int i = 0; i < st.have; ++i) wait_copied(st.slot[i]);
+  }
+};
+
+// Copy chunk x between its host range and slot sl (to the host, or from it),
+// split between pool tasks, or by the caller when the whole transfer is small.
+void start_copy(Stage::Slot& sl, CopyPool& pool, bool inlined, const Chunk& x, bool to_host) {
+  auto part = [&sl, to_host](const Chunk& y, int64_t at) {
+    double* p = (double*)sl.p + at;
+    if (to_host) copy_cols(y.host, y.ldh, p, y.rows, y.rows, y.nc);
+    else copy_cols(p, y.rows, y.host, y.ldh, y.rows, y.nc);
+  };
+  if (inlined) {
+    part(x, 0);
+    return;
+  }
+  const bool by_rows = x.nc == 1;
+  const int64_t len = by_rows ? x.rows : x.nc;
+  const int64_t n = std::max<int64_t>(1, std::min<int64_t>(len, x.bytes() / kTaskBytes));
+  sl.copying.store((int)n, std::memory_order_relaxed);
+  for (int64_t i = 0; i < n; ++i) {
+    const int64_t a = len * i / n, b = len * (i + 1) / n;
+    Chunk y = x;
+    if (by_rows) {
+      y.host += a;
+      y.rows = y.ldh = b - a;
+    } else {
+      y.host += a * x.ldh;
+      y.nc = b - a;
+    }
+    const int64_t at = by_rows ? a : a * x.rows;
+    auto task = [&sl, part, y, at] {
+      part(y, at);
+      sl.copying.fetch_sub(1, std::memory_order_release);
+    };
+    try {
+      pool.submit(task);
+    } catch (const std::bad_alloc&) {   // (not queued: the count has to come down)
+      task();
+    }
+  }
+}
+
+bool small(const std::vector<Chunk>& ch) {
+  return ch.size() == 1 && ch[0].bytes() <= kInlineBytes;
+}
+
+void d2h_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chunk>& ch) {
+  const size_t n = ch.size();
+  if (n == 0) return;
+  st.grow((int)std::min<size_t>(n, Stage::kSlots));
+  CopiesDone done{st};
+  const int ring = st.have, base = st.next;
+  const bool inlined = small(ch);
+  auto at = [&](size_t k) -> Stage::Slot& { return st.slot[(base + k) % ring]; };
+  size_t i = 0;
+  for (size_t k = 0; k < n; ++k) {
+    // DMAs into every slot whose last host copy is over
+    for (; i < n && i < k + ring; ++i) {
+      Stage::Slot& sl = at(i);
+      if (i > k && sl.copying.load(std::memory_order_acquire)) break;
+      wait_copied(sl);
+      const Chunk& x = ch[i];
+      if (x.after) PSX_HIP(hipStreamWaitEvent(s, x.after, 0));
+      const size_t colb = sizeof(double) * (size_t)x.rows;
+      // (an upload still reading the slot, perhaps on another stream)
+      if (hipEventQuery(sl.ev) != hipSuccess) {
+        (void)hipGetLastError();
+        PSX_HIP(hipStreamWaitEvent(s, sl.ev, 0));
+      }
+      if (x.ldd == x.rows)
+        PSX_HIP(hipMemcpyAsync(sl.p, x.dev, x.bytes(), hipMemcpyDeviceToHost, s));
+      else
+        PSX_HIP(hipMemcpy2DAsync(sl.p, colb, x.dev, x.ldd * sizeof(double), colb, (size_t)x.nc,
+                                 hipMemcpyDeviceToHost, s));
+      PSX_HIP(hipEventRecord(sl.ev, s));
+    }
+    Stage::Slot& sl = at(k);
+    PSX_HIP(hipEventSynchronize(sl.ev));
+    const Chunk& x = ch[k];
+    start_copy(sl, pool, inlined, x, true);
+  }
+  st.next = (int)((base + n) % ring);
+}
+
+void h2d_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chunk>& ch) {
+  const size_t n = ch.size();
+  if (n == 0) return;
+  st.grow((int)std::min<size_t>(n, Stage::kSlots));
+  CopiesDone done{st};
+  const int ring = st.have, base = st.next;
+  const bool inlined = small(ch);
+  auto at = [&](size_t k) -> Stage::Slot& { return st.slot[(base + k) % ring]; };
+  size_t i = 0;
+  for (size_t k = 0; k < n; ++k) {
+    // host copies into every slot whose last DMA is over
+    for (; i < n && i < k + ring; ++i) {
+      Stage::Slot& sl = at(i);
+      if (i > k && hipEventQuery(sl.ev) != hipSuccess) {
+        (void)hipGetLastError();
+        break;
+      }
+      PSX_HIP(hipEventSynchronize(sl.ev));
+      const Chunk& x = ch[i];
+      start_copy(sl, pool, inlined, x, false);
+    }
+    Stage::Slot& sl = at(k);
+    wait_copied(sl);
+    const Chunk& x = ch[k];
+    const size_t colb = sizeof(double) * (size_t)x.rows;
+    if (x.ldd == x.rows)
+      PSX_HIP(hipMemcpyAsync(x.dev, sl.p, x.bytes(), hipMemcpyHostToDevice, s));
+    else
+      PSX_HIP(hipMemcpy2DAsync(x.dev, x.ldd * sizeof(double), sl.p, colb, colb, (size_t)x.nc,
+                               hipMemcpyHostToDevice, s));
+    PSX_HIP(hipEventRecord(sl.ev, s));
+  }
+  st.next = (int)((base + n) % ring);
 }
 }  // namespace
 
-void d2h_matrices_on(hipStream_t s, void* const stage[2], hipEvent_t const ev[2],
-                     const D2HMatrix* m, int nm) {
-  // Every matrix is cut into stage-sized column blocks and all blocks go
-  // through one two-buffer pipeline, so the DMA stays busy across matrix
-  // boundaries.  Small matrices, and columns longer than a stage buffer, are
-  // copied directly, ahead of the pipeline.
+void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatrix* m, int nm) {
   std::vector<Chunk> ch;
-  for (int i = 0; i < nm; ++i) {
-    const D2HMatrix& x = m[i];
-    if (x.rows <= 0 || x.cols <= 0) continue;
-    const size_t colb = sizeof(double) * (size_t)x.rows;
-    if (colb > kStageBytes && (x.cols == 1 || (x.ldh == x.rows && x.ldd == x.rows))) {
-      const int64_t total = x.rows * x.cols, full = total / kLineDoubles;
-      const int64_t rem = total % kLineDoubles;
-      const int64_t cpc = (int64_t)(kStageBytes / (sizeof(double) * kLineDoubles));
-      for (int64_t j0 = 0; j0 < full; j0 += cpc)
-        ch.push_back({x.host + j0 * kLineDoubles, kLineDoubles, x.dev + j0 * kLineDoubles,
-                      kLineDoubles, kLineDoubles, std::min(cpc, full - j0), x.after});
-      if (rem)
-        ch.push_back({x.host + full * kLineDoubles, rem, x.dev + full * kLineDoubles, rem, rem,
-                      1, x.after});
-      continue;
-    }
-    // (a piece that waits for an event is always staged: a direct copy to
-    // pageable memory would hold this thread until the event fires)
-    if ((!x.after && colb * (size_t)x.cols <= kDirectBytes) || colb > kStageBytes) {
-      if (x.after) PSX_HIP(hipStreamWaitEvent(s, x.after, 0));
-      PSX_HIP(hipMemcpy2DAsync(x.host, x.ldh * sizeof(double), x.dev, x.ldd * sizeof(double),
-                               colb, (size_t)x.cols, hipMemcpyDeviceToHost, s));
-      continue;
-    }
-    const int64_t cpc = (int64_t)(kStageBytes / colb);  // columns per block
-    for (int64_t j0 = 0; j0 < x.cols; j0 += cpc)
-      ch.push_back({x.host + j0 * x.ldh, x.ldh, x.dev + j0 * x.ldd, x.ldd, x.rows,
-                    std::min(cpc, x.cols - j0), x.after});
-  }
-  const size_t nch = ch.size();
-  auto issue = [&](size_t k) {
-    if (ch[k].after) PSX_HIP(hipStreamWaitEvent(s, ch[k].after, 0));
-    chunk_to_stage(s, stage[k & 1], ch[k]);
-    PSX_HIP(hipEventRecord(ev[k & 1], s));
-  };
-  if (nch > 0) issue(0);
-  if (nch > 1) issue(1);
-  for (size_t k = 0; k < nch; ++k) {
-    const Chunk& x = ch[k];
-    PSX_HIP(hipEventSynchronize(ev[k & 1]));
-    copy_cols(x.host, x.ldh, (const double*)stage[k & 1], x.rows, x.rows, x.nc);
-    if (k + 2 < nch) issue(k + 2);
-  }
-  PSX_HIP(hipStreamSynchronize(s));
+  int64_t total = 0;
+  for (int i = 0; i < nm; ++i)
+    total += std::max<int64_t>(m[i].rows, 0) * std::max<int64_t>(m[i].cols, 0);
+  const int64_t most = chunk_doubles(total);
+  for (int i = 0; i < nm; ++i)
+    cut(ch, most, m[i].host, m[i].ldh, const_cast<double*>(m[i].dev), m[i].ldd, m[i].rows, m[i].cols,
+        m[i].after);
+  d2h_chunks(s, stage, pool, ch);
 }
 
 void d2h_matrices(Ctx* c, const D2HMatrix* m, int nm) {
-  for (int i = 0; i < nm; ++i)
-    if ((size_t)m[i].rows * (size_t)m[i].cols * sizeof(double) > kDirectBytes || m[i].after)
-      ensure_stage(c);
-  d2h_matrices_on(c->stream, c->stage, c->stage_ev, m, nm);
+  ensure_stage(c);
+  d2h_matrices_on(c->stream, c->stage, *c->pool, m, nm);
 }
 
 void d2h_matrix(Ctx* c, double* host, int64_t ldh, const double* dev, int64_t ldd,
@@ -474,57 +628,54 @@ void d2h_matrix(Ctx* c, double* host, int64_t ldh, const double* dev, int64_t ld
 
 void d2h_matrices_overlapped(Ctx* c, const D2HMatrix* m, int nm) {
   ensure_stage(c);
-  d2h_matrices_on(c->xstream, c->stage, c->stage_ev, m, nm);
+  d2h_matrices_on(c->xstream, c->stage, *c->pool, m, nm);
 }
 
 namespace {
 void h2d_matrix_on(Ctx* c, hipStream_t s, double* dev, int64_t ldd, const double* host,
                    int64_t ldh, int64_t rows, int64_t cols) {
-  const size_t colb = sizeof(double) * (size_t)rows;
-  if (rows <= 0 || cols <= 0) return;
-  if (colb > kStageBytes && (cols == 1 || (ldd == rows && ldh == rows))) {
-    const int64_t total = rows * cols, full = total / kLineDoubles, rem = total % kLineDoubles;
-    if (full) h2d_matrix_on(c, s, dev, kLineDoubles, host, kLineDoubles, kLineDoubles, full);
-    if (rem)
-      h2d_matrix_on(c, s, dev + full * kLineDoubles, rem, host + full * kLineDoubles, rem, rem,
-                    1);
-    return;
-  }
-  if (colb * (size_t)cols <= kDirectBytes || colb > kStageBytes) {
-    PSX_HIP(hipMemcpy2DAsync(dev, ldd * sizeof(double), host, ldh * sizeof(double), colb,
-                             (size_t)cols, hipMemcpyHostToDevice, s));
-    PSX_HIP(hipStreamSynchronize(s));
-    return;
-  }
-  const int64_t cpc = (int64_t)(kStageBytes / colb);
-  const int64_t nch = (cols + cpc - 1) / cpc;
-  for (int64_t k = 0; k < nch; ++k) {
-    const int b = (int)(k & 1);
-    const int64_t j0 = k * cpc, nc = std::min(cpc, cols - j0);
-    PSX_HIP(hipEventSynchronize(c->stage_ev[b]));  // buffer b free again
-    copy_cols((double*)c->stage[b], rows, host + j0 * ldh, ldh, rows, nc);
-    if (ldd == rows)
-      PSX_HIP(hipMemcpyAsync(dev + j0 * ldd, c->stage[b], colb * (size_t)nc,
-                             hipMemcpyHostToDevice, s));
-    else
-      PSX_HIP(hipMemcpy2DAsync(dev + j0 * ldd, ldd * sizeof(double), c->stage[b], colb, colb,
-                               (size_t)nc, hipMemcpyHostToDevice, s));
-    PSX_HIP(hipEventRecord(c->stage_ev[b], s));
-  }
-  PSX_HIP(hipStreamSynchronize(s));
+  std::vector<Chunk> ch;
+  cut(ch, chunk_doubles(std::max<int64_t>(rows, 0) * std::max<int64_t>(cols, 0)),
+      const_cast<double*>(host), ldh, dev, ldd, rows, cols, nullptr);
+  h2d_chunks(s, c->stage, *c->pool, ch);
 }
 }  // namespace
 
 void h2d_matrix(Ctx* c, double* dev, int64_t ldd, const double* host, int64_t ldh,
                 int64_t rows, int64_t cols) {
-  if ((size_t)rows * (size_t)cols * sizeof(double) > kDirectBytes) ensure_stage(c);
+  ensure_stage(c);
   h2d_matrix_on(c, c->stream, dev, ldd, host, ldh, rows, cols);
 }
 
 void h2d_matrix_x(Ctx* c, double* dev, int64_t ldd, const double* host, int64_t ldh,
                   int64_t rows, int64_t cols) {
   ensure_stage(c);
+  // behind the uploads of the context stream: side by side the earlier one, for
+  // which kernels wait, would share the link (1 ms on two 100 MB maps)
+  if (const int have = c->stage.have)
+    PSX_HIP(hipStreamWaitEvent(c->xstream, c->stage.slot[(c->stage.next + have - 1) % have].ev, 0));
   h2d_matrix_on(c, c->xstream, dev, ldd, host, ldh, rows, cols);
+  PSX_HIP(hipStreamSynchronize(c->xstream));
+}
+
+void h2d_pieces(Ctx* c, void* dev, const std::vector<HostPiece>& pieces) {
+  ensure_stage(c);
+  size_t end = 0;
+  for (const HostPiece& p : pieces) end = std::max(end, p.offset + p.bytes);
+  if (end <= Stage::kSlotBytes) {
+    c->stage.grow(1);
+    Stage::Slot& sl = c->stage.slot[c->stage.next];
+    PSX_HIP(hipEventSynchronize(sl.ev));
+    for (const HostPiece& p : pieces) std::memcpy(sl.p + p.offset, p.host, p.bytes);
+    PSX_HIP(hipMemcpyAsync(dev, sl.p, end, hipMemcpyHostToDevice, c->stream));
+    PSX_HIP(hipEventRecord(sl.ev, c->stream));
+    c->stage.next = (c->stage.next + 1) % c->stage.have;
+    return;
+  }
+  for (const HostPiece& p : pieces)
+    h2d_matrix(c, (double*)((char*)dev + p.offset), (int64_t)(p.bytes / sizeof(double)),
+               (const double*)p.host, (int64_t)(p.bytes / sizeof(double)),
+               (int64_t)(p.bytes / sizeof(double)), 1);
 }
 
 }  // namespace psx

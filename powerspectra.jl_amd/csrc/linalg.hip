@@ -1188,11 +1188,11 @@ static size_t pivot_bytes(int n) {
 // SingularException for a zero pivot in a finished factorisation; waits for
 // the context stream.
 static void check_pivots(Ctx* c, int n, const int* ipiv) {
-  int hinfo = 0;
-  PSX_HIP(hipMemcpyAsync(&hinfo, ipiv + n + 32, sizeof(hinfo), hipMemcpyDeviceToHost, c->stream));
+  ensure_stage(c);
+  PSX_HIP(hipMemcpyAsync(c->flag, ipiv + n + 32, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   PSX_HIP(hipStreamSynchronize(c->stream));
-  PSX_REQUIRE(hinfo == 0, PSX_ERR_SINGULAR,
-              "LU: zero pivot at position " + std::to_string(hinfo) +
+  PSX_REQUIRE(*c->flag == 0, PSX_ERR_SINGULAR,
+              "LU: zero pivot at position " + std::to_string(*c->flag) +
                   " (Julia SingularException)");
 }
 
@@ -1269,7 +1269,9 @@ void lu_solve_concurrent(Ctx* c, const LuSystem* sys, int count) {
     throw;
   }
   // SingularException for the first system with a zero pivot
-  std::vector<int> info(count, 0);
+  static_assert(1 + kLuExtraLanes <= kFlags, "a pinned word for each system");
+  ensure_stage(c);
+  int* const info = c->flag;
   for (int i = 0; i < count; ++i)
     PSX_HIP(hipMemcpyAsync(&info[i], sys[i].ipiv + sys[i].n + 32, sizeof(int),
                            hipMemcpyDeviceToHost, c->stream));
@@ -1459,14 +1461,9 @@ int psx_lu_factor(psx_ctx* hctx, int n, const double* A, int64_t lda, double* LU
     int* dp = reinterpret_cast<int*>(x.take(pb));
     h2d_matrix(c, dA, n, A, lda, n, n);
     lu_factor_dev(c, n, dA, n, dp, dp + n + 32);
-    int hinfo = 0;
     PSX_HIP(hipMemcpyAsync(ipiv, dp, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
-    PSX_HIP(hipMemcpyAsync(&hinfo, dp + n + 32, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     d2h_matrix(c, LU, ldlu, dA, n, n, n);
-    PSX_HIP(hipStreamSynchronize(c->stream));
-    PSX_REQUIRE(hinfo == 0, PSX_ERR_SINGULAR,
-                "LU: zero pivot at position " + std::to_string(hinfo) +
-                    " (Julia SingularException)");
+    check_pivots(c, n, dp);
   });
 }
 

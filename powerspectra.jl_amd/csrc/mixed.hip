@@ -960,8 +960,7 @@ void run_mixed(Ctx* c, const MixRequest& rq) {
         hp[2 * kMaxCols + 4 * b + i] = rq.dspec[b][i];
         hp[2 * kMaxCols + 4 * kMaxBlk + 4 * b + i] = rq.dratio[b][i];
       }
-  PSX_HIP(hipMemcpyAsync(ptrs, hp.data(), sizeof(void*) * hp.size(), hipMemcpyHostToDevice,
-                         c->stream));
+  h2d_pieces(c, ptrs, {{hp.data(), sizeof(void*) * hp.size(), 0}});
 
   PrepArgs pa{};
   pa.W = (const double* const*)ptrs;
@@ -1037,10 +1036,10 @@ void run_mixed(Ctx* c, const MixRequest& rq) {
                        0, c->stream, sa);
   }
   if (rq.epi == EPI_COV) {
-    int h = 0;
-    PSX_HIP(hipMemcpyAsync(&h, err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    PSX_HIP(hipMemcpyAsync(c->flag, err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     PSX_HIP(hipStreamSynchronize(c->stream));
-    PSX_REQUIRE(h == 0, PSX_ERR_DOMAIN, "sqrt of a negative spectrum product (Julia DomainError)");
+    PSX_REQUIRE(*c->flag == 0, PSX_ERR_DOMAIN,
+                "sqrt of a negative spectrum product (Julia DomainError)");
   }
 }
 

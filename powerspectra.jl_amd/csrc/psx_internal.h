@@ -3,12 +3,17 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <condition_variable>
 #include <cstdint>
+#include <deque>
 #include <functional>
 #include <initializer_list>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/powerspectra_hip.h"
@@ -68,6 +73,41 @@ struct CachedSlot {
   bool busy = false;
 };
 
+// Host threads that copy between pinned and pageable memory, kept by the
+// context and shared by its servers.  Tasks may come from several threads.
+class CopyPool {
+ public:
+  explicit CopyPool(int threads);
+  ~CopyPool();
+  void submit(const std::function<void()>& task);
+
+ private:
+  void work();
+  std::mutex mu_;
+  std::condition_variable cv_;
+  std::deque<std::function<void()>> tasks_;
+  std::vector<std::thread> threads_;
+  bool stop_ = false;
+};
+
+// A ring of pinned slots for staged copies on one stream at a time.  Slots are
+// allocated as a copy needs them, and kept.
+struct Stage {
+  static constexpr size_t kSlotBytes = size_t(8) << 20;
+  static constexpr int kSlots = 8;
+  struct Slot {
+    char* p = nullptr;
+    hipEvent_t ev = nullptr;        // the slot's last DMA
+    std::atomic<int> copying{0};    // host threads that read or write it
+  };
+  Slot slot[kSlots];
+  int have = 0, next = 0;
+  void grow(int n);                 // at least min(n, kSlots) slots
+  void release();                   // nothing may be in flight
+};
+
+constexpr int kFlags = 16;
+
 struct Ctx {
   int device = 0;
   size_t budget = 0;
@@ -89,11 +129,13 @@ struct Ctx {
   // an allocation would otherwise exceed the budget): the device copies of a
   // host-pointer call's inputs and outputs, and the work area of a transform
   CachedSlot xfer, work;
-  // two pinned host staging buffers for large host <-> device copies, and the
-  // stream that copies device results out while later kernels still run
-  void* stage[2] = {nullptr, nullptr};
-  hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  // pinned host slots and threads for host <-> device copies, the stream that
+  // copies device results out while later kernels still run, and kFlags pinned
+  // words for what kernels report (the covariance flag, zero pivots)
+  Stage stage;
+  std::unique_ptr<CopyPool> pool;
   hipStream_t xstream = nullptr;
+  int* flag = nullptr;
   // one event per l1 band of a banded contraction
   hipEvent_t band_ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   // extra streams, rocBLAS handles and events for independent factorizations
@@ -171,13 +213,11 @@ void alm2map_pol_dev(Ctx* c, int nside, int lmax, int nmaps, const double* dteb,
 
 // Column-major matrix copies between host memory (any pageable buffer,
 // leading dimension ldh) and device memory (leading dimension ldd), in
-// stream order on the context stream; they return when the host side is
-// complete.  Large copies are staged through the context's pinned buffers.
+// stream order on the context stream, through the context's pinned slots.
+// d2h returns when the host side is complete; h2d returns when the host
+// buffer has been read (the device side is complete in stream order).
 void d2h_matrix(Ctx* c, double* host, int64_t ldh, const double* dev, int64_t ldd,
                 int64_t rows, int64_t cols);
-// size of each of the two pinned staging buffers (the context's, and each
-// server slot's)
-constexpr size_t kStageBytes = size_t(32) << 20;
 // several matrices through one pipeline (the DMA does not drain between them)
 struct D2HMatrix {
   double* host;
@@ -191,18 +231,28 @@ void d2h_matrices(Ctx* c, const D2HMatrix* m, int nm);
 // the same on the context's copy stream, so that the pieces waiting for
 // events of the context stream copy out while later work there still runs
 void d2h_matrices_overlapped(Ctx* c, const D2HMatrix* m, int nm);
-// the same on stream s through two caller-owned pinned buffers of
-// kStageBytes each and their events
-void d2h_matrices_on(hipStream_t s, void* const stage[2], hipEvent_t const ev[2],
-                     const D2HMatrix* m, int nm);
+// the same on stream s through the caller's slots
+void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatrix* m, int nm);
 void h2d_matrix(Ctx* c, double* dev, int64_t ldd, const double* host, int64_t ldh,
                 int64_t rows, int64_t cols);
-// The same copy through the staging pipeline on the context's copy stream:
-// returns when the data is on the device, without waiting for (or ordering
-// against) work on the context stream.  The caller keeps both streams off the
-// destination meanwhile.
+// The same copy through the slots on the context's copy stream, behind earlier
+// uploads: returns when the data is on the device, without waiting for (or
+// ordering against) later work on the context stream.  The caller keeps both streams off the destination
+// meanwhile.
 void h2d_matrix_x(Ctx* c, double* dev, int64_t ldd, const double* host, int64_t ldh,
                   int64_t rows, int64_t cols);
+// Host arrays into one device range, by one copy where they fit a slot: the
+// bytes of each piece at its offset from dev.  In stream order on the context
+// stream; returns when the pieces have been read.
+struct HostPiece {
+  const void* host;
+  size_t bytes, offset;
+};
+void h2d_pieces(Ctx* c, void* dev, const std::vector<HostPiece>& pieces);
+void ensure_stage(Ctx* c);
+// outputs up to this size run in one launch and are copied after it; larger
+// ones are computed in bands, each copied out while the later ones compute
+constexpr size_t kBandBytes = size_t(32) << 20;
 
 // Launch helper: records HIP events around the launch when timing is on.
 struct TimedLaunch {
@@ -279,9 +329,10 @@ void run_contraction_noalloc(Ctx* c, const ContractRequest& rq);
 // contraction_scratch_bytes(rq)).  Returns the device address of the
 // covariance domain-error flag inside the scratch (nonzero after the kernel
 // when a spectrum product under a square root was negative), or nullptr for
-// mode-coupling requests.  On the context stream the flag is checked here.
+// mode-coupling requests.  On the context stream the flag is waited for and
+// checked here, unless `check` is off.
 int* run_contraction_on(Ctx* c, const ContractRequest& rq, hipStream_t s,
-                        void* scratch, size_t scratch_bytes);
+                        void* scratch, size_t scratch_bytes, bool check = true);
 size_t contraction_scratch_bytes(const ContractRequest& rq);
 // A contraction into packed device outputs (rq.ldo = n) followed by their
 // copy to the host blocks host[k] (leading dimension ldh).  Large outputs run

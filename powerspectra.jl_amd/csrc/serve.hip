@@ -118,8 +118,8 @@ struct Job {
 
 struct Slot {
   hipStream_t stream = nullptr;
-  void* stage[2] = {nullptr, nullptr};
-  hipEvent_t ev[2] = {nullptr, nullptr};
+  Stage stage;
+  int* flag = nullptr;      // pinned: the covariance flag of the slot's request
   std::thread th;
 };
 
@@ -173,14 +173,15 @@ void execute(Server* S, Slot* sl, Job& j) {
     std::lock_guard<std::recursive_mutex> lk(S->ctx->mu);
     err = run_contraction_on(S->ctx, rq, sl->stream, j.scratch_mem, j.scratch_bytes);
   }
-  int h = 0;
-  if (err) PSX_HIP(hipMemcpyAsync(&h, err, sizeof(int), hipMemcpyDeviceToHost, sl->stream));
+  *sl->flag = 0;
+  if (err)
+    PSX_HIP(hipMemcpyAsync(sl->flag, err, sizeof(int), hipMemcpyDeviceToHost, sl->stream));
   PSX_HIP(hipStreamSynchronize(sl->stream));
-  PSX_REQUIRE(h == 0, PSX_ERR_DOMAIN, "sqrt of a negative spectrum product (Julia DomainError)");
+  PSX_REQUIRE(*sl->flag == 0, PSX_ERR_DOMAIN, "sqrt of a negative spectrum product (Julia DomainError)");
   if (j.host_out) {
     D2HMatrix m[5];
     for (int k = 0; k < j.nout; ++k) m[k] = {j.rq.out[k], j.rq.ld, outs[k], n, n, n};
-    d2h_matrices_on(sl->stream, sl->stage, sl->ev, m, j.nout);
+    d2h_matrices_on(sl->stream, sl->stage, *S->ctx->pool, m, j.nout);
   }
 }
 
@@ -385,10 +386,8 @@ void free_server(Server* S) {
   for (auto& sl : S->slots) {
     if (sl->stream) (void)hipStreamSynchronize(sl->stream);
     if (sl->stream) (void)hipStreamDestroy(sl->stream);
-    for (int i = 0; i < 2; ++i) {
-      if (sl->ev[i]) (void)hipEventDestroy(sl->ev[i]);
-      if (sl->stage[i]) (void)hipHostFree(sl->stage[i]);
-    }
+    sl->stage.release();
+    if (sl->flag) (void)hipHostFree(sl->flag);
   }
   std::lock_guard<std::recursive_mutex> lk(S->ctx->mu);
   for (auto& kv : S->resident) {
@@ -430,17 +429,17 @@ int psx_server_create(psx_ctx* hctx, int slots, size_t arena_bytes, int lmax_max
       // tables for the largest request, built now: they must not be
       // reallocated while requests run
       ensure_tables(c, (2 * lmax_max + 1) + 2 * lmax_max + 512);
+      ensure_stage(c);
       S->arena_mem = (char*)ctx_alloc(c, arena_bytes);
     }
     S->arena.init(S->arena_mem, arena_bytes);
     for (int i = 0; i < slots; ++i) {
       auto sl = std::make_unique<Slot>();
       PSX_HIP(hipStreamCreateWithFlags(&sl->stream, hipStreamNonBlocking));
-      for (int b = 0; b < 2; ++b) {
-        PSX_HIP(hipHostMalloc(&sl->stage[b], kStageBytes, hipHostMallocDefault));
-        PSX_HIP(hipEventCreateWithFlags(&sl->ev[b], hipEventDisableTiming));
-      }
-      S->slots.push_back(std::move(sl));
+      S->slots.push_back(std::move(sl));   // (freed by free_server from here on)
+      Slot& q = *S->slots.back();
+      PSX_HIP(hipHostMalloc((void**)&q.flag, sizeof(int), hipHostMallocDefault));
+      q.stage.grow(Stage::kSlots);
     }
     for (auto& sl : S->slots) sl->th = std::thread(worker, S, sl.get());
   });
