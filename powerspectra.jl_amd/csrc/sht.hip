@@ -35,6 +35,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace psx {
@@ -42,33 +43,11 @@ namespace psx {
 namespace {
 
 constexpr int kMaxPolarRing = 8192;         // pixels of the longest polar ring (nside <= 2048)
-constexpr int kLChunk = 8;                  // l values per LDS reduction round
-#ifndef PSX_SHT_PAIRS
-#define PSX_SHT_PAIRS 4
-#endif
-constexpr int kPairsPerThread = PSX_SHT_PAIRS;   // ring pairs per analysis thread
-#ifndef PSX_SYN_PAIRS
-#define PSX_SYN_PAIRS 4
-#endif
-constexpr int kSynPairs = PSX_SYN_PAIRS;     // ring pairs per synthesis thread
-// The spin-2 synthesis runs 2 ring pairs per thread at 5 waves per SIMD
-// (96 VGPRs, 28 bytes spilled outside the l loop): more waves cover its four
-// dependent recurrence chains better than more pairs per thread (4 pairs at
-// 3 waves took 1.8x as long at nside 1024, lmax 3071).
-#ifndef PSX_SYN2_PAIRS
-#define PSX_SYN2_PAIRS 2
-#endif
-#ifndef PSX_SYN2_WAVES
-#define PSX_SYN2_WAVES 5
-#endif
-constexpr int kSyn2Pairs = PSX_SYN2_PAIRS;   // ring pairs per spin-2 synthesis thread
-#ifndef PSX_AN2_PAIRS
-#define PSX_AN2_PAIRS 4
-#endif
-#ifndef PSX_AN2_WAVES
-#define PSX_AN2_WAVES 3
-#endif
-constexpr int kAn2Pairs = PSX_AN2_PAIRS;     // ring pairs per spin-2 analysis thread
+constexpr int kLChunk = 8;                  // most l values between rescalings
+// Ring pairs per spin-2 synthesis thread: 2 at 5 waves per SIMD (96 VGPRs) cover the
+// four dependent recurrence chains better than more pairs per thread (4 pairs at 3
+// waves took 1.8x as long at nside 1024, lmax 3071).
+constexpr int kSyn2Pairs = 2, kSyn2Waves = 5;
 constexpr int kSynChunk = 4;                // l values read ahead per synthesis round
 constexpr double kBig = 0x1p600;            // rescaling threshold
 constexpr double kInvBig = 0x1p-600;
@@ -525,29 +504,64 @@ __global__ void __launch_bounds__(256) fold_analysis(RingArgs R, const double2* 
   }
 }
 
-// Recurrence coefficients per (l, m), l >= m + 2, in a_lm order:
-//   lambda_l = A (z lambda_{l-1} - B lambda_{l-2}),
-//   A = sqrt((4l^2 - 1)/(l^2 - m^2)),  B = sqrt(((l-1)^2 - m^2)/(4(l-1)^2 - 1)).
-__global__ void __launch_bounds__(256) rec_coefs(int lmax, double2* __restrict__ AB) {
-  const int m = blockIdx.y;
-  const int l = m + blockIdx.x * blockDim.x + threadIdx.x;
-  if (l > lmax) return;
-  double a = 0.0, b = 0.0;
-  if (l >= m + 2) {
-    const double L = l, M = m;
-    a = sqrt((4.0 * L * L - 1.0) / ((L - M) * (L + M)));
-    b = sqrt(((L - 1.0 - M) * (L - 1.0 + M)) / (4.0 * (L - 1.0) * (L - 1.0) - 1.0));
-  } else if (l == m + 1) {
-    a = sqrt(2.0 * m + 3.0);
+// The recurrence lambda_l = A_l z lambda_{l-1} - A_l B_l lambda_{l-2},
+//   A = sqrt((4l^2 - 1)/(l^2 - m^2)),  A_l B_l = A_l / A_{l-1},
+// runs on L_l = lambda_l / s_l with s_l s_{l-1} = A_l, s_m = 1:
+//   L_l = (alpha_l z) L_{l-1} - L_{l-2},  alpha_l = s_{l-1}^2,
+// two operations a step instead of three; s_l multiplies the a_lm instead
+// (before a synthesis, after an analysis).  alpha comes from the rounded s, so
+// every step is exact to a few ulp of its own whatever the rounding of the
+// product behind s_l.  alpha and s per (l, m), in a_lm order; alpha_m is 0.
+__global__ void __launch_bounds__(64) rec_coefs(int lmax, double* __restrict__ alpha,
+                                                double* __restrict__ scl) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m > lmax) return;
+  const int64_t i0 = alm_idx(lmax, m, m) - m;
+  const double M = m;
+  double s = 1.0;
+  alpha[i0 + m] = 0.0;
+  scl[i0 + m] = s;
+  for (int l = m + 1; l <= lmax; ++l) {
+    const double L = l;
+    const double a = sqrt((4.0 * L * L - 1.0) / ((L - M) * (L + M)));
+    alpha[i0 + l] = s * s;
+    s = a / s;
+    scl[i0 + l] = s;
   }
-  AB[alm_idx(lmax, l, m)] = make_double2(a, b);
+}
+
+// A synthesis's coefficients a_lm s_lm of N sets, those of one (l, m) adjacent
+// so that one scalar load takes them all, and per row m whether any is not finite.
+template <int N>
+struct ScaleArgs {
+  const double2* in[N];
+  double2* out;
+  int* odd;
+};
+template <int N>
+__global__ void __launch_bounds__(256) scale_rows(int lmax, const double* __restrict__ scl,
+                                                  ScaleArgs<N> A) {
+  const int m = blockIdx.x;
+  const int64_t i0 = alm_idx(lmax, m, m);
+  const int n = lmax + 1 - m;
+  int bad = 0;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    const double f = scl[i0 + i];
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      const double2 a = A.in[q][i0 + i];
+      A.out[(i0 + i) * N + q] = make_double2(a.x * f, a.y * f);
+      bad |= !(fabs(a.x) < HUGE_VAL && fabs(a.y) < HUGE_VAL);
+    }
+  }
+  bad = __syncthreads_or(bad);
+  if (threadIdx.x == 0) A.odd[m] = bad;
 }
 
 struct LegArgs {
   RingArgs R;
-  const double2* AB;      // recurrence coefficients
+  const double* alpha;    // recurrence coefficients
   const double* logc;     // log of sqrt((2m+1)/(4 pi) prod (2k-1)/(2k)), per m
-  int nchunk;             // pair chunks
 };
 
 // Scaled lambda_mm for ring k: mantissa and scale s <= 0 (value = mant 2^(600 s)).
@@ -575,17 +589,40 @@ __device__ __forceinline__ double scale_weight(int s) {
   return s == 0 ? 1.0 : (s == -1 ? kInvBig : 0.0);
 }
 
-// Rescaling runs once per chunk of kLChunk steps, so the steps themselves
+// A wave's ring pairs (64 P consecutive ones) are in one of three phases, which
+// only move forward as l grows: dead (every weight is 0: the step is the
+// recurrence alone), mixed, live (every scale is 0: no weights, no rescaling).
+// Each phase has its own code, without branches per pair or step.  Above the
+// turning point m ~ l sin(theta) a pair is dead for most of its l: at nside 1024,
+// lmax 3071 16 % of all steps are, and 70 % are live.  A dead pair's terms are 0
+// times its coefficient: with coefficients that are not finite it counts as mixed
+// (kOdd: those of an analysis, whose lanes are summed apart, as well).
+enum Phase { kDead, kMixed, kLive, kOdd };
+template <Phase PH>
+using PhaseC = std::integral_constant<Phase, PH>;
+constexpr int kNoScale = -(1 << 28);   // lanes past the last pair, which hold 0
+template <int P>
+__device__ __forceinline__ Phase phase_of(const int (&sc)[P], bool keep) {
+  bool live = true, dead = !keep;
+#pragma unroll
+  for (int r = 0; r < P; ++r) {
+    live = live && (sc[r] == 0 || sc[r] == kNoScale);
+    dead = dead && sc[r] < -1;
+  }
+  return __all(dead) ? kDead : __all(live) ? kLive : kMixed;
+}
+
+// Rescaling runs once per chunk of up to kLChunk steps, so the steps themselves
 // carry no branch: from a mantissa below 2^600 the recurrence grows by less
-// than 2^48 over 8 steps (sqrt(2m+3) sqrt(m) sqrt(2m/3) ... < 2^48 for
-// m <= 8191), far from double overflow, and a value that crosses 2^600 inside
-// a chunk is still weighted exactly (or dropped when it is below 2^-600).
-__device__ __forceinline__ void rescale_pair(double& a, double& b, int& s, double& wgt) {
+// than 2^56 over 8 steps (sqrt(2m+3) sqrt(m) sqrt(2m/3) ... < 2^48 for
+// m <= 8191, and the ratio of two s_l), far from double overflow, and a value
+// that crosses 2^600 inside a chunk is still weighted exactly (or dropped when
+// it is below 2^-600).
+__device__ __forceinline__ void rescale_pair(double& a, double& b, int& s) {
   if (s < 0 && fabs(a) > kBig) {
     a *= kInvBig;
     b *= kInvBig;
     s += 1;
-    wgt = scale_weight(s);
   }
 }
 
@@ -595,144 +632,243 @@ constexpr int kMaxGroup = 4;
 
 template <int NM>
 struct MapPtrs {
-  const double2* in[NM];   // analysis: F+ of each map; synthesis: a_lm
+  const double2* in[NM];   // analysis: F+ of each map
   const double2* in2[NM];  // analysis: F- of each map
   double2* out[NM];        // analysis: partial sums; synthesis: G
 };
 
-// l values per LDS reduction round of the analysis: 2 NM values per l and
-// thread go through the round's 16 rows of 256 doubles (32 KB)
-__host__ __device__ constexpr int an_lchunk(int nm) { return nm == 1 ? 8 : nm == 2 ? 4 : 2; }
-
-// DPP move of a double inside a row of 16 lanes (both 32-bit halves).
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double x) {
-  const long long v = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(v & 0xffffffffLL), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, 0xF, 0xF, false);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+// A round's 16 sums over a wave.  The matrix cores add up lanes: with B the unit
+// column n, a 4x4x4 product adds to column n of D the sum of A's four k, so four
+// products take four values a lane to one, and products of four such results sum
+// over the rows that are left.  20 instructions leave one value a lane, where
+// summing through LDS moved 16 doubles a lane in and out, and those of one l run
+// while the next one's are formed.  Lane g + 4 b + 16 n holds block b's part of
+// value n of group g.
+struct RoundSums {
+  double unit[4];
+  __device__ __forceinline__ RoundSums() {
+#pragma unroll
+    for (int n = 0; n < 4; ++n) unit[n] = (threadIdx.x & 3) == n ? 1.0 : 0.0;
+  }
+  static __device__ __forceinline__ int lane(int g, int n, int b) { return g + 4 * b + 16 * n; }
+  // group g of the round into e
+  __device__ __forceinline__ void add(int g, const double (&v)[4], double& e) const {
+    double d = 0.0;
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      d = __builtin_amdgcn_mfma_f64_4x4x4f64(v[n], unit[n], d, 0, 0, 0);
+    e = __builtin_amdgcn_mfma_f64_4x4x4f64(d, unit[g], e, 0, 0, 0);
+  }
+  // the same, where the values of `odd` (a bit each) may not be finite and 0 times
+  // them would reach the others
+  __device__ __forceinline__ void add_apart(int g, const double (&v)[4], unsigned odd,
+                                            double& e) const {
+    double u[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) u[n] = odd >> n & 1 ? 0.0 : v[n];
+    add(g, u, e);
+    const int t = threadIdx.x & 63;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      double s = v[n];
+      for (int x = 1; x < 64; x <<= 1) s += __shfl_xor(s, x);
+      if ((odd >> n & 1) && (t & ~12) == lane(g, n, 0)) e = t & 12 ? 0.0 : s;
+    }
+  }
+};
+// Keeps the pairs' steps in order, their vector instructions at least: left to
+// itself the compiler runs each sum's dependent chain in one piece, and two waves a
+// SIMD do not cover its latency.
+__device__ __forceinline__ void sched_step() {
+  __builtin_amdgcn_sched_barrier(0x4 | 0x8 | 0x10 | 0x80);   // scalar, matrix, memory, LDS pass
 }
+// Coefficients up to this keep every sum of an analysis finite: |L_lm| < 2^14 and
+// 2^13 ring pairs.
+constexpr double kHuge = 0x1p960;
 
-// Sum over the 16 lanes of a row: quad_perm [1,0,3,2], quad_perm [2,3,0,1],
-// row_ror 4, row_ror 8.  Every lane ends with the row's sum (lanes of quads
-// 0, 2 and of quads 1, 3 may differ in the last bit: the caller takes lane 0).
-__device__ __forceinline__ double row16_sum(double s) {
-  s += dpp_f64<0xB1>(s);
-  s += dpp_f64<0x4E>(s);
-  s += dpp_f64<0x124>(s);
-  s += dpp_f64<0x128>(s);
+// The waves' sums of kSumRounds rounds gather in LDS and are added up and stored
+// together: one barrier and one run of stores per block of rounds.  The round's
+// stride leaves the readers' 16 values of four rounds on different banks.
+constexpr int kSumRounds = 8;
+template <int T>
+struct SumBuf {
+  double v[2][kSumRounds][T + 8];
+};
+// Sum of value n of group g over the workgroup's waves
+template <int T>
+__device__ __forceinline__ double sum_waves(const double (&row)[T + 8], int g, int n) {
+  double s = 0.0;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) {
+    const double* p = row + 64 * w;
+    s += (p[RoundSums::lane(g, n, 0)] + p[RoundSums::lane(g, n, 1)]) +
+         (p[RoundSums::lane(g, n, 2)] + p[RoundSums::lane(g, n, 3)]);
+  }
   return s;
 }
 
+// Barrier for LDS traffic alone: __syncthreads also waits for the stores to
+// global memory.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Analysis partial sums: part_q[chunk][idx(l, m)] = sum over the chunk's pairs
-// of lambda_lm(z_p) F+-_p(m) for each map q of the group.  Each thread carries
-// kPairsPerThread independent recurrences; per round of LC l values the 256
-// partial sums of every (l, map, re/im) are reduced through LDS (16 lanes per
-// output, each summing a stride-16 column of its row so that a wave's reads
-// are consecutive doubles, then a DPP sum over the 16 lanes), in the same
-// order whatever the group size (one map alone gives the same sums).  The
-// round holding l = m, m + 1 and the last, partial round take the checked
-// path; the rounds between carry no per-step branch.
-template <int NM>
-__global__ void __launch_bounds__(256) legendre_analysis(LegArgs A, MapPtrs<NM> M) {
-  constexpr int LC = an_lchunk(NM);
-  constexpr int NO = 2 * LC * NM;  // outputs per round
-  static_assert(NO <= 16, "one output per row of 16 lanes");
-  constexpr int P = kPairsPerThread;
-  __shared__ double red[NO][256];
+// of L_l(z_p) F+-_p(m) for each map q of the group.  Each of T threads carries
+// P independent recurrences; per round of LC l values the 16 sums of every (l,
+// map, re/im) over the pairs are formed in the same order whatever the group size
+// (one map alone gives the same sums).  Bound by latency at two waves a SIMD (the
+// coefficients of P pairs fill the registers) and by the FP64 units, half busy:
+// nside 1024, lmax 3071, 2 maps 4.15 -> 3.7 ms against sums through LDS with weights
+// on every step, nside 512, lmax 1535 645 -> 595 us; with P = 4 4.4 ms.
+template <int NM, int P, int T>
+__global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(2)))
+legendre_analysis(LegArgs A, MapPtrs<NM> M) {
+  constexpr int LC = 8 / NM;       // 16 sums per round
+  __shared__ SumBuf<T> sums;
+  __shared__ int scl[P][T];        // (only rescaling needs them: kept out of registers)
   const int m = blockIdx.y;
   const int chunk = blockIdx.x;
   const int lmax = A.R.lmax;
   const int tid = threadIdx.x;
-  const double2* ABm = A.AB + alm_idx(lmax, m, m);   // ABm[l - m]
-  double z[P], l1[P], l2[P], wgt[P];
-  int sc[P];
+  const double* const al = A.alpha + alm_idx(lmax, m, m) - m;   // al[l]
+  double z[P], l1[P], l2[P];
   double2 fp[NM][P], fm[NM][P];
+  unsigned odd = 0;                // values of a group whose map is not finite
+  Phase ph;
+  {
+    int sc[P];
+    bool fin[NM];
 #pragma unroll
-  for (int r = 0; r < P; ++r) {
-    const int p = (chunk * P + r) * 256 + tid;
-    const bool live = p < A.R.npairs;
-    const int pp = live ? p : 0;
-    z[r] = A.R.z[pp];
-    lambda_start(A, pp, m, l1[r], sc[r]);
-    wgt[r] = scale_weight(sc[r]);
-    l2[r] = 0.0;
-    const int64_t o = (int64_t)m * A.R.npairs + pp;
+    for (int q = 0; q < NM; ++q) fin[q] = true;
 #pragma unroll
-    for (int q = 0; q < NM; ++q) {
-      fp[q][r] = live ? M.in[q][o] : make_double2(0.0, 0.0);
-      fm[q][r] = live ? M.in2[q][o] : make_double2(0.0, 0.0);
-    }
-  }
-  const int o = tid >> 4, g = tid & 15;
-  const int oj = o / (2 * NM), oq = (o >> 1) % NM, oc = o & 1;
-  const int64_t nalm = alm_idx(lmax, lmax + 1, lmax + 1);
-  double2* outq = M.out[0];
-#pragma unroll
-  for (int q = 1; q < NM; ++q)
-    if (oq == q) outq = M.out[q];
-  outq += (int64_t)chunk * nalm;
-  auto round = [&](const int l0, const bool edge) {
-#pragma unroll
-    for (int j = 0; j < LC; ++j) {
-      const int l = l0 + j;
-      double accr[NM], acci[NM];
-#pragma unroll
-      for (int q = 0; q < NM; ++q) accr[q] = acci[q] = 0.0;
-      if (!edge || l <= lmax) {
-        const double2 ab = sload(ABm + (l - m));   // (0, 0) at l = m
-        const bool odd = j & 1;                    // l0 - m is a multiple of LC
-#pragma unroll
-        for (int r = 0; r < P; ++r) {
-          double lam;
-          if (edge && l == m) {
-            lam = l1[r];
-          } else {
-            lam = (edge && l == m + 1) ? ab.x * z[r] * l1[r]
-                                       : ab.x * fma(z[r], l1[r], -ab.y * l2[r]);
-            l2[r] = l1[r];
-            l1[r] = lam;
-          }
-          const double lt = lam * wgt[r];
-#pragma unroll
-          for (int q = 0; q < NM; ++q) {
-            const double2 f = odd ? fm[q][r] : fp[q][r];
-            accr[q] = fma(lt, f.x, accr[q]);
-            acci[q] = fma(lt, f.y, acci[q]);
-          }
-        }
+    for (int r = 0; r < P; ++r) {
+      const int p = (chunk * (T / 64) + (tid >> 6)) * (64 * P) + 64 * r + (tid & 63);
+      const bool in = p < A.R.npairs;
+      const int pp = in ? p : 0;
+      z[r] = A.R.z[pp];
+      double start;
+      lambda_start(A, pp, m, start, sc[r]);
+      if (!in) {
+        start = 0.0;
+        sc[r] = kNoScale;
       }
+      scl[r][tid] = sc[r];
+      l1[r] = 0.0;                 // so that the first step gives the start value
+      l2[r] = -start;
+      const int64_t o = (int64_t)m * A.R.npairs + pp;
 #pragma unroll
       for (int q = 0; q < NM; ++q) {
-        red[(j * NM + q) * 2][tid] = accr[q];
-        red[(j * NM + q) * 2 + 1][tid] = acci[q];
+        fp[q][r] = in ? M.in[q][o] : make_double2(0.0, 0.0);
+        fm[q][r] = in ? M.in2[q][o] : make_double2(0.0, 0.0);
+        fin[q] = fin[q] && fabs(fp[q][r].x) < kHuge && fabs(fp[q][r].y) < kHuge &&
+                 fabs(fm[q][r].x) < kHuge && fabs(fm[q][r].y) < kHuge;
       }
     }
 #pragma unroll
-    for (int r = 0; r < P; ++r) rescale_pair(l1[r], l2[r], sc[r], wgt[r]);
-    __syncthreads();
-    if (o < NO) {                  // whole rows of 16 lanes
-      double h[4];
+    for (int q = 0; q < NM; ++q)
+      if (!__all(fin[q])) odd |= (NM == 1 ? 0xFu : 3u << (2 * q));
+    ph = odd ? kOdd : phase_of(sc, false);
+  }
+  const RoundSums rs;
+  const int64_t nalm = alm_idx(lmax, lmax + 1, lmax + 1);
+  const int64_t o0 = (int64_t)chunk * nalm + alm_idx(lmax, m, m) - m;
+  double an[LC];                   // the next round's, loaded a round ahead
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const double* row = &red[o][64 * k + g];
-        h[k] = (row[0] + row[16]) + (row[32] + row[48]);
-      }
-      const double s = row16_sum((h[0] + h[1]) + (h[2] + h[3]));
-      const int l = l0 + oj;
-      if (g == 0 && l <= lmax) ((double*)(outq + alm_idx(lmax, l, m)))[oc] = s;
+  for (int j = 0; j < LC; ++j) an[j] = sload(al + m + j);
+  // (steps past lmax read on in the tables and are not stored)
+  auto round = [&](const int l0, auto phase) -> double {
+    constexpr Phase PH = decltype(phase)::value;
+    constexpr bool weighted = PH == kMixed || PH == kOdd;
+    double a[LC];
+#pragma unroll
+    for (int j = 0; j < LC; ++j) {
+      a[j] = an[j];
+      an[j] = sload(al + l0 + LC + j);
     }
-    __syncthreads();
+    double w[P], acc[4], e = 0.0;  // (acc: one group, 2/NM values of l)
+    if constexpr (weighted)
+#pragma unroll
+      for (int r = 0; r < P; ++r) w[r] = scale_weight(scl[r][tid]);
+#pragma unroll
+    for (int j = 0; j < LC; ++j) {
+      double* c = acc + (NM == 1 ? 2 * (j & 1) : 0);
+#pragma unroll
+      for (int r = 0; r < P; ++r) {
+        const double lam = fma(a[j] * z[r], l1[r], -l2[r]);
+        l2[r] = l1[r];
+        l1[r] = lam;
+        if constexpr (PH == kDead) continue;
+        const double lt = weighted ? lam * w[r] : lam;
+#pragma unroll
+        for (int q = 0; q < NM; ++q) {
+          const double2 f = j & 1 ? fm[q][r] : fp[q][r];   // l0 - m is a multiple of LC
+          c[2 * q] = r == 0 ? lt * f.x : fma(lt, f.x, c[2 * q]);
+          c[2 * q + 1] = r == 0 ? lt * f.y : fma(lt, f.y, c[2 * q + 1]);
+        }
+        sched_step();
+      }
+      if (NM == 1 && !(j & 1)) continue;
+      const int g = NM == 1 ? j >> 1 : j;
+      if constexpr (PH == kOdd) rs.add_apart(g, acc, odd, e);
+      else if constexpr (PH != kDead) rs.add(g, acc, e);
+    }
+    if constexpr (PH != kLive) {
+      double mx = 0.0;
+#pragma unroll
+      for (int r = 0; r < P; ++r) mx = fmax(mx, fabs(l1[r]));
+      if (__any(mx > kBig)) {
+        int sc[P];
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+          sc[r] = scl[r][tid];
+          rescale_pair(l1[r], l2[r], sc[r]);
+          scl[r][tid] = sc[r];
+        }
+        if constexpr (PH != kOdd) ph = phase_of(sc, false);
+      }
+    }
+    return e;
   };
-  int l0 = m;
-  round(l0, true);
-  for (l0 += LC; l0 + LC - 1 <= lmax; l0 += LC) round(l0, false);
-  if (l0 <= lmax) round(l0, true);
+  // one loop per phase; the waves of a workgroup meet at the barriers of blocks,
+  // whichever loop each is in
+  const int rounds = (lmax - m) / LC + 1;
+  int i = 0;
+  auto store = [&](double e) {
+    const int buf = i / kSumRounds & 1, lb = m + (i & -kSumRounds) * LC;
+    sums.v[buf][i % kSumRounds][tid] = e;
+    ++i;
+    if (i % kSumRounds != 0 && i != rounds) return;
+    lds_barrier();                 // (the other buffer's readers are past it too)
+#pragma unroll
+    for (int o = tid; o < 16 * kSumRounds; o += T) {
+      const int n = o & 3, g = o >> 2 & 3;
+      const int q = NM == 1 ? 0 : n >> 1, l = lb + (o >> 4) * LC + (NM == 1 ? 2 * g + (n >> 1) : g);
+      if (l <= lmax) {
+        double2* outq = M.out[0];
+#pragma unroll
+        for (int x = 1; x < NM; ++x)
+          if (q == x) outq = M.out[x];
+        ((double*)(outq + o0 + l))[n & 1] = sum_waves<T>(sums.v[buf][o >> 4], g, n);
+      }
+    }
+  };
+  while (ph == kOdd && i < rounds) store(round(m + i * LC, PhaseC<kOdd>{}));
+  while (ph == kDead && i < rounds) store(round(m + i * LC, PhaseC<kDead>{}));
+  while (ph != kLive && i < rounds) store(round(m + i * LC, PhaseC<kMixed>{}));
+  while (i < rounds) store(round(m + i * LC, PhaseC<kLive>{}));
 }
 
-// alm (+)= w sum_chunk part[chunk]
+// Ring pairs per analysis workgroup: 8 pairs a thread (4 below 512 pairs) and
+// as few waves as cover them all, up to 4.
+inline int an_pairs(int npairs) {
+  return npairs > 1024 ? 2048 : npairs > 512 ? 1024 : npairs > 256 ? 512 : 256;
+}
+
+// alm (+)= w scl sum_chunk part[chunk]
 __global__ void __launch_bounds__(256) sum_partials(const double2* __restrict__ part,
                                                     int nchunk, int64_t nalm, double w,
+                                                    const double* __restrict__ scl,
                                                     int accumulate, double2* __restrict__ alm) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nalm) return;
@@ -743,6 +879,7 @@ __global__ void __launch_bounds__(256) sum_partials(const double2* __restrict__ 
     si += v.y;
   }
   double2 a = accumulate ? alm[i] : make_double2(0.0, 0.0);
+  w *= scl[i];
   a.x = fma(w, sr, a.x);
   a.y = fma(w, si, a.y);
   alm[i] = a;
@@ -762,77 +899,77 @@ inline int64_t g_elems(int lmax, int nr) {
   return (int64_t)((nr + kGRings - 1) / kGRings) * kGRings * (lmax + 1);
 }
 
-// ring pairs per synthesis thread: fewer for larger groups (per pair and
-// map, four accumulators)
-#ifndef PSX_SYN_PAIRS4
-#define PSX_SYN_PAIRS4 2
-#endif
-#ifndef PSX_SYN_WAVES
-#define PSX_SYN_WAVES 1
-#endif
-__host__ __device__ constexpr int syn_pairs(int nm) { return nm <= 2 ? kSynPairs : PSX_SYN_PAIRS4; }
+// ring pairs per synthesis thread: fewer for larger groups (per pair and map, four
+// accumulators; 4 maps of 2048 pairs, lmax 3071: 4.1 ms with 2, 4.7 with 4)
+__host__ __device__ constexpr int syn_pairs(int nm) { return nm <= 2 ? 4 : 2; }
 
 // Synthesis: G_q[m][k] = sum_l a_q,lm lambda_lm(z_k) for SP ring pairs per
 // thread and each map q of the group (north: even + odd l+m parts, south:
-// even - odd); a_lm and the recurrence coefficients are uniform across the
+// even - odd); a_lm s_lm and the recurrence coefficients are uniform across the
 // workgroup and read with scalar loads, kSynChunk at a time ahead of the
-// steps that use them (a rescale check per such round: growth over 4 steps
-// stays below 2^26).
+// steps that use them.  Bound by the FP64 units (70 % busy at a clock that falls to
+// 2.06 GHz under them): nside 1024, lmax 3071, 4 maps 5.8 -> 4.1 ms against the
+// unnormalised recurrence with weights on every step; a second set of scalars,
+// loaded a round ahead, gave 4.3 ms.
 template <int NM>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PSX_SYN_WAVES)))
-legendre_synthesis(LegArgs A, MapPtrs<NM> M) {
+__global__ void __launch_bounds__(256)
+legendre_synthesis(LegArgs A, const double2* __restrict__ coef, const int* __restrict__ odd,
+                   MapPtrs<NM> M) {
   constexpr int SP = syn_pairs(NM);
   const int m = blockIdx.y;
   const int lmax = A.R.lmax;
-  const int64_t i0 = alm_idx(lmax, m, m);
-  const double2* ABm = A.AB + i0;
-  double z[SP], l1[SP], l2[SP], wgt[SP];
+  const int64_t i0 = alm_idx(lmax, m, m) - m;
+  const double* const al = A.alpha + i0;                 // al[l]
+  double z[SP], l1[SP], l2[SP];
   double er[NM][SP], ei[NM][SP], orr[NM][SP], oi[NM][SP];
-  int sc[SP], pr[SP];
+  int sc[SP];
+  const double2* const cm = coef + i0 * NM;              // cm[l NM + q]
+  const bool keep = odd[m] != 0;
+  const int p0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * SP) + (threadIdx.x & 63);
 #pragma unroll
   for (int r = 0; r < SP; ++r) {
-    const int p = (blockIdx.x * SP + r) * blockDim.x + threadIdx.x;
-    pr[r] = p;
-    const int pp = p < A.R.npairs ? p : 0;
+    const bool in = p0 + 64 * r < A.R.npairs;
+    const int pp = in ? p0 + 64 * r : 0;
     z[r] = A.R.z[pp];
-    lambda_start(A, pp, m, l1[r], sc[r]);
-    wgt[r] = scale_weight(sc[r]);
-    l2[r] = 0.0;
+    double start;
+    lambda_start(A, pp, m, start, sc[r]);
+    if (!in) {
+      start = 0.0;
+      sc[r] = kNoScale;
+    }
+    l1[r] = 0.0;                   // so that the first step gives the start value
+    l2[r] = -start;
 #pragma unroll
     for (int q = 0; q < NM; ++q) er[q][r] = ei[q][r] = orr[q][r] = oi[q][r] = 0.0;
   }
-  // the first round holds l = m, m + 1, the last may pass lmax: both take
-  // the checked path, the rounds between load and step unconditionally
-  auto round = [&](const int l0, const bool edge) {
-    double2 a[NM][kSynChunk], ab[kSynChunk];
+  Phase ph = phase_of(sc, keep);
+  auto round = [&](const int l0, const bool edge, auto phase) {
+    constexpr Phase PH = decltype(phase)::value;
+    double2 a[NM][kSynChunk];
+    double ab[kSynChunk];
 #pragma unroll
     for (int j = 0; j < kSynChunk; ++j) {
       const bool in = !edge || l0 + j <= lmax;
 #pragma unroll
       for (int q = 0; q < NM; ++q)
-        a[q][j] = in ? sload(M.in[q] + i0 + (l0 + j - m)) : make_double2(0.0, 0.0);
-      ab[j] = in ? sload(ABm + (l0 + j - m)) : make_double2(0.0, 0.0);
+        if constexpr (PH != kDead)
+          a[q][j] = in ? sload(cm + (int64_t)(l0 + j) * NM + q) : make_double2(0.0, 0.0);
+      ab[j] = in ? sload(al + l0 + j) : 0.0;
     }
 #pragma unroll
-    for (int j = 0; j < kSynChunk; ++j) {
-      const int l = l0 + j;
-      if (edge && l > lmax) break;
-      const bool odd = j & 1;                      // l0 - m is a multiple of kSynChunk
+    for (int r = 0; r < SP; ++r) {
+      double w = 1.0;
+      if constexpr (PH == kMixed) w = scale_weight(sc[r]);
 #pragma unroll
-      for (int r = 0; r < SP; ++r) {
-        double lam;
-        if (edge && l == m) {
-          lam = l1[r];
-        } else {
-          lam = (edge && l == m + 1) ? ab[j].x * z[r] * l1[r]
-                                     : ab[j].x * fma(z[r], l1[r], -ab[j].y * l2[r]);
-          l2[r] = l1[r];
-          l1[r] = lam;
-        }
-        const double lt = lam * wgt[r];
+      for (int j = 0; j < kSynChunk; ++j) {
+        const double lam = fma(ab[j] * z[r], l1[r], -l2[r]);
+        l2[r] = l1[r];
+        l1[r] = lam;
+        if constexpr (PH == kDead) continue;
+        const double lt = PH == kMixed ? lam * w : lam;
 #pragma unroll
         for (int q = 0; q < NM; ++q) {
-          if (odd) {
+          if (j & 1) {                                   // l0 - m is a multiple of kSynChunk
             orr[q][r] = fma(lt, a[q][j].x, orr[q][r]);
             oi[q][r] = fma(lt, a[q][j].y, oi[q][r]);
           } else {
@@ -842,16 +979,29 @@ legendre_synthesis(LegArgs A, MapPtrs<NM> M) {
         }
       }
     }
+    if constexpr (PH != kLive) {
+      double mx = 0.0;
 #pragma unroll
-    for (int r = 0; r < SP; ++r) rescale_pair(l1[r], l2[r], sc[r], wgt[r]);
+      for (int r = 0; r < SP; ++r) mx = fmax(mx, fabs(l1[r]));
+      if (__any(mx > kBig)) {
+#pragma unroll
+        for (int r = 0; r < SP; ++r) rescale_pair(l1[r], l2[r], sc[r]);
+        ph = phase_of(sc, keep);
+      }
+    }
   };
   int l0 = m;
-  round(l0, true);
-  for (l0 += kSynChunk; l0 + kSynChunk - 1 <= lmax; l0 += kSynChunk) round(l0, false);
-  if (l0 <= lmax) round(l0, true);
+  const int le = lmax - (kSynChunk - 1);                 // the last whole round's l0
+  for (; ph == kDead && l0 <= le; l0 += kSynChunk)
+    round(l0, false, PhaseC<kDead>{});
+  for (; ph != kLive && l0 <= le; l0 += kSynChunk)
+    round(l0, false, PhaseC<kMixed>{});
+  for (; l0 <= le; l0 += kSynChunk) round(l0, false, PhaseC<kLive>{});
+  // (the weights are those of any phase; zeros past lmax)
+  if (l0 <= lmax) round(l0, true, PhaseC<kMixed>{});
 #pragma unroll
   for (int r = 0; r < SP; ++r) {
-    const int p = pr[r];
+    const int p = p0 + 64 * r;
     if (p >= A.R.npairs) continue;
     const int kn = p, ks = A.R.nr - 1 - p;
 #pragma unroll
@@ -999,37 +1149,44 @@ constexpr int kLChunk2 = 4;                 // l values per LDS round, spin 2
 struct PolArgs {
   RingArgs R;
   const double* omz;      // 1 - z per ring, exact near the north pole
-  const double* abc;      // recurrence coefficients, 3 per (l, m)
+  const double2* ab;      // recurrence coefficients alpha, beta per (l, m)
   const double* logc2;    // log(N_m K_m) - (m - 2) ln 2 per m (m >= 2)
   int nchunk;
 };
 
-// Per (l, m), in a_lm order, the coefficients producing degree l from l - 1
-// and l - 2 (L = l - 1; zero for l <= max(m, 2)):
+// The recurrences producing degree l from l - 1 and l - 2 (L = l - 1),
 //   X_l = (a z + b) X_{l-1} - c X_{l-2},   Y_l = (a z - b) Y_{l-1} - c Y_{l-2},
-//   a = sqrt((2L+3)(2L+1)) (L+1) / q,  b = 2 m a / (L (L+1)),
-//   c = sqrt((2L+3)/(2L-1)) (L+1) sqrt((L^2-m^2)(L^2-4)) / (L q),
+//   a = sqrt((2L+3)(2L+1)) (L+1) / q,  b = 2 m a / (L (L+1)),  c = a_l / a_{l-1},
 //   q = sqrt(((L+1)^2-m^2)((L+1)^2-4))
-// (the Wigner-d recurrence in l with m' = -+2, times N_l).  The integer
-// products stay below 2^53 for l <= 8191.
-__global__ void __launch_bounds__(256) rec_coefs_s2(int lmax, double* __restrict__ abc) {
-  const int m = blockIdx.y;
-  const int l = m + blockIdx.x * blockDim.x + threadIdx.x;
-  if (l > lmax) return;
+// (the Wigner-d recurrence in l with m' = -+2, times N_l), run on X_l / t_l and
+// Y_l / t_l with t_l t_{l-1} = a_l, t = 1 at l = max(m, 2):
+//   X_l = (alpha z + beta) X_{l-1} - X_{l-2},  alpha = t_{l-1}^2, beta = alpha b/a
+// (t is applied to a_E, a_B as s is to a_lm).  alpha, beta and t per (l, m), in
+// a_lm order, 0 below l = max(m, 2), where t is 1 and alpha, beta still 0.  The
+// integer products stay below 2^53 for l <= 8191.
+__global__ void __launch_bounds__(64) rec_coefs_s2(int lmax, double2* __restrict__ ab,
+                                                   double* __restrict__ scl) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m > lmax) return;
+  const int64_t i0 = alm_idx(lmax, m, m) - m;
   const int ls = m > 2 ? m : 2;
-  double a = 0.0, b = 0.0, c = 0.0;
-  if (l > ls) {
-    const double L = l - 1, L1 = l, M = m;
-    const double q = sqrt((L1 - M) * (L1 + M) * (L1 - 2.0) * (L1 + 2.0));
-    a = sqrt((2.0 * L + 3.0) * (2.0 * L + 1.0)) * L1 / q;
-    b = a * 2.0 * M / (L * L1);
-    c = sqrt((2.0 * L + 3.0) / (2.0 * L - 1.0)) * L1 *
-        sqrt((L - M) * (L + M) * (L - 2.0) * (L + 2.0)) / (L * q);
+  const double M = m;
+  double t = 1.0;
+  for (int l = m; l <= lmax; ++l) {
+    double al = 0.0, be = 0.0, sl = 0.0;
+    if (l == ls) sl = 1.0;
+    if (l > ls) {
+      const double L = l - 1, L1 = l;
+      const double q = sqrt((L1 - M) * (L1 + M) * (L1 - 2.0) * (L1 + 2.0));
+      const double a = sqrt((2.0 * L + 3.0) * (2.0 * L + 1.0)) * L1 / q;
+      al = t * t;
+      be = al * 2.0 * M / (L * L1);
+      t = a / t;
+      sl = t;
+    }
+    ab[i0 + l] = make_double2(al, be);
+    scl[i0 + l] = sl;
   }
-  double* o = abc + 3 * alm_idx(lmax, l, m);
-  o[0] = a;
-  o[1] = b;
-  o[2] = c;
 }
 
 // X and Y at l = max(m, 2) on north ring k, as mantissas of a common scale
@@ -1062,245 +1219,304 @@ __device__ inline void pol_start(const PolArgs& A, int k, int m, double& x, doub
   }
 }
 
-// One step of the X/Y recurrences of a ring pair (the start value at l = ls);
-// returns 2 lambda+ and 2 lambda- weighted by the pair's scale (see
-// rescale_pair: rescaling runs once per chunk of steps).
-__device__ __forceinline__ void pol_adv(bool start, double a, double b, double c, double z,
-                                        double& x1, double& x2, double& y1, double& y2,
-                                        double wgt, double& tp, double& tm) {
-  double x, y;
-  if (start) {
-    x = x1;
-    y = y1;
-  } else {
-    const double az = a * z;
-    x = fma(az + b, x1, -c * x2);
-    y = fma(az - b, y1, -c * y2);
-    x2 = x1;
-    x1 = x;
-    y2 = y1;
-    y1 = y;
-  }
-  tp = (x + y) * wgt;
-  tm = (x - y) * wgt;
+// One step of the X/Y recurrences of a ring pair.  Before the first, at
+// l = max(m, 2), (1) holds 0 and (2) the negated start values, with alpha = beta
+// = 0.
+__device__ __forceinline__ void pol_adv(double2 ab, double z, double& x1, double& x2, double& y1,
+                                        double& y2) {
+  const double az = ab.x * z;
+  const double x = fma(az + ab.y, x1, -x2);
+  const double y = fma(az - ab.y, y1, -y2);
+  x2 = x1;
+  x1 = x;
+  y2 = y1;
+  y1 = y;
 }
 
+// As rescale_pair, X and Y on one scale.
 __device__ __forceinline__ void pol_rescale(double& x1, double& x2, double& y1, double& y2,
-                                            int& s, double& wgt) {
+                                            int& s) {
   if (s < 0 && fmax(fabs(x1), fabs(y1)) > kBig) {
     x1 *= kInvBig;
     x2 *= kInvBig;
     y1 *= kInvBig;
     y2 *= kInvBig;
     s += 1;
-    wgt = scale_weight(s);
   }
 }
 
 // Spin-2 analysis partial sums: part[comp][chunk][idx(l, m)], comp 0 = E, 1 = B,
 // of sum over the chunk's pairs of [2 lambda+ Q + 2i lambda- U] (E) and
 // [2 lambda+ U - 2i lambda- Q] (B); F holds Q+, Q-, U+, U- at stride fs.
-// The spin-2 analysis asks for PSX_AN2_WAVES waves per SIMD with
-// kAn2Pairs ring pairs per thread (152 VGPRs at 4 pairs and 3 waves, no
-// spills).
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PSX_AN2_WAVES)))
-legendre_analysis_s2(PolArgs A, const double2* __restrict__ F,
-                                                            int64_t fs, double2* __restrict__ part) {
-  __shared__ double red[kLChunk2][4][256];
+// lambda+ pairs with the (-1)^{l+m} fold, lambda- with the other, so in X and Y
+// with the four combinations of a ring pair
+//   c1, c2 = Q+ +- i U-,   c3, c4 = U+ -+ i Q-:
+//   l + m even:  E += X c1 + Y c2,          B += X c3 + Y c4,
+//   l + m odd:   E += i (X c3 - Y c4),      B -= i (X c1 - Y c2),
+// eight operations and no sums X +- Y.  Sums over the pairs as in legendre_analysis.
+template <int P>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P > 2 ? 2 : 4)))
+legendre_analysis_s2(PolArgs A, const double2* __restrict__ F, int64_t fs,
+                     double2* __restrict__ part) {
+  constexpr int T = 256;
+  static_assert(kLChunk2 == 4, "16 sums per round");
+  __shared__ SumBuf<T> sums;
   const int m = blockIdx.y;
   const int chunk = blockIdx.x;
   const int lmax = A.R.lmax;
   const int tid = threadIdx.x;
   const int ls = m > 2 ? m : 2;
-  const double* Cm = A.abc + 3 * alm_idx(lmax, m, m);   // Cm[3 (l - m) + 0..2]
+  const int64_t i0 = alm_idx(lmax, m, m) - m;
+  const double2* const al = A.ab + i0;               // al[l]
   const int64_t nalm = alm_idx(lmax, lmax + 1, lmax + 1);
-  double z[kAn2Pairs], x1[kAn2Pairs], x2[kAn2Pairs];
-  double y1[kAn2Pairs], y2[kAn2Pairs], wgt[kAn2Pairs];
-  int sc[kAn2Pairs];
-  double2 qp[kAn2Pairs], qm[kAn2Pairs], up[kAn2Pairs], um[kAn2Pairs];
+  double z[P], x1[P], x2[P], y1[P], y2[P];
+  int sc[P];
+  double2 c1[P], c2[P], c3[P], c4[P];
+  bool fin = true;
 #pragma unroll
-  for (int r = 0; r < kAn2Pairs; ++r) {
-    const int p = (chunk * kAn2Pairs + r) * 256 + tid;
-    const bool live = p < A.R.npairs;
-    const int pp = live ? p : 0;
+  for (int r = 0; r < P; ++r) {
+    const int p = (chunk * (T / 64) + (tid >> 6)) * (64 * P) + 64 * r + (tid & 63);
+    const bool in = p < A.R.npairs;
+    const int pp = in ? p : 0;
     z[r] = A.R.z[pp];
-    pol_start(A, pp, m, x1[r], y1[r], sc[r]);
-    wgt[r] = scale_weight(sc[r]);
-    x2[r] = y2[r] = 0.0;
-    const int64_t o = (int64_t)m * A.R.npairs + pp;   // in bounds for every lane
-    const double keep = live ? 1.0 : 0.0;
-    qp[r] = F[o];
-    qm[r] = F[fs + o];
-    up[r] = F[2 * fs + o];
-    um[r] = F[3 * fs + o];
-    qp[r].x *= keep;
-    qp[r].y *= keep;
-    qm[r].x *= keep;
-    qm[r].y *= keep;
-    up[r].x *= keep;
-    up[r].y *= keep;
-    um[r].x *= keep;
-    um[r].y *= keep;
+    double xs, ys;
+    pol_start(A, pp, m, xs, ys, sc[r]);
+    double2 qp = make_double2(0.0, 0.0), qm = qp, up = qp, um = qp;
+    if (in) {
+      const int64_t o = (int64_t)m * A.R.npairs + p;
+      qp = F[o];
+      qm = F[fs + o];
+      up = F[2 * fs + o];
+      um = F[3 * fs + o];
+    } else {
+      xs = ys = 0.0;
+      sc[r] = kNoScale;
+    }
+    x1[r] = y1[r] = 0.0;
+    x2[r] = -xs;
+    y2[r] = -ys;
+    c1[r] = make_double2(qp.x - um.y, qp.y + um.x);
+    c2[r] = make_double2(qp.x + um.y, qp.y - um.x);
+    c3[r] = make_double2(up.x + qm.y, up.y - qm.x);
+    c4[r] = make_double2(up.x - qm.y, up.y + qm.x);
+    fin = fin && fabs(c1[r].x) < kHuge && fabs(c1[r].y) < kHuge && fabs(c2[r].x) < kHuge &&
+          fabs(c2[r].y) < kHuge && fabs(c3[r].x) < kHuge && fabs(c3[r].y) < kHuge &&
+          fabs(c4[r].x) < kHuge && fabs(c4[r].y) < kHuge;
   }
-  const int o = tid >> 4, g = tid & 15;
-  const int oj = o >> 2, oc = o & 3;
-  double* const outp = (double*)(part + ((int64_t)(oc >> 1) * A.nchunk + chunk) * nalm);
-  // the first round holds l = ls, the last may pass lmax: both take the
-  // checked path, the rounds between carry no per-step branch
-  auto round = [&](const int l0, const bool edge) {
+  Phase ph = __all(fin) ? phase_of(sc, false) : kOdd;
+  const RoundSums rs;
+  double2 an[kLChunk2];                              // the next round's
+#pragma unroll
+  for (int j = 0; j < kLChunk2; ++j) an[j] = sload(al + m + j);
+  // the first round holds l = ls and may hold less; steps past lmax read on in
+  // the tables and are not stored
+  auto round = [&](const int l0, auto first, auto phase) -> double {
+    constexpr Phase PH = decltype(phase)::value;
+    constexpr bool edge = decltype(first)::value;
+    constexpr bool weighted = PH == kMixed || PH == kOdd;
+    double2 a[kLChunk2];
 #pragma unroll
     for (int j = 0; j < kLChunk2; ++j) {
-      const int l = l0 + j;
-      double er = 0.0, ei = 0.0, br = 0.0, bi = 0.0;
-      if (!edge || (l <= lmax && l >= ls)) {
-        double a = 0.0, b = 0.0, c = 0.0;
-        if (!edge || l > ls) {
-          const double* cf = Cm + 3 * (l - m);
-          a = sload(cf);
-          b = sload(cf + 1);
-          c = sload(cf + 2);
-        }
-        const bool odd = j & 1;                    // l0 - m is a multiple of kLChunk2
-#pragma unroll
-        for (int r = 0; r < kAn2Pairs; ++r) {
-          double tp, tm;
-          pol_adv(edge && l == ls, a, b, c, z[r], x1[r], x2[r], y1[r], y2[r], wgt[r], tp, tm);
-          // lambda+ pairs with the (-1)^{l+m} fold, lambda- with the other
-          const double2 qa = odd ? qm[r] : qp[r], qb = odd ? qp[r] : qm[r];
-          const double2 ua = odd ? um[r] : up[r], ub = odd ? up[r] : um[r];
-          er = fma(tp, qa.x, fma(-tm, ub.y, er));
-          ei = fma(tp, qa.y, fma(tm, ub.x, ei));
-          br = fma(tp, ua.x, fma(tm, qb.y, br));
-          bi = fma(tp, ua.y, fma(-tm, qb.x, bi));
-        }
-      }
-      red[j][0][tid] = er;
-      red[j][1][tid] = ei;
-      red[j][2][tid] = br;
-      red[j][3][tid] = bi;
+      a[j] = an[j];
+      an[j] = sload(al + l0 + kLChunk2 + j);
     }
+    double w[P], sum = 0.0;
+    if constexpr (weighted)
 #pragma unroll
-    for (int r = 0; r < kAn2Pairs; ++r)
-      if (!edge || l0 + kLChunk2 > ls) pol_rescale(x1[r], x2[r], y1[r], y2[r], sc[r], wgt[r]);
-    __syncthreads();
-    {
-      // 16 lanes per output, each summing a stride-16 column of the row
-      double h[4];
+      for (int r = 0; r < P; ++r) w[r] = scale_weight(sc[r]);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const double* row = &red[oj][oc][64 * k + g];
-        h[k] = (row[0] + row[16]) + (row[32] + row[48]);
+    for (int j = 0; j < kLChunk2; ++j) {
+      if (edge && l0 + j < ls) continue;
+      double e[4];                                   // E, B (re, im) of this l
+#pragma unroll
+      for (int r = 0; r < P; ++r) {
+        pol_adv(a[j], z[r], x1[r], x2[r], y1[r], y2[r]);
+        if constexpr (PH == kDead) continue;
+        const double x = weighted ? x1[r] * w[r] : x1[r], y = weighted ? y1[r] * w[r] : y1[r];
+        const bool set = r == 0;
+        if (j & 1) {                                 // l0 - m is a multiple of kLChunk2
+          e[0] = fma(y, c4[r].y, set ? -x * c3[r].y : fma(-x, c3[r].y, e[0]));
+          e[1] = fma(-y, c4[r].x, set ? x * c3[r].x : fma(x, c3[r].x, e[1]));
+          e[2] = fma(-y, c2[r].y, set ? x * c1[r].y : fma(x, c1[r].y, e[2]));
+          e[3] = fma(y, c2[r].x, set ? -x * c1[r].x : fma(-x, c1[r].x, e[3]));
+        } else {
+          e[0] = fma(y, c2[r].x, set ? x * c1[r].x : fma(x, c1[r].x, e[0]));
+          e[1] = fma(y, c2[r].y, set ? x * c1[r].y : fma(x, c1[r].y, e[1]));
+          e[2] = fma(y, c4[r].x, set ? x * c3[r].x : fma(x, c3[r].x, e[2]));
+          e[3] = fma(y, c4[r].y, set ? x * c3[r].y : fma(x, c3[r].y, e[3]));
+        }
+        sched_step();
       }
-      const double sum = row16_sum((h[0] + h[1]) + (h[2] + h[3]));
-      const int l = l0 + oj;
-      if (g == 0 && l <= lmax) outp[2 * alm_idx(lmax, l, m) + (oc & 1)] = sum;
+      if constexpr (PH == kOdd) rs.add_apart(j, e, 0xFu, sum);
+      else if constexpr (PH != kDead) rs.add(j, e, sum);
     }
-    __syncthreads();
+    if constexpr (PH != kLive) {
+      double mx = 0.0;
+#pragma unroll
+      for (int r = 0; r < P; ++r) mx = fmax(mx, fmax(fabs(x1[r]), fabs(y1[r])));
+      if (__any(mx > kBig)) {
+#pragma unroll
+        for (int r = 0; r < P; ++r) pol_rescale(x1[r], x2[r], y1[r], y2[r], sc[r]);
+        if (ph != kOdd) ph = phase_of(sc, false);
+      }
+    }
+    return sum;
   };
-  int l0 = m;
-  round(l0, true);
-  for (l0 += kLChunk2; l0 + kLChunk2 - 1 <= lmax; l0 += kLChunk2) round(l0, false);
-  if (l0 <= lmax) round(l0, true);
+  const int rounds = (lmax - m) / kLChunk2 + 1;
+  int i = 0;
+  auto store = [&](double e) {                       // (as in legendre_analysis)
+    const int buf = i / kSumRounds & 1, lb = m + (i & -kSumRounds) * kLChunk2;
+    sums.v[buf][i % kSumRounds][tid] = e;
+    ++i;
+    if (i % kSumRounds != 0 && i != rounds) return;
+    lds_barrier();
+    const int n = tid & 3, g = tid >> 2 & 3, l = lb + (tid >> 4) * kLChunk2 + g;
+    if (tid < 16 * kSumRounds && l <= lmax)
+      ((double*)(part + ((int64_t)(n >> 1) * A.nchunk + chunk) * nalm + i0 + l))[n & 1] =
+          sum_waves<T>(sums.v[buf][tid >> 4], g, n);
+  };
+  using First = std::true_type;
+  using Later = std::false_type;
+  if (m < ls) {
+    if (ph == kOdd) store(round(m, First{}, PhaseC<kOdd>{}));
+    else store(round(m, First{}, PhaseC<kMixed>{}));
+  }
+  while (ph == kOdd && i < rounds) store(round(m + i * kLChunk2, Later{}, PhaseC<kOdd>{}));
+  while (ph == kDead && i < rounds) store(round(m + i * kLChunk2, Later{}, PhaseC<kDead>{}));
+  while (ph != kLive && i < rounds) store(round(m + i * kLChunk2, Later{}, PhaseC<kMixed>{}));
+  while (i < rounds) store(round(m + i * kLChunk2, Later{}, PhaseC<kLive>{}));
 }
+
+// Ring pairs per spin-2 analysis thread: 4, fewer where 256 threads of 4 would
+// outnumber the pairs (512 pairs, lmax 767: 228 us with 4, 177 with 2); with 2 at
+// 2048 pairs, lmax 3071 it takes 7.8 ms instead of 6.7.
+inline int an2_pairs(int npairs) { return npairs > 512 ? 4 : npairs > 256 ? 2 : 1; }
 
 // Spin-2 synthesis: GQ[m][k], GU[m][k] = Q_m, U_m of every ring, kSyn2Pairs
 // ring pairs per thread; lambda+ terms go to the part of the (-1)^{l+m}
 // parity, lambda- terms to the other (north = even + odd, south = even - odd).
-// a_E, a_B and the coefficients of kLChunk2 steps are read ahead with scalar
-// loads.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PSX_SYN2_WAVES)))
-legendre_synthesis_s2(PolArgs A,
-                                                             const double2* __restrict__ aE,
-                                                             const double2* __restrict__ aB,
-                                                             double2* __restrict__ GQ,
-                                                             double2* __restrict__ GU) {
+// The sums that hold X alone and Y alone are
+//   V1, V2 = (Qe +- i Uo)/2,   V3, V4 = (Ue +- i Qo)/2:
+//   l + m even:  V1 += X a_E,    V2 += Y a_E,    V3 += Y a_B,    V4 += X a_B,
+//   l + m odd:   V1 += i X a_B,  V2 -= i Y a_B,  V3 += i Y a_E,  V4 -= i X a_E.
+// a_E, a_B (times t) and the coefficients of kLChunk2 steps are read ahead with
+// scalar loads.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSyn2Waves)))
+legendre_synthesis_s2(PolArgs A, const double2* __restrict__ coef, const int* __restrict__ odd,
+                      double2* __restrict__ GQ, double2* __restrict__ GU) {
+  constexpr int P = kSyn2Pairs;
   const int m = blockIdx.y;
   const int lmax = A.R.lmax;
   const int ls = m > 2 ? m : 2;
-  const int64_t i0 = alm_idx(lmax, m, m);
-  const double2* em = aE + i0;
-  const double2* bm = aB + i0;
-  const double* Cm = A.abc + 3 * i0;
-  double z[kSyn2Pairs], x1[kSyn2Pairs], x2[kSyn2Pairs], y1[kSyn2Pairs], y2[kSyn2Pairs];
-  double wgt[kSyn2Pairs];
-  double2 qe[kSyn2Pairs], qo[kSyn2Pairs], ue[kSyn2Pairs], uo[kSyn2Pairs];
-  int sc[kSyn2Pairs], pr[kSyn2Pairs];
+  const int64_t i0 = alm_idx(lmax, m, m) - m;
+  const double2* const cm = coef + 2 * i0;           // cm[2 l] a_E t, cm[2 l + 1] a_B t
+  const double2* const al = A.ab + i0;
+  const bool keep = odd[m] != 0;
+  double z[P], x1[P], x2[P], y1[P], y2[P];
+  double2 v1[P], v2[P], v3[P], v4[P];
+  int sc[P];
+  const int p0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 * P) + (threadIdx.x & 63);
 #pragma unroll
-  for (int r = 0; r < kSyn2Pairs; ++r) {
-    const int p = (blockIdx.x * kSyn2Pairs + r) * blockDim.x + threadIdx.x;
-    pr[r] = p;
-    const int pp = p < A.R.npairs ? p : 0;
+  for (int r = 0; r < P; ++r) {
+    const bool in = p0 + 64 * r < A.R.npairs;
+    const int pp = in ? p0 + 64 * r : 0;
     z[r] = A.R.z[pp];
-    pol_start(A, pp, m, x1[r], y1[r], sc[r]);
-    wgt[r] = scale_weight(sc[r]);
-    x2[r] = y2[r] = 0.0;
-    qe[r] = qo[r] = ue[r] = uo[r] = make_double2(0.0, 0.0);
+    double xs, ys;
+    pol_start(A, pp, m, xs, ys, sc[r]);
+    if (!in) {
+      xs = ys = 0.0;
+      sc[r] = kNoScale;
+    }
+    x1[r] = y1[r] = 0.0;
+    x2[r] = -xs;
+    y2[r] = -ys;
+    v1[r] = v2[r] = v3[r] = v4[r] = make_double2(0.0, 0.0);
   }
-  // the first round holds l = ls, the last may pass lmax: both take the
-  // checked path, the rounds between load and step unconditionally
-  auto round = [&](const int l0, const bool edge) {
-    double2 e[kLChunk2], b[kLChunk2];
-    double ca[kLChunk2], cb[kLChunk2], cc[kLChunk2];
+  Phase ph = phase_of(sc, keep);
+  // the first round holds l = ls and may hold less, the last may pass lmax
+  auto round = [&](const int l0, const bool edge, auto phase) {
+    constexpr Phase PH = decltype(phase)::value;
+    double2 e[kLChunk2], b[kLChunk2], a[kLChunk2];
 #pragma unroll
     for (int j = 0; j < kLChunk2; ++j) {
       const int l = l0 + j;
-      const bool in = !edge || (l >= ls && l <= lmax);
-      e[j] = in ? sload(em + (l - m)) : make_double2(0.0, 0.0);
-      b[j] = in ? sload(bm + (l - m)) : make_double2(0.0, 0.0);
-      const double* cf = Cm + 3 * (l - m);
-      const bool rec = !edge || (in && l > ls);
-      ca[j] = rec ? sload(cf) : 0.0;
-      cb[j] = rec ? sload(cf + 1) : 0.0;
-      cc[j] = rec ? sload(cf + 2) : 0.0;
+      const bool in = !edge || l <= lmax;
+      if constexpr (PH != kDead) {
+        e[j] = in ? sload(cm + 2 * l) : make_double2(0.0, 0.0);
+        b[j] = in ? sload(cm + 2 * l + 1) : make_double2(0.0, 0.0);
+      }
+      a[j] = in ? sload(al + l) : make_double2(0.0, 0.0);
     }
 #pragma unroll
-    for (int j = 0; j < kLChunk2; ++j) {
-      const int l = l0 + j;
-      if (edge && l > lmax) break;
-      if (edge && l < ls) continue;
-      const bool odd = j & 1;                      // l0 - m is a multiple of kLChunk2
+    for (int r = 0; r < P; ++r) {
+      double w = 1.0;
+      if constexpr (PH == kMixed) w = scale_weight(sc[r]);
 #pragma unroll
-      for (int r = 0; r < kSyn2Pairs; ++r) {
-        double tp, tm;
-        pol_adv(edge && l == ls, ca[j], cb[j], cc[j], z[r], x1[r], x2[r], y1[r], y2[r], wgt[r],
-                tp, tm);
-        // lambda+ a_E and i lambda- a_B (Q); lambda+ a_B and -i lambda- a_E (U)
-        const double2 pq = make_double2(tp * e[j].x, tp * e[j].y);
-        const double2 mq = make_double2(-tm * b[j].y, tm * b[j].x);
-        const double2 pu = make_double2(tp * b[j].x, tp * b[j].y);
-        const double2 mu = make_double2(tm * e[j].y, -tm * e[j].x);
-        const double2 q_e = odd ? mq : pq, q_o = odd ? pq : mq;
-        const double2 u_e = odd ? mu : pu, u_o = odd ? pu : mu;
-        qe[r].x += q_e.x;
-        qe[r].y += q_e.y;
-        qo[r].x += q_o.x;
-        qo[r].y += q_o.y;
-        ue[r].x += u_e.x;
-        ue[r].y += u_e.y;
-        uo[r].x += u_o.x;
-        uo[r].y += u_o.y;
+      for (int j = 0; j < kLChunk2; ++j) {
+        if (edge && l0 + j < ls) continue;
+        pol_adv(a[j], z[r], x1[r], x2[r], y1[r], y2[r]);
+        if constexpr (PH == kDead) continue;
+        const double x = PH == kMixed ? x1[r] * w : x1[r], y = PH == kMixed ? y1[r] * w : y1[r];
+        if (j & 1) {                                 // l0 - m is a multiple of kLChunk2
+          v1[r].x = fma(-x, b[j].y, v1[r].x);
+          v1[r].y = fma(x, b[j].x, v1[r].y);
+          v2[r].x = fma(y, b[j].y, v2[r].x);
+          v2[r].y = fma(-y, b[j].x, v2[r].y);
+          v3[r].x = fma(-y, e[j].y, v3[r].x);
+          v3[r].y = fma(y, e[j].x, v3[r].y);
+          v4[r].x = fma(x, e[j].y, v4[r].x);
+          v4[r].y = fma(-x, e[j].x, v4[r].y);
+        } else {
+          v1[r].x = fma(x, e[j].x, v1[r].x);
+          v1[r].y = fma(x, e[j].y, v1[r].y);
+          v2[r].x = fma(y, e[j].x, v2[r].x);
+          v2[r].y = fma(y, e[j].y, v2[r].y);
+          v3[r].x = fma(y, b[j].x, v3[r].x);
+          v3[r].y = fma(y, b[j].y, v3[r].y);
+          v4[r].x = fma(x, b[j].x, v4[r].x);
+          v4[r].y = fma(x, b[j].y, v4[r].y);
+        }
       }
     }
+    if constexpr (PH != kLive) {
+      double mx = 0.0;
 #pragma unroll
-    for (int r = 0; r < kSyn2Pairs; ++r)
-      if (!edge || l0 + kLChunk2 > ls) pol_rescale(x1[r], x2[r], y1[r], y2[r], sc[r], wgt[r]);
+      for (int r = 0; r < P; ++r) mx = fmax(mx, fmax(fabs(x1[r]), fabs(y1[r])));
+      if (__any(mx > kBig)) {
+#pragma unroll
+        for (int r = 0; r < P; ++r) pol_rescale(x1[r], x2[r], y1[r], y2[r], sc[r]);
+        ph = phase_of(sc, keep);
+      }
+    }
   };
   int l0 = m;
-  round(l0, true);
-  for (l0 += kLChunk2; l0 + kLChunk2 - 1 <= lmax; l0 += kLChunk2) round(l0, false);
-  if (l0 <= lmax) round(l0, true);
+  const int le = lmax - (kLChunk2 - 1);              // the last whole round's l0
+  if (l0 < ls) {
+    round(l0, true, PhaseC<kMixed>{});
+    l0 += kLChunk2;
+  }
+  for (; ph == kDead && l0 <= le; l0 += kLChunk2)
+    round(l0, false, PhaseC<kDead>{});
+  for (; ph != kLive && l0 <= le; l0 += kLChunk2)
+    round(l0, false, PhaseC<kMixed>{});
+  for (; l0 <= le; l0 += kLChunk2) round(l0, false, PhaseC<kLive>{});
+  if (l0 <= lmax) round(l0, true, PhaseC<kMixed>{});
 #pragma unroll
-  for (int r = 0; r < kSyn2Pairs; ++r) {
-    const int p = pr[r];
+  for (int r = 0; r < P; ++r) {
+    const int p = p0 + 64 * r;
     if (p >= A.R.npairs) continue;
     const int kn = p, ks = A.R.nr - 1 - p;
     const int64_t on = gidx(lmax, m, kn), os = gidx(lmax, m, ks);
+    const double2 qe = make_double2(v1[r].x + v2[r].x, v1[r].y + v2[r].y);
+    const double2 ue = make_double2(v3[r].x + v4[r].x, v3[r].y + v4[r].y);
+    const double2 uo = make_double2(v1[r].y - v2[r].y, v2[r].x - v1[r].x);
+    const double2 qo = make_double2(v3[r].y - v4[r].y, v4[r].x - v3[r].x);
     // the factor -1/2 turns 2 lambda+- sums into Q_m, U_m
-    GQ[on] = make_double2(-0.5 * (qe[r].x + qo[r].x), -0.5 * (qe[r].y + qo[r].y));
-    GU[on] = make_double2(-0.5 * (ue[r].x + uo[r].x), -0.5 * (ue[r].y + uo[r].y));
+    GQ[on] = make_double2(-0.5 * (qe.x + qo.x), -0.5 * (qe.y + qo.y));
+    GU[on] = make_double2(-0.5 * (ue.x + uo.x), -0.5 * (ue.y + uo.y));
     if (ks != kn) {
-      GQ[os] = make_double2(-0.5 * (qe[r].x - qo[r].x), -0.5 * (qe[r].y - qo[r].y));
-      GU[os] = make_double2(-0.5 * (ue[r].x - uo[r].x), -0.5 * (ue[r].y - uo[r].y));
+      GQ[os] = make_double2(-0.5 * (qe.x - qo.x), -0.5 * (qe.y - qo.y));
+      GU[os] = make_double2(-0.5 * (ue.x - uo.x), -0.5 * (ue.y - uo.y));
     }
   }
 }
@@ -1422,9 +1638,10 @@ struct ShtPlan {
   int64_t* dfirst = nullptr;
   int64_t* dxoff = nullptr;
   double *dz = nullptr, *dlogsin = nullptr, *dphi0 = nullptr, *dlogc = nullptr;
-  double2* dAB = nullptr;
+  double *dalpha = nullptr, *dscl = nullptr;
   // spin 2, built on first use
-  double *domz = nullptr, *dabc = nullptr, *dlogc2 = nullptr;
+  double *domz = nullptr, *dlogc2 = nullptr, *dscl2 = nullptr;
+  double2* dab2 = nullptr;
   rocfft_plan fwd = nullptr, inv = nullptr;
   rocfft_execution_info info = nullptr;
   void* work = nullptr;
@@ -1465,11 +1682,13 @@ void build_pol_tables(Ctx* c, ShtPlan* P) {
   }
   P->domz = (double*)ctx_alloc(c, sizeof(double) * R.nr);
   P->dlogc2 = (double*)ctx_alloc(c, sizeof(double) * (lmax + 1));
-  P->dabc = (double*)ctx_alloc(c, 3 * sizeof(double) * P->nalm);
+  // (the analysis reads up to two rounds past the last row)
+  P->dab2 = (double2*)ctx_alloc(c, sizeof(double2) * (P->nalm + 2 * kLChunk2));
+  P->dscl2 = (double*)ctx_alloc(c, sizeof(double) * P->nalm);
   PSX_HIP(hipMemcpy(P->domz, omz.data(), sizeof(double) * R.nr, hipMemcpyHostToDevice));
   PSX_HIP(hipMemcpy(P->dlogc2, logc2.data(), sizeof(double) * (lmax + 1), hipMemcpyHostToDevice));
-  dim3 grid((unsigned)((lmax + 1 + 255) / 256), (unsigned)(lmax + 1));
-  hipLaunchKernelGGL(rec_coefs_s2, grid, dim3(256), 0, c->stream, lmax, P->dabc);
+  hipLaunchKernelGGL(rec_coefs_s2, dim3((unsigned)((lmax + 64) / 64)), dim3(64), 0, c->stream, lmax,
+                     P->dab2, P->dscl2);
   PSX_HIP(hipGetLastError());
   PSX_HIP(hipStreamSynchronize(c->stream));
 }
@@ -1479,7 +1698,7 @@ ShtPlan* get_plan(Ctx* c, int nside, int lmax, bool pol = false) {
   auto key = std::make_tuple((void*)c, nside, lmax);
   auto it = g_plans.find(key);
   if (it != g_plans.end()) {
-    if (pol && !it->second->dabc) build_pol_tables(c, it->second);
+    if (pol && !it->second->dab2) build_pol_tables(c, it->second);
     return it->second;
   }
   if (!g_fft_ready) {
@@ -1490,8 +1709,9 @@ ShtPlan* get_plan(Ctx* c, int nside, int lmax, bool pol = false) {
   P->R = make_rings(nside);
   P->lmax = lmax;
   P->nalm = alm_idx(lmax, lmax + 1, lmax + 1);
-  P->nchunk = (P->R.npairs + 256 * kPairsPerThread - 1) / (256 * kPairsPerThread);
-  P->nchunk2 = (P->R.npairs + 256 * kAn2Pairs - 1) / (256 * kAn2Pairs);
+  P->nchunk = (P->R.npairs + an_pairs(P->R.npairs) - 1) / an_pairs(P->R.npairs);
+  const int per2 = 256 * an2_pairs(P->R.npairs);
+  P->nchunk2 = (P->R.npairs + per2 - 1) / per2;
   const Rings& R = P->R;
   P->dn = (int*)ctx_alloc(c, sizeof(int) * R.nr);
   P->dfirst = (int64_t*)ctx_alloc(c, sizeof(int64_t) * R.nr);
@@ -1500,7 +1720,9 @@ ShtPlan* get_plan(Ctx* c, int nside, int lmax, bool pol = false) {
   P->dlogsin = (double*)ctx_alloc(c, sizeof(double) * R.nr);
   P->dphi0 = (double*)ctx_alloc(c, sizeof(double) * R.nr);
   P->dlogc = (double*)ctx_alloc(c, sizeof(double) * (lmax + 1));
-  P->dAB = (double2*)ctx_alloc(c, sizeof(double2) * P->nalm);
+  // alpha, then s (the analysis reads up to two rounds past the last row)
+  P->dalpha = (double*)ctx_alloc(c, sizeof(double) * (2 * P->nalm + 2 * kLChunk));
+  P->dscl = P->dalpha + P->nalm;
   PSX_HIP(hipMemcpy(P->dn, R.n.data(), sizeof(int) * R.nr, hipMemcpyHostToDevice));
   PSX_HIP(hipMemcpy(P->dfirst, R.first.data(), sizeof(int64_t) * R.nr, hipMemcpyHostToDevice));
   PSX_HIP(hipMemcpy(P->dxoff, R.xoff.data(), sizeof(int64_t) * R.nr, hipMemcpyHostToDevice));
@@ -1514,11 +1736,9 @@ ShtPlan* get_plan(Ctx* c, int nside, int lmax, bool pol = false) {
     logc[m] = (double)(0.5L * (logl((2.0L * m + 1.0L) / (4.0L * (long double)kPi)) + acc));
   }
   PSX_HIP(hipMemcpy(P->dlogc, logc.data(), sizeof(double) * (lmax + 1), hipMemcpyHostToDevice));
-  {
-    dim3 grid((unsigned)((lmax + 1 + 255) / 256), (unsigned)(lmax + 1));
-    hipLaunchKernelGGL(rec_coefs, grid, dim3(256), 0, c->stream, lmax, P->dAB);
-    PSX_HIP(hipGetLastError());
-  }
+  hipLaunchKernelGGL(rec_coefs, dim3((unsigned)((lmax + 64) / 64)), dim3(64), 0, c->stream, lmax,
+                     P->dalpha, P->dscl);
+  PSX_HIP(hipGetLastError());
   // equatorial rings: 2 nside + 1 transforms of length 4 nside
   const size_t len = (size_t)4 * nside, batch = (size_t)2 * nside + 1;
   const size_t hl = len / 2 + 1;
@@ -1588,7 +1808,8 @@ void release_sht_plans(Ctx* c) {
 
 namespace {
 
-// Device working set for one map.
+// Device working set for one map of a group; the partial sums of the group's
+// maps are adjacent (launch_synthesis).
 struct ShtBufs {
   double2 *X = nullptr, *Fp = nullptr, *Fm = nullptr, *part = nullptr, *G = nullptr;
   double *syn = nullptr, *res = nullptr;
@@ -1602,7 +1823,8 @@ size_t sht_work_bytes(const ShtPlan& P) {
          2 * sizeof(double) * (size_t)R.npix + 8 * 256;  // 7 buffers, 256-aligned
 }
 
-ShtBufs carve(const ShtPlan& P, void* mem) {
+// n maps' buffers in n (sht_work_bytes, rounded up to 256)
+void carve(const ShtPlan& P, void* mem, int n, ShtBufs* out) {
   const Rings& R = P.R;
   char* p = (char*)mem;
   auto take = [&](size_t b) {
@@ -1611,18 +1833,20 @@ ShtBufs carve(const ShtPlan& P, void* mem) {
     return q;
   };
   const size_t fl = (size_t)(P.lmax + 1) * R.npairs;
-  ShtBufs B;
-  B.X = (double2*)take(sizeof(double2) * R.xlen);
-  B.Fp = (double2*)take(sizeof(double2) * fl);
-  B.Fm = (double2*)take(sizeof(double2) * fl);
-  B.part = (double2*)take(sizeof(double2) * P.nchunk * P.nalm);
-  B.G = (double2*)take(sizeof(double2) * g_elems(P.lmax, R.nr));
-  B.syn = (double*)take(sizeof(double) * R.npix);
-  B.res = (double*)take(sizeof(double) * R.npix);
-  return B;
+  for (int q = 0; q < n; ++q)
+    out[q].part = (double2*)take(sizeof(double2) * P.nchunk * P.nalm);
+  for (int q = 0; q < n; ++q) {
+    ShtBufs& B = out[q];
+    B.X = (double2*)take(sizeof(double2) * R.xlen);
+    B.Fp = (double2*)take(sizeof(double2) * fl);
+    B.Fm = (double2*)take(sizeof(double2) * fl);
+    B.G = (double2*)take(sizeof(double2) * g_elems(P.lmax, R.nr));
+    B.syn = (double*)take(sizeof(double) * R.npix);
+    B.res = (double*)take(sizeof(double) * R.npix);
+  }
 }
 
-LegArgs leg(const ShtPlan& P) { return LegArgs{P.ra(), P.dAB, P.dlogc, P.nchunk}; }
+LegArgs leg(const ShtPlan& P) { return LegArgs{P.ra(), P.dalpha, P.dlogc}; }
 
 // Ring Fourier coefficients of one map, folded into B.Fp, B.Fm.
 void fold_in(Ctx* c, ShtPlan& P, const ShtBufs& B, const double* dmap) {
@@ -1652,34 +1876,48 @@ void launch_analysis(ShtPlan& P, hipStream_t s, const ShtBufs* B) {
     M.in2[q] = B[q].Fm;
     M.out[q] = B[q].part;
   }
-  hipLaunchKernelGGL(legendre_analysis<NM>, dim3((unsigned)P.nchunk, (unsigned)(P.lmax + 1)),
-                     dim3(256), 0, s, leg(P), M);
+  const dim3 grid((unsigned)P.nchunk, (unsigned)(P.lmax + 1));
+  const int np = an_pairs(P.R.npairs);
+  if (np == 2048)
+    hipLaunchKernelGGL((legendre_analysis<NM, 8, 256>), grid, dim3(256), 0, s, leg(P), M);
+  else if (np == 1024)
+    hipLaunchKernelGGL((legendre_analysis<NM, 8, 128>), grid, dim3(128), 0, s, leg(P), M);
+  else if (np == 512)
+    hipLaunchKernelGGL((legendre_analysis<NM, 8, 64>), grid, dim3(64), 0, s, leg(P), M);
+  else
+    hipLaunchKernelGGL((legendre_analysis<NM, 4, 64>), grid, dim3(64), 0, s, leg(P), M);
   PSX_HIP(hipGetLastError());
 }
 
+// (no analysis runs meanwhile: the memory of the group's partial sums holds the
+// scaled a_lm and that of a residual the flags of their rows)
 template <int NM>
 void launch_synthesis(ShtPlan& P, hipStream_t s, const ShtBufs* B, const double2* const* alms) {
   MapPtrs<NM> M{};
+  ScaleArgs<NM> S{};
   for (int q = 0; q < NM; ++q) {
-    M.in[q] = alms[q];
+    S.in[q] = alms[q];
     M.out[q] = B[q].G;
   }
+  S.out = B[0].part;
+  S.odd = (int*)B[0].res;
+  hipLaunchKernelGGL(scale_rows<NM>, dim3((unsigned)(P.lmax + 1)), dim3(256), 0, s, P.lmax,
+                     (const double*)P.dscl, S);
+  PSX_HIP(hipGetLastError());
   constexpr int SP = syn_pairs(NM);
   hipLaunchKernelGGL(legendre_synthesis<NM>,
                      dim3((unsigned)((P.R.npairs + 256 * SP - 1) / (256 * SP)),
                           (unsigned)(P.lmax + 1)),
-                     dim3(256), 0, s, leg(P), M);
+                     dim3(256), 0, s, leg(P), (const double2*)S.out, (const int*)S.odd, M);
   PSX_HIP(hipGetLastError());
 }
 
 // maps per analysis pass (the analysis holds each map's F+- of its ring pairs
 // in registers and reduces 2 values per map and l through LDS)
-#ifndef PSX_AN_GROUP
-#define PSX_AN_GROUP 2
-#endif
+constexpr int kAnGroup = 2;
 
 // alms[q] (+)= A(maps[q]) for a group of nm <= kMaxGroup maps: Legendre passes
-// of up to PSX_AN_GROUP maps (the recurrence shared), ring transforms per map.
+// of up to kAnGroup maps (the recurrence shared), ring transforms per map.
 // The maps of each analysis launch are folded just before it; `before`, if
 // given, is called with q before map q is first read.
 void analysis_group(Ctx* c, ShtPlan& P, const ShtBufs* B, int nm, const double* const* maps,
@@ -1687,23 +1925,22 @@ void analysis_group(Ctx* c, ShtPlan& P, const ShtBufs* B, int nm, const double* 
                     const std::function<void(int)>* before = nullptr) {
   PSX_REQUIRE(nm >= 1 && nm <= kMaxGroup, PSX_ERR_ARGUMENT, "1..4 maps per transform group");
   hipStream_t s = c->stream;
-  for (int q0 = 0; q0 < nm; q0 += PSX_AN_GROUP) {
-    const int k = std::min(PSX_AN_GROUP, nm - q0);
+  for (int q0 = 0; q0 < nm; q0 += kAnGroup) {
+    const int k = std::min(kAnGroup, nm - q0);
     for (int q = q0; q < q0 + k; ++q) {
       if (before) (*before)(q);
       fold_in(c, P, B[q], maps[q]);
     }
     switch (k) {
       case 1: launch_analysis<1>(P, s, B + q0); break;
-      case 2: launch_analysis<2>(P, s, B + q0); break;
-      case 3: launch_analysis<3>(P, s, B + q0); break;
-      default: launch_analysis<4>(P, s, B + q0); break;
+      default: launch_analysis<2>(P, s, B + q0); break;
     }
   }
   const double w = 4.0 * kPi / (double)P.R.npix;
   for (int q = 0; q < nm; ++q) {
     hipLaunchKernelGGL(sum_partials, dim3((unsigned)((P.nalm + 255) / 256)), dim3(256), 0, s,
-                       B[q].part, P.nchunk, P.nalm, w, accumulate ? 1 : 0, alms[q]);
+                       B[q].part, P.nchunk, P.nalm, w, (const double*)P.dscl, accumulate ? 1 : 0,
+                       alms[q]);
     PSX_HIP(hipGetLastError());
   }
 }
@@ -1773,7 +2010,7 @@ PolBufs carve_pol(const ShtPlan& P, void* mem) {
   return B;
 }
 
-PolArgs pleg(const ShtPlan& P) { return PolArgs{P.ra(), P.domz, P.dabc, P.dlogc2, P.nchunk2}; }
+PolArgs pleg(const ShtPlan& P) { return PolArgs{P.ra(), P.domz, P.dab2, P.dlogc2, P.nchunk2}; }
 
 // Ring Fourier coefficients of one real map, folded into F+ and F-.
 void ring_fold(Ctx* c, ShtPlan& P, const double* dmap, double2* X, double2* Fp, double2* Fm) {
@@ -1819,18 +2056,21 @@ void analysis_pol(Ctx* c, ShtPlan& P, const PolBufs& B, const double* dQ, const 
   hipStream_t s = c->stream;
   ring_fold(c, P, dQ, B.X[0], B.F, B.F + B.fs);
   ring_fold(c, P, dU, B.X[1], B.F + 2 * B.fs, B.F + 3 * B.fs);
-  hipLaunchKernelGGL(legendre_analysis_s2, dim3((unsigned)P.nchunk2, (unsigned)(P.lmax + 1)),
-                     dim3(256), 0, s, pleg(P), (const double2*)B.F, B.fs, B.part);
+  const auto an = an2_pairs(R.npairs) == 4   ? legendre_analysis_s2<4>
+                  : an2_pairs(R.npairs) == 2 ? legendre_analysis_s2<2>
+                                             : legendre_analysis_s2<1>;
+  hipLaunchKernelGGL(an, dim3((unsigned)P.nchunk2, (unsigned)(P.lmax + 1)), dim3(256), 0, s,
+                     pleg(P), (const double2*)B.F, B.fs, B.part);
   PSX_HIP(hipGetLastError());
   // the kernel sums 2 lambda+- terms; a_E, a_B carry -w
   const double w = -0.5 * 4.0 * kPi / (double)R.npix;
   const unsigned nb = (unsigned)((P.nalm + 255) / 256);
   hipLaunchKernelGGL(sum_partials, dim3(nb), dim3(256), 0, s, (const double2*)B.part, P.nchunk2,
-                     P.nalm, w, accumulate ? 1 : 0, aE);
+                     P.nalm, w, (const double*)P.dscl2, accumulate ? 1 : 0, aE);
   PSX_HIP(hipGetLastError());
   hipLaunchKernelGGL(sum_partials, dim3(nb), dim3(256), 0, s,
                      (const double2*)(B.part + (int64_t)P.nchunk2 * P.nalm), P.nchunk2, P.nalm, w,
-                     accumulate ? 1 : 0, aB);
+                     (const double*)P.dscl2, accumulate ? 1 : 0, aB);
   PSX_HIP(hipGetLastError());
 }
 
@@ -1838,10 +2078,16 @@ void analysis_pol(Ctx* c, ShtPlan& P, const PolBufs& B, const double* dQ, const 
 void synthesis_pol(Ctx* c, ShtPlan& P, const PolBufs& B, const double2* aE, const double2* aB,
                    double* dQ, double* dU) {
   const Rings& R = P.R;
+  // (as for one map: the memory of the partial sums and of the residual is free)
+  ScaleArgs<2> S{{aE, aB}, B.part, (int*)B.res};
+  hipLaunchKernelGGL(scale_rows<2>, dim3((unsigned)(P.lmax + 1)), dim3(256), 0, c->stream, P.lmax,
+                     (const double*)P.dscl2, S);
+  PSX_HIP(hipGetLastError());
   hipLaunchKernelGGL(legendre_synthesis_s2,
                      dim3((unsigned)((R.npairs + 256 * kSyn2Pairs - 1) / (256 * kSyn2Pairs)),
                           (unsigned)(P.lmax + 1)),
-                     dim3(256), 0, c->stream, pleg(P), aE, aB, B.G[0], B.G[1]);
+                     dim3(256), 0, c->stream, pleg(P), (const double2*)S.out, (const int*)S.odd,
+                     B.G[0], B.G[1]);
   PSX_HIP(hipGetLastError());
   ring_unfold(c, P, B.G[0], B.X[0], dQ);
   ring_unfold(c, P, B.G[1], B.X[1], dU);
@@ -1873,7 +2119,7 @@ void map2alm_ptrs(Ctx* c, int nside, int lmax, int niter, int n, const double* c
   const int gmax = std::min(n, kMaxGroup);
   WorkBuf wk(c, per * (size_t)std::max(gmax, 1));
   ShtBufs B[kMaxGroup];
-  for (int q = 0; q < gmax; ++q) B[q] = carve(P, (char*)wk.base() + q * per);
+  carve(P, wk.base(), gmax, B);
   const int64_t npix = P.R.npix;
   for (int g0 = 0; g0 < n; g0 += kMaxGroup) {
     const int nm = std::min(kMaxGroup, n - g0);
@@ -1930,7 +2176,7 @@ void alm2map_dev(Ctx* c, int nside, int lmax, int nmaps, const double* dalms, do
   const int gmax = std::min(nmaps, kMaxGroup);
   WorkBuf wk(c, per * (size_t)std::max(gmax, 1));
   ShtBufs B[kMaxGroup];
-  for (int q = 0; q < gmax; ++q) B[q] = carve(P, (char*)wk.base() + q * per);
+  carve(P, wk.base(), gmax, B);
   for (int g0 = 0; g0 < nmaps; g0 += kMaxGroup) {
     const int nm = std::min(kMaxGroup, nmaps - g0);
     const double2* alm[kMaxGroup];
@@ -2097,7 +2343,7 @@ int psx_mask_spectra(psx_ctx* h, int nside, int lmax, int niter, int nmaps, cons
     double* dc = x.take(cb);
     // the first analysis launch's maps go in first; the others are copied on
     // the copy stream while that launch and its ring transforms run
-    const int first = std::min(nmaps, PSX_AN_GROUP);
+    const int first = std::min(nmaps, kAnGroup);
     h2d_matrix(c, dm, npix, maps, npix, npix, first);
     const std::function<void(int)> rest = [&](int q) {
       if (q == first)

@@ -343,3 +343,65 @@ def test_alm2cl_device_limits(pkg, ctx):
         ctx.alm2cl([a[:5]], 2)
     with pytest.raises(pkg.ArgumentError):
         ctx.alm2cl([a[:0]], -1)
+
+
+def _alm_dot(a, b, lmax):
+    """sum over all m, negative ones too, of Re(conj(a) b), a real field's alm."""
+    w = np.full(a.shape[-1], 2.0)
+    w[:lmax + 1] = 1.0
+    return float((w * (a.conj() * b).real).sum())
+
+
+@pytest.mark.parametrize("nside,lmax", [
+    (1, 0), (1, 4), (2, 3), (64, 129), (128, 257), (128, 300), (256, 515), (512, 1026),
+])
+def test_analysis_is_the_adjoint_of_synthesis(pkg, ctx, nside, lmax):
+    # map2alm without refinement is 4 pi/npix times the transpose of alm2map, at
+    # each split of the ring pairs over threads and for ragged last rounds of l.
+    # Either side's relative L2 error is below 5e-14 here, so by Cauchy-Schwarz
+    # the two products differ by at most 1e-13 |S a| |m|.
+    rng = np.random.default_rng(100 * nside + lmax)
+    npix, na = 12 * nside * nside, (lmax + 1) * (lmax + 2) // 2
+    w = 4.0 * np.pi / npix
+
+    def alms(n):
+        a = rng.standard_normal((n, na)) + 1j * rng.standard_normal((n, na))
+        a[:, :lmax + 1] = a[:, :lmax + 1].real
+        return a
+
+    for n in (1, 2, 3, 4):
+        a, m = alms(n), rng.standard_normal((n, npix))
+        s, t = ctx.alm2map(a, nside, lmax), ctx.map2alm(m, nside, lmax, 0)
+        for q in range(n):
+            lhs, rhs = w * float(s[q] @ m[q]), _alm_dot(a[q], t[q], lmax)
+            assert abs(lhs - rhs) <= 1e-13 * w * np.linalg.norm(s[q]) * np.linalg.norm(m[q])
+    if lmax < 2:
+        return
+    a, m = alms(3), rng.standard_normal((3, npix))
+    s = np.asarray(ctx.alm2map_pol(a, nside, lmax)).reshape(3, npix)
+    t = np.asarray(ctx.map2alm_pol(m, nside, lmax, 0)).reshape(3, na)
+    a[1:, np.concatenate([[0, 1], [lmax + 1]])] = 0.0      # no E, B below l = 2
+    lhs = w * float((s[1:] * m[1:]).sum())
+    rhs = sum(_alm_dot(a[k], t[k], lmax) for k in (1, 2))
+    assert abs(lhs - rhs) <= 1e-13 * w * np.linalg.norm(s[1:]) * np.linalg.norm(m[1:])
+
+
+@pytest.mark.parametrize("nside,lmax", [(16, 40), (256, 600)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 1e300])
+def test_values_that_are_not_finite_stay_in_their_map(pkg, ctx, nside, lmax, bad):
+    rng = np.random.default_rng(5)
+    npix, na = 12 * nside * nside, (lmax + 1) * (lmax + 2) // 2
+    m = rng.standard_normal((2, npix))
+    m[0, 3] = bad
+    t = ctx.map2alm(m, nside, lmax, 0)
+    assert np.array_equal(t[1], ctx.map2alm(m[1:], nside, lmax, 0)[0])
+    if np.isfinite(bad):
+        assert np.isfinite(t[0]).all() and abs(t[0][0]) > 1e290
+    else:
+        assert not np.isfinite(t[0].real).any()
+    a = rng.standard_normal((2, na)) + 1j * rng.standard_normal((2, na))
+    a[:, :lmax + 1] = a[:, :lmax + 1].real
+    a[0, na - 2] = bad                              # of high m: the caps are far below it
+    s = ctx.alm2map(a, nside, lmax)
+    assert np.array_equal(s[1], ctx.alm2map(a[1:], nside, lmax)[0])
+    assert np.isfinite(s[0]).all() if np.isfinite(bad) else not np.isfinite(s[0]).any()
