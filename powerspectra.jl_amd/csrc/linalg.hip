@@ -725,6 +725,153 @@ size_t lu_work_bytes(int n) {
   return move_off + sizeof(int) * (8 * kLuPanel + 1) + 256;
 }
 
+// ---- triangular solves with many right-hand sides ---------------------------
+// Blocked left substitution X = T^{-1} B for the LU factors (T = unit lower L
+// or upper U) and m right-hand sides, in kTsmRows-row blocks: the diagonal
+// block is solved by substitution (trsm_block), and the rows still to come are
+// updated by a rocBLAS GEMM of depth kTsmRows.  Substitution keeps LAPACK's
+// backward error on ill-conditioned U, which a trsm built on inverted diagonal
+// blocks does not.
+//   A wave takes kTsmCols right-hand sides, lane i holding rows i, i + 64, ..
+// of the block; the value solved at a step goes through scalar registers to
+// all lanes.  The triangle passes through LDS, kTsmAhead columns at a time,
+// one set ahead of the steps, so that a workgroup's waves read it from L2
+// once: with each wave reading it for itself the L2 bounds the kernel (103 and
+// 169 us at m = 2509; 34 and 58 us with LDS).  Issue-bound on the broadcasts,
+// the quotients and the updates.  64-row blocks, one right-hand side a thread,
+// ran 45 us each (180 for 256 rows) on 14 workgroups, and their depth-64 GEMMs
+// were bound by the traffic of B.
+constexpr int kTsmRows = 256;
+constexpr int kTsmCols = 2;
+constexpr int kTsmWaves = 8;
+constexpr int kTsmAhead = 16;
+
+// ROWS: rows the diagonal block has at most.
+template <bool UPPER, int ROWS>
+__global__ void __launch_bounds__(64 * kTsmWaves) trsm_block(const double* __restrict__ A,
+                                                             int64_t lda, int n, int R0,
+                                                             double* __restrict__ B, int64_t ldb,
+                                                             int m) {
+  constexpr int kTsmSub = ROWS / 64;
+  constexpr int kTsmStage = kTsmAhead * ROWS / (64 * kTsmWaves);  // values a thread stages
+  __shared__ double Ts[2][kTsmAhead][ROWS];
+  const int t = threadIdx.x, lane = t & 63;
+  const int col0 = __builtin_amdgcn_readfirstlane(
+      ((int)blockIdx.x * kTsmWaves + (t >> 6)) * kTsmCols);
+  const int cn = min(ROWS, n - R0);
+  const double* T = A + R0 + (int64_t)R0 * lda;     // T[row + column lda]
+  double* b = B + R0 + (int64_t)col0 * ldb;
+  // acc: what the sub-blocks already solved take from one still to come,
+  // summed by itself and subtracted once, as the GEMM between blocks does
+  double x[kTsmSub][kTsmCols], acc[kTsmSub][kTsmCols], d[kTsmSub], rd[kTsmSub];
+  bool plain = true;
+#pragma unroll
+  for (int s = 0; s < kTsmSub; ++s) {
+    const int r = 64 * s + lane;
+#pragma unroll
+    for (int q = 0; q < kTsmCols; ++q) {
+      x[s][q] = r < cn && col0 + q < m ? b[r + (int64_t)q * ldb] : 0.0;
+      acc[s][q] = 0.0;
+    }
+    d[s] = UPPER && r < cn ? T[r + (int64_t)r * lda] : 1.0;
+    rd[s] = 1.0 / d[s];
+    plain &= fabs(d[s]) > 0x1p-1000 && fabs(d[s]) < 0x1p1000;
+  }
+  // every pivot's reciprocal in the normal range: quotients by it, with one
+  // residual correction (the correctly rounded quotient)
+  const bool fast = __builtin_amdgcn_ballot_w64(!plain) == 0;
+  // sets of kTsmAhead columns, from the first (lower) or last (upper) that
+  // holds one of the block; a thread stages kTsmStage of a set's entries in
+  // its row, zero beyond the block
+  const int row = t % ROWS, part = (t / ROWS) * kTsmStage;
+  double ahead[kTsmStage];
+  auto load = [&](int f) {
+#pragma unroll
+    for (int e = 0; e < kTsmStage; ++e) {
+      const int j = f * kTsmAhead + part + e;
+      ahead[e] = row < cn && j < cn ? T[row + (int64_t)j * lda] : 0.0;
+    }
+  };
+  constexpr int kSets = 64 / kTsmAhead;             // of a 64-row sub-block
+  const int last = (cn - 1) / kTsmAhead;
+  load(UPPER ? last : 0);
+#pragma unroll
+  for (int ss = 0; ss < kTsmSub; ++ss) {
+    const int s = UPPER ? kTsmSub - 1 - ss : ss;
+    const int f0 = s * kSets, f1 = min(f0 + kSets - 1, last);
+#pragma unroll
+    for (int c = 0; c < kTsmCols; ++c) x[s][c] -= acc[s][c];
+#pragma unroll 1
+    for (int i = f0; i <= f1; ++i) {
+      const int f = UPPER ? f1 - (i - f0) : i, buf = f & 1;
+#pragma unroll
+      for (int e = 0; e < kTsmStage; ++e) Ts[buf][part + e][row] = ahead[e];
+      __syncthreads();                              // also ends the reads of set f -+ 1
+      const int nf = UPPER ? f - 1 : f + 1;
+      if (nf >= 0 && nf <= last) load(nf);
+      const int j0 = (f - f0) * kTsmAhead;
+#pragma unroll
+      for (int u = 0; u < kTsmAhead; ++u) {
+        const int e = UPPER ? kTsmAhead - 1 - u : u, j = j0 + e;
+        const bool off = UPPER ? lane < j : lane > j;
+        double tv[kTsmSub];
+#pragma unroll
+        for (int q = 0; q < kTsmSub; ++q)
+          if (UPPER ? q <= s : q >= s) tv[q] = Ts[buf][e][64 * q + lane];
+#pragma unroll
+        for (int c = 0; c < kTsmCols; ++c) {
+          double y = x[s][c], xj;
+          if (UPPER) {
+            if (fast) {
+              const double z = y * rd[s];
+              const double w = fma(fma(-z, d[s], y), rd[s], z);
+              xj = lu_lane(w, j);
+              // an overflow, whose correction is NaN, or a NaN: divide
+              if ((__double2hiint(xj) & 0x7ff00000) != 0x7ff00000) {
+                y = w;
+              } else {
+                y = y / d[s];
+                xj = lu_lane(y, j);
+              }
+            } else {
+              y = y / d[s];
+              xj = lu_lane(y, j);
+            }
+          } else {
+            xj = lu_lane(y, j);
+          }
+          const double own = fma(-tv[s], xj, x[s][c]);
+          x[s][c] = off ? own : (UPPER && lane == j) ? y : x[s][c];
+#pragma unroll
+          for (int q = 0; q < kTsmSub; ++q)
+            if (UPPER ? q < s : q > s) acc[q][c] = fma(tv[q], xj, acc[q][c]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < kTsmSub; ++s) {
+    const int r = 64 * s + lane;
+#pragma unroll
+    for (int q = 0; q < kTsmCols; ++q)
+      if (r < cn && col0 + q < m) b[r + (int64_t)q * ldb] = x[s][q];
+  }
+}
+
+static unsigned trsm_grid(int m) {
+  return (unsigned)((m + kTsmWaves * kTsmCols - 1) / (kTsmWaves * kTsmCols));
+}
+
+// U rows of the factorization: B (nb x m) = L^{-1} B with the unit lower nb x nb
+// block at A, nb <= ROWS, in the same matrix.  (rocBLAS's trsm inverts diagonal
+// blocks and multiplies in several launches: 85 us at nb = 128, m = 2400 to 6000.)
+template <int ROWS>
+static void panel_trsm(hipStream_t s, int nb, const double* A, int64_t lda, double* B, int m) {
+  hipLaunchKernelGGL((trsm_block<false, ROWS>), dim3(trsm_grid(m)), dim3(64 * kTsmWaves), 0, s, A,
+                     lda, nb, 0, B, lda, m);
+  PSX_HIP(hipGetLastError());
+}
+
 // dA (n x n) becomes its LU factors; the interchanges are applied to the nrhs
 // columns of dB on the way.
 void lu_factor_on(const LuLane& L, int n, double* dA, int64_t lda, int* dipiv, int* dinfo,
@@ -774,10 +921,8 @@ void lu_factor_on(const LuLane& L, int n, double* dA, int64_t lda, int* dipiv, i
         hipLaunchKernelGGL(lu_leaf_move, dim3((nb + 255) / 256), dim3(256), 0, s,
                            dA + (int64_t)k * lda, lda, nb, cl, nc, k, w);
         if (cend < kend)   // rest of the panel: U = L11^-1 A
-          PSX_ROC(rocblas_dtrsm(h, rocblas_side_left, rocblas_fill_lower,
-                                rocblas_operation_none, rocblas_diagonal_unit, nc, kend - cend,
-                                &one, dA + cl + (int64_t)cl * lda, (rocblas_int)lda,
-                                dA + cl + (int64_t)cend * lda, (rocblas_int)lda));
+          panel_trsm<64>(s, nc, dA + cl + (int64_t)cl * lda, lda, dA + cl + (int64_t)cend * lda,
+                         kend - cend);
       }
       if (!deferred) {
         if (k > 0)
@@ -810,9 +955,7 @@ void lu_factor_on(const LuLane& L, int n, double* dA, int64_t lda, int* dipiv, i
     if (kend < n) {        // trailing matrix
       double* L11 = dA + k + (int64_t)k * lda;
       double* A12 = dA + k + (int64_t)kend * lda;
-      PSX_ROC(rocblas_dtrsm(h, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none,
-                            rocblas_diagonal_unit, nb, n - kend, &one, L11, (rocblas_int)lda,
-                            A12, (rocblas_int)lda));
+      panel_trsm<kLuPanel>(s, nb, L11, lda, A12, n - kend);
       PSX_ROC(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, n - kend, n - kend,
                             nb, &mone, dA + kend + (int64_t)k * lda, (rocblas_int)lda, A12,
                             (rocblas_int)lda, &one, dA + kend + (int64_t)kend * lda,
@@ -982,138 +1125,6 @@ void lu_trs_dev(Ctx* c, int n, const double* dA, int64_t lda, double* dx) {
   lu_trs_on(c->stream, n, dA, lda, dx);
 }
 
-// ---- triangular solves with many right-hand sides ---------------------------
-// Blocked left substitution X = T^{-1} B for the LU factors (T = unit lower L
-// or upper U) and m right-hand sides, in kTsmRows-row blocks: the diagonal
-// block is solved by substitution (trsm_block), and the rows still to come are
-// updated by a rocBLAS GEMM of depth kTsmRows.  Substitution keeps LAPACK's
-// backward error on ill-conditioned U, which a trsm built on inverted diagonal
-// blocks does not.
-//   A wave takes kTsmCols right-hand sides, lane i holding rows i, i + 64, ..
-// of the block; the value solved at a step goes through scalar registers to
-// all lanes.  The triangle passes through LDS, kTsmAhead columns at a time,
-// one set ahead of the steps, so that a workgroup's waves read it from L2
-// once: with each wave reading it for itself the L2 bounds the kernel (103 and
-// 169 us at m = 2509; 34 and 58 us with LDS).  Issue-bound on the broadcasts,
-// the quotients and the updates.  64-row blocks, one right-hand side a thread,
-// ran 45 us each (180 for 256 rows) on 14 workgroups, and their depth-64 GEMMs
-// were bound by the traffic of B.
-constexpr int kTsmRows = 256;
-constexpr int kTsmSub = kTsmRows / 64;
-constexpr int kTsmCols = 2;
-constexpr int kTsmWaves = 8;
-constexpr int kTsmAhead = 16;
-constexpr int kTsmStage = kTsmAhead * kTsmRows / (64 * kTsmWaves);  // values a thread stages
-
-template <bool UPPER>
-__global__ void __launch_bounds__(64 * kTsmWaves) trsm_block(const double* __restrict__ A,
-                                                             int64_t lda, int n, int R0,
-                                                             double* __restrict__ B, int64_t ldb,
-                                                             int m) {
-  __shared__ double Ts[2][kTsmAhead][kTsmRows];
-  const int t = threadIdx.x, lane = t & 63;
-  const int col0 = __builtin_amdgcn_readfirstlane(
-      ((int)blockIdx.x * kTsmWaves + (t >> 6)) * kTsmCols);
-  const int cn = min(kTsmRows, n - R0);
-  const double* T = A + R0 + (int64_t)R0 * lda;     // T[row + column lda]
-  double* b = B + R0 + (int64_t)col0 * ldb;
-  // acc: what the sub-blocks already solved take from one still to come,
-  // summed by itself and subtracted once, as the GEMM between blocks does
-  double x[kTsmSub][kTsmCols], acc[kTsmSub][kTsmCols], d[kTsmSub], rd[kTsmSub];
-  bool plain = true;
-#pragma unroll
-  for (int s = 0; s < kTsmSub; ++s) {
-    const int r = 64 * s + lane;
-#pragma unroll
-    for (int q = 0; q < kTsmCols; ++q) {
-      x[s][q] = r < cn && col0 + q < m ? b[r + (int64_t)q * ldb] : 0.0;
-      acc[s][q] = 0.0;
-    }
-    d[s] = UPPER && r < cn ? T[r + (int64_t)r * lda] : 1.0;
-    rd[s] = 1.0 / d[s];
-    plain &= fabs(d[s]) > 0x1p-1000 && fabs(d[s]) < 0x1p1000;
-  }
-  // every pivot's reciprocal in the normal range: quotients by it, with one
-  // residual correction (the correctly rounded quotient)
-  const bool fast = __builtin_amdgcn_ballot_w64(!plain) == 0;
-  // sets of kTsmAhead columns, from the first (lower) or last (upper) that
-  // holds one of the block; a thread stages kTsmStage of a set's entries in
-  // its row, zero beyond the block
-  const int row = t % kTsmRows, part = (t / kTsmRows) * kTsmStage;
-  double ahead[kTsmStage];
-  auto load = [&](int f) {
-#pragma unroll
-    for (int e = 0; e < kTsmStage; ++e) {
-      const int j = f * kTsmAhead + part + e;
-      ahead[e] = row < cn && j < cn ? T[row + (int64_t)j * lda] : 0.0;
-    }
-  };
-  constexpr int kSets = 64 / kTsmAhead;             // of a 64-row sub-block
-  const int last = (cn - 1) / kTsmAhead;
-  load(UPPER ? last : 0);
-#pragma unroll
-  for (int ss = 0; ss < kTsmSub; ++ss) {
-    const int s = UPPER ? kTsmSub - 1 - ss : ss;
-    const int f0 = s * kSets, f1 = min(f0 + kSets - 1, last);
-#pragma unroll
-    for (int c = 0; c < kTsmCols; ++c) x[s][c] -= acc[s][c];
-#pragma unroll 1
-    for (int i = f0; i <= f1; ++i) {
-      const int f = UPPER ? f1 - (i - f0) : i, buf = f & 1;
-#pragma unroll
-      for (int e = 0; e < kTsmStage; ++e) Ts[buf][part + e][row] = ahead[e];
-      __syncthreads();                              // also ends the reads of set f -+ 1
-      const int nf = UPPER ? f - 1 : f + 1;
-      if (nf >= 0 && nf <= last) load(nf);
-      const int j0 = (f - f0) * kTsmAhead;
-#pragma unroll
-      for (int u = 0; u < kTsmAhead; ++u) {
-        const int e = UPPER ? kTsmAhead - 1 - u : u, j = j0 + e;
-        const bool off = UPPER ? lane < j : lane > j;
-        double tv[kTsmSub];
-#pragma unroll
-        for (int q = 0; q < kTsmSub; ++q)
-          if (UPPER ? q <= s : q >= s) tv[q] = Ts[buf][e][64 * q + lane];
-#pragma unroll
-        for (int c = 0; c < kTsmCols; ++c) {
-          double y = x[s][c], xj;
-          if (UPPER) {
-            if (fast) {
-              const double z = y * rd[s];
-              const double w = fma(fma(-z, d[s], y), rd[s], z);
-              xj = lu_lane(w, j);
-              // an overflow, whose correction is NaN, or a NaN: divide
-              if ((__double2hiint(xj) & 0x7ff00000) != 0x7ff00000) {
-                y = w;
-              } else {
-                y = y / d[s];
-                xj = lu_lane(y, j);
-              }
-            } else {
-              y = y / d[s];
-              xj = lu_lane(y, j);
-            }
-          } else {
-            xj = lu_lane(y, j);
-          }
-          const double own = fma(-tv[s], xj, x[s][c]);
-          x[s][c] = off ? own : (UPPER && lane == j) ? y : x[s][c];
-#pragma unroll
-          for (int q = 0; q < kTsmSub; ++q)
-            if (UPPER ? q < s : q > s) acc[q][c] = fma(tv[q], xj, acc[q][c]);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int s = 0; s < kTsmSub; ++s) {
-    const int r = 64 * s + lane;
-#pragma unroll
-    for (int q = 0; q < kTsmCols; ++q)
-      if (r < cn && col0 + q < m) b[r + (int64_t)q * ldb] = x[s][q];
-  }
-}
-
 // B (n x m, ldb) = T^{-1} B with T the unit lower (UPPER false) or upper
 // factor packed in dA.
 static void trsm_left_dev(Ctx* c, bool upper, int n, const double* dA, int64_t lda, double* dB,
@@ -1121,15 +1132,15 @@ static void trsm_left_dev(Ctx* c, bool upper, int n, const double* dA, int64_t l
   rocblas_handle h = blas(c);
   hipStream_t s = c->stream;
   const int nb = (n + kTsmRows - 1) / kTsmRows;
-  const unsigned g = (unsigned)((m + kTsmWaves * kTsmCols - 1) / (kTsmWaves * kTsmCols));
+  const unsigned g = trsm_grid(m);
   const double one = 1.0, mone = -1.0;
   for (int q = 0; q < nb; ++q) {
     const int R0 = (upper ? nb - 1 - q : q) * kTsmRows, cn = std::min(kTsmRows, n - R0);
     if (upper)
-      hipLaunchKernelGGL(trsm_block<true>, dim3(g), dim3(64 * kTsmWaves), 0, s, dA, lda, n, R0, dB,
+      hipLaunchKernelGGL((trsm_block<true, kTsmRows>), dim3(g), dim3(64 * kTsmWaves), 0, s, dA, lda, n, R0, dB,
                          ldb, m);
     else
-      hipLaunchKernelGGL(trsm_block<false>, dim3(g), dim3(64 * kTsmWaves), 0, s, dA, lda, n, R0, dB,
+      hipLaunchKernelGGL((trsm_block<false, kTsmRows>), dim3(g), dim3(64 * kTsmWaves), 0, s, dA, lda, n, R0, dB,
                          ldb, m);
     PSX_HIP(hipGetLastError());
     if (!upper && R0 + cn < n)  // rows below: B2 -= L21 X1
