@@ -676,12 +676,6 @@ struct RoundSums {
     }
   }
 };
-// Keeps the pairs' steps in order, their vector instructions at least: left to
-// itself the compiler runs each sum's dependent chain in one piece, and two waves a
-// SIMD do not cover its latency.
-__device__ __forceinline__ void sched_step() {
-  __builtin_amdgcn_sched_barrier(0x4 | 0x8 | 0x10 | 0x80);   // scalar, matrix, memory, LDS pass
-}
 // Coefficients up to this keep every sum of an analysis finite: |L_lm| < 2^14 and
 // 2^13 ring pairs.
 constexpr double kHuge = 0x1p960;
@@ -806,7 +800,6 @@ legendre_analysis(LegArgs A, MapPtrs<NM> M) {
           c[2 * q] = r == 0 ? lt * f.x : fma(lt, f.x, c[2 * q]);
           c[2 * q + 1] = r == 0 ? lt * f.y : fma(lt, f.y, c[2 * q + 1]);
         }
-        sched_step();
       }
       if (NM == 1 && !(j & 1)) continue;
       const int g = NM == 1 ? j >> 1 : j;
@@ -1345,7 +1338,6 @@ legendre_analysis_s2(PolArgs A, const double2* __restrict__ F, int64_t fs,
           e[2] = fma(y, c4[r].x, set ? x * c3[r].x : fma(x, c3[r].x, e[2]));
           e[3] = fma(y, c4[r].y, set ? x * c3[r].y : fma(x, c3[r].y, e[3]));
         }
-        sched_step();
       }
       if constexpr (PH == kOdd) rs.add_apart(j, e, 0xFu, sum);
       else if constexpr (PH != kDead) rs.add(j, e, sum);
