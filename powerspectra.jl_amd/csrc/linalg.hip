@@ -261,11 +261,13 @@ __global__ void __launch_bounds__(kLuRows) lu_leaf_col(double* A, int64_t lda, i
 // Multipliers are stored in place as they are made; pivot rows are kept in LDS
 // from their column on.  After the columns, wave 0 turns the pivots into
 // LAPACK's interchanges and the leaf's own columns are reordered.
-//   Measured: 42, 54 and 60 us a 32-column leaf of 512, 1024 and 1536 rows, 32
-// to 40 us a 16-column one of 2048 to 3072, 22 to 29 us an 8-column one of 4096
-// to 6144: 1.3 to 3.6 us a column, against 2.6 to 3.7 with 1024 threads and all
-// columns unrolled, and 5.7 for a launch per column above 3072 rows.  Device
-// solves: n = 2509 13.7 -> 7.5 ms, n = 6144 45.9 -> 28.3 ms.
+//   Measured: 44, 53 and 57 us a 32-column leaf of 512, 1024 and 1536 rows, 28
+// to 34 us a 16-column one of 2048 to 3072, 19 to 25 us an 8-column one of 4096
+// to 6144: 1.4 to 3.1 us a column, against 2.6 to 3.7 with 1024 threads and all
+// columns unrolled, and 5.7 for a launch per column above 3072 rows.  Bound by the
+// instructions a row takes, 31 vector and 29 scalar ones with a mask for the rows
+// still live (28 us at 6144 rows), and by a column's chain of steps below that.
+// Device solves: n = 2509 13.7 -> 7 ms, n = 6144 45.9 -> 26 ms.
 constexpr int kLuWgThreads = 512;
 constexpr int kLuWgWaves = kLuWgThreads / 64;
 constexpr int kLuWgRowsMax = 12 * kLuWgThreads;  // leaf rows one workgroup takes
@@ -317,10 +319,14 @@ struct LuSlots {
 };
 
 // Up to kLuStage columns from column j0 of the leaf on, WD columns still live
-// at its start (register q holds column j + q at step j).
+// at its start (register q holds column j + q at step j).  Rows that are gone
+// (pivots, bit k of `gone`, and rows past the matrix) hold zeros, which no search
+// with a positive maximum picks and no update changes, so that the rows need no
+// masks; a column whose maximum in a wave is zero or that holds an Inf or NaN is
+// searched row by row with them.
 template <int NR, int W, int WD>
-__device__ __forceinline__ void lu_wg_stage(double (&vals)[NR][W], bool (&live)[NR], int t, int c,
-                                            int j0, int nc, double* A, int64_t lda,
+__device__ __forceinline__ void lu_wg_stage(double (&vals)[NR][W], unsigned& gone, int t, int c,
+                                            int j0, int nc, int n, double* A, int64_t lda,
                                             LuSlots<W>& s, double (*P)[W], int* spiv,
                                             const LuWork& w) {
   const int lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -328,25 +334,50 @@ __device__ __forceinline__ void lu_wg_stage(double (&vals)[NR][W], bool (&live)[
 #pragma unroll 1
   for (int j = j0; j < j1; ++j) {
     const int B = j & 1;
+    int kw, lw;
     {
-      double v = -1.0;
-      bool nan = false;
+      double v = fabs(vals[0][0]), odd = 0.0 * vals[0][0];
+      int kv = 0;
 #pragma unroll
-      for (int k = 0; k < NR; ++k) {
-        const double x = vals[k][0];
-        nan |= live[k] & (x != x);
-        v = lu_max(v, live[k] ? fabs(x) : -1.0);
+      for (int k = 1; k < NR; ++k) {
+        const double x = fabs(vals[k][0]);
+        kv = x > v ? k : kv;
+        v = lu_max(v, x);
+        odd = fma(0.0, vals[k][0], odd);
       }
       double mx = lu_wave_max(v);
-      if (__builtin_amdgcn_ballot_w64(nan)) mx = INFINITY;
-      // the lowest row that reaches it: rows ascend with k, then with the lane
-      int kw = -1, lw = 0;
+      if (mx > 0.0 && !__builtin_amdgcn_ballot_w64(odd != 0.0)) {
+        // the lowest row that reaches it: rows ascend with k, then with the lane
+        unsigned long long m = __builtin_amdgcn_ballot_w64(v == mx);
+        if (m & (m - 1)) {
+          int k = 0;
+          unsigned long long mk;
+          while (!(mk = m & __builtin_amdgcn_ballot_w64(kv == k))) ++k;
+          m = mk;
+        }
+        lw = __builtin_ctzll(m);
+        kw = __builtin_amdgcn_readlane(kv, lw);
+      } else {
+        double u = -1.0;
+        bool nan = false;
 #pragma unroll
-      for (int k = NR - 1; k >= 0; --k) {
-        const unsigned long long m =
-            __builtin_amdgcn_ballot_w64(live[k] & !(fabs(vals[k][0]) < mx));
-        kw = m ? k : kw;
-        lw = m ? __builtin_ctzll(m) : lw;
+        for (int k = 0; k < NR; ++k) {
+          const double x = vals[k][0];
+          if (!(gone >> k & 1)) {
+            nan |= x != x;
+            u = fmax(u, fabs(x));
+          }
+        }
+        mx = __builtin_amdgcn_ballot_w64(nan) ? (double)INFINITY : lu_wave_max(u);
+        kw = -1;
+        lw = 0;
+#pragma unroll
+        for (int k = NR - 1; k >= 0; --k) {
+          const unsigned long long m =
+              __builtin_amdgcn_ballot_w64(!(gone >> k & 1) && !(fabs(vals[k][0]) < mx));
+          kw = m ? k : kw;
+          lw = m ? __builtin_ctzll(m) : lw;
+        }
       }
 #pragma unroll
       for (int k = 0; k < NR; ++k)
@@ -388,8 +419,17 @@ __device__ __forceinline__ void lu_wg_stage(double (&vals)[NR][W], bool (&live)[
       spiv[j] = p;
       if (piv == 0.0 && *w.info == 0) *w.info = c + j + 1;
     }
+    if (g == wv) {                       // the pivot row is gone
 #pragma unroll
-    for (int k = 0; k < NR; ++k) live[k] &= c + t + kLuWgThreads * k != p;
+      for (int k = 0; k < NR; ++k)
+        if (kw == k) {
+          if (lane == lw) {
+            gone |= 1u << k;
+#pragma unroll
+            for (int q = 0; q < WD; ++q) vals[k][q] = 0.0;
+          }
+        }
+    }
     double* a = A + (int64_t)(c + j) * lda + c + t;
     // quotients by the rounded reciprocal with one residual correction: the
     // correctly rounded quotient (|value| <= |pivot|); pivots whose reciprocal
@@ -408,9 +448,12 @@ __device__ __forceinline__ void lu_wg_stage(double (&vals)[NR][W], bool (&live)[
 #pragma unroll
       for (int k = 0; k < NR; ++k) l[k] = vals[k][0] / by;
     }
+    // (a row that is gone stores what nothing reads; the last ones may lie past
+    // the matrix)
+    constexpr int kSure = NR > 6 ? NR - 2 : NR - 1;
 #pragma unroll
     for (int k = 0; k < NR; ++k)
-      if (live[k]) a[kLuWgThreads * k] = l[k];
+      if (k < kSure || c + t + kLuWgThreads * k < n) a[kLuWgThreads * k] = l[k];
 #pragma unroll
     for (int q = 1; q < WD; ++q) {
       const double u = lu_lane(ul, q);
@@ -474,22 +517,23 @@ __global__ void __launch_bounds__(kLuWgThreads) lu_leaf_wg(double* A, int64_t ld
   const int t = threadIdx.x;
   const int nc = cend - c;
   double vals[NR][W];
-  bool live[NR];
+  unsigned gone = 0;
 #pragma unroll
   for (int k = 0; k < NR; ++k) {
     const int r = c + t + kLuWgThreads * k;
-    live[k] = r < n;
+    const bool in = r < n;
+    gone |= (unsigned)!in << k;
 #pragma unroll
     for (int jj = 0; jj < W; ++jj)
-      vals[k][jj] = (live[k] && jj < nc) ? A[r + (int64_t)(c + jj) * lda] : 0.0;
+      vals[k][jj] = (in && jj < nc) ? A[r + (int64_t)(c + jj) * lda] : 0.0;
   }
-  lu_wg_stage<NR, W, W>(vals, live, t, c, 0, nc, A, lda, slots, P, spiv, w);
+  lu_wg_stage<NR, W, W>(vals, gone, t, c, 0, nc, n, A, lda, slots, P, spiv, w);
   if constexpr (W > kLuStage)
-    lu_wg_stage<NR, W, W - kLuStage>(vals, live, t, c, kLuStage, nc, A, lda, slots, P, spiv, w);
+    lu_wg_stage<NR, W, W - kLuStage>(vals, gone, t, c, kLuStage, nc, n, A, lda, slots, P, spiv, w);
   if constexpr (W > 2 * kLuStage) {
-    lu_wg_stage<NR, W, W - 2 * kLuStage>(vals, live, t, c, 2 * kLuStage, nc, A, lda, slots, P,
+    lu_wg_stage<NR, W, W - 2 * kLuStage>(vals, gone, t, c, 2 * kLuStage, nc, n, A, lda, slots, P,
                                          spiv, w);
-    lu_wg_stage<NR, W, W - 3 * kLuStage>(vals, live, t, c, 3 * kLuStage, nc, A, lda, slots, P,
+    lu_wg_stage<NR, W, W - 3 * kLuStage>(vals, gone, t, c, 3 * kLuStage, nc, n, A, lda, slots, P,
                                          spiv, w);
   }
   if (t < W) dest[t] = -1;
