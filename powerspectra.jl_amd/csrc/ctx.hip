@@ -329,6 +329,9 @@ constexpr int kCopyThreads = 11;                    // and the calling thread
 constexpr size_t kChunkBytes = size_t(1) << 20;
 constexpr size_t kTaskBytes = size_t(768) << 10;    // of a chunk, per task
 constexpr size_t kInlineBytes = size_t(256) << 10;  // copied by the caller itself
+// one piece up to this goes to the runtime as it is, which copies it at once: a slot,
+// its event and the pinned copy take 6 us more
+constexpr size_t kDirectBytes = size_t(16) << 10;
 }  // namespace
 
 CopyPool::CopyPool(int threads) {
@@ -660,6 +663,11 @@ void h2d_matrix_x(Ctx* c, double* dev, int64_t ldd, const double* host, int64_t 
 
 void h2d_pieces(Ctx* c, void* dev, const std::vector<HostPiece>& pieces) {
   ensure_stage(c);
+  if (pieces.size() == 1 && pieces[0].bytes <= kDirectBytes) {
+    PSX_HIP(hipMemcpyAsync((char*)dev + pieces[0].offset, pieces[0].host, pieces[0].bytes,
+                           hipMemcpyHostToDevice, c->stream));
+    return;
+  }
   size_t end = 0;
   for (const HostPiece& p : pieces) end = std::max(end, p.offset + p.bytes);
   if (end <= Stage::kSlotBytes) {
