@@ -320,8 +320,9 @@ int psx_memcpy_d2h(psx_ctx* h, void* dst, const void* src, size_t bytes) {
 // through a ring of pinned slots: the DMA runs ahead in some while host threads
 // copy others, a chunk split between several threads, which also fault in a
 // fresh destination's pages.  Chunks are an eighth of the transfer, at most a
-// slot (8 MB, 147 us at 57 GB/s: 2 MB chunks lost 20 % of that rate between
-// DMAs on 400 MB) and at least kChunkBytes, so that short ones overlap too.
+// slot (12 MB, 220 us at 57 GB/s: 2 MB chunks lost 20 % of that rate between
+// DMAs on 400 MB, 8 MB ones 3 % where a transfer comes in 25 pieces) and at least
+// kChunkBytes, so that short ones overlap too.
 namespace psx {
 
 namespace {

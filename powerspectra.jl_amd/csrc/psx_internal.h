@@ -93,8 +93,8 @@ class CopyPool {
 // A ring of pinned slots for staged copies on one stream at a time.  Slots are
 // allocated as a copy needs them, and kept.
 struct Stage {
-  static constexpr size_t kSlotBytes = size_t(8) << 20;
-  static constexpr int kSlots = 8;
+  static constexpr size_t kSlotBytes = size_t(12) << 20;
+  static constexpr int kSlots = 5;
   struct Slot {
     char* p = nullptr;
     hipEvent_t ev = nullptr;        // the slot's last DMA
