@@ -328,6 +328,7 @@ namespace psx {
 namespace {
 constexpr int kCopyThreads = 11;                    // and the calling thread
 constexpr size_t kChunkBytes = size_t(1) << 20;
+constexpr int kParts = 8;                           // chunks of a transfer, where they fit
 constexpr size_t kTaskBytes = size_t(768) << 10;    // of a chunk, per task
 constexpr size_t kInlineBytes = size_t(256) << 10;  // copied by the caller itself
 // one piece up to this goes to the runtime as it is, which copies it at once: a slot,
@@ -460,10 +461,10 @@ void cut(std::vector<Chunk>& ch, int64_t most, double* host, int64_t ldh, double
     ch.push_back({host + j * ldh, ldh, dev + j * ldd, ldd, rows, std::min(cpc, cols - j), after});
 }
 
-// doubles a chunk holds in a transfer of `total`
-int64_t chunk_doubles(int64_t total) {
+// doubles a chunk holds in a transfer of `total` in about `parts` chunks
+int64_t chunk_doubles(int64_t total, int parts = kParts) {
   const int64_t lo = kChunkBytes / sizeof(double), hi = Stage::kSlotBytes / sizeof(double);
-  return std::min(hi, std::max(lo, (total / 8 + 511) & ~int64_t(511)));
+  return std::min(hi, std::max(lo, (total / parts + 511) & ~int64_t(511)));
 }
 
 void copy_cols(double* dst, int64_t ldd, const double* src, int64_t lds, int64_t rows,
@@ -607,12 +608,13 @@ void h2d_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chun
 }
 }  // namespace
 
-void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatrix* m, int nm) {
+void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatrix* m, int nm,
+                     int parts) {
   std::vector<Chunk> ch;
   int64_t total = 0;
   for (int i = 0; i < nm; ++i)
     total += std::max<int64_t>(m[i].rows, 0) * std::max<int64_t>(m[i].cols, 0);
-  const int64_t most = chunk_doubles(total);
+  const int64_t most = chunk_doubles(total, parts);
   for (int i = 0; i < nm; ++i)
     cut(ch, most, m[i].host, m[i].ldh, const_cast<double*>(m[i].dev), m[i].ldd, m[i].rows, m[i].cols,
         m[i].after);
@@ -621,7 +623,7 @@ void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatri
 
 void d2h_matrices(Ctx* c, const D2HMatrix* m, int nm) {
   ensure_stage(c);
-  d2h_matrices_on(c->stream, c->stage, *c->pool, m, nm);
+  d2h_matrices_on(c->stream, c->stage, *c->pool, m, nm, kParts);
 }
 
 void d2h_matrix(Ctx* c, double* host, int64_t ldh, const double* dev, int64_t ldd,
@@ -632,7 +634,7 @@ void d2h_matrix(Ctx* c, double* host, int64_t ldh, const double* dev, int64_t ld
 
 void d2h_matrices_overlapped(Ctx* c, const D2HMatrix* m, int nm) {
   ensure_stage(c);
-  d2h_matrices_on(c->xstream, c->stage, *c->pool, m, nm);
+  d2h_matrices_on(c->xstream, c->stage, *c->pool, m, nm, kParts);
 }
 
 namespace {

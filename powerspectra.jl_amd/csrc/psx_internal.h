@@ -231,8 +231,9 @@ void d2h_matrices(Ctx* c, const D2HMatrix* m, int nm);
 // the same on the context's copy stream, so that the pieces waiting for
 // events of the context stream copy out while later work there still runs
 void d2h_matrices_overlapped(Ctx* c, const D2HMatrix* m, int nm);
-// the same on stream s through the caller's slots
-void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatrix* m, int nm);
+// the same on stream s through the caller's slots, in about `parts` chunks
+void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatrix* m, int nm,
+                     int parts);
 void h2d_matrix(Ctx* c, double* dev, int64_t ldd, const double* host, int64_t ldh,
                 int64_t rows, int64_t cols);
 // The same copy through the slots on the context's copy stream, behind earlier
