@@ -3,9 +3,10 @@
 // (src/covariance.jl:8-14).  Julia's `lu` is LAPACK getrf with partial
 // pivoting and throws SingularException on an exact zero pivot.  The
 // factorisation is this file's blocked getrf (HIP leaf kernels + rocBLAS
-// updates) in LAPACK layout; the solves apply its interchanges (a gather for
-// many columns, rocSOLVER's laswp for a few) and run this file's forward and
-// back substitution (rocBLAS updates between diagonal blocks).
+// updates) in LAPACK layout; right-hand sides at hand move their rows with its
+// panels, decouple_covmat's second ones by a gather (rocSOLVER's laswp above
+// kPermMax rows), and this file's forward and back substitution follow (rocBLAS
+// updates between diagonal blocks).
 #include "psx_internal.h"
 
 #include <utility>
@@ -52,8 +53,8 @@ void dgemm_dev(Ctx* c, int m, int n, int k, const double* dA, int64_t lda, const
 }
 
 // ---- LU with partial pivoting ---------------------------------------------
-// Right-looking blocked getrf.  Panels of kLuPanel columns end with a trailing
-// update by rocBLAS (dtrsm + dgemm of depth kLuPanel).  Inside a panel, leaves
+// Right-looking blocked getrf.  Panels of kLuPanel columns end with their U rows
+// (panel_trsm) and a trailing rocBLAS dgemm of depth kLuPanel.  Inside a panel, leaves
 // of 8 to 32 columns are factored by one workgroup holding the leaf's rows in
 // registers (lu_leaf_wg), or, above kLuWgRowsMax rows, one column per launch
 // (lu_leaf_col).  Ties in |pivot| go to the smallest row index, NaN ranks
