@@ -49,6 +49,7 @@ constexpr int kLChunk = 8;                  // most l values between rescalings
 // waves took 1.8x as long at nside 1024, lmax 3071).
 constexpr int kSyn2Pairs = 2, kSyn2Waves = 5;
 constexpr int kSynChunk = 4;                // l values read ahead per synthesis round
+constexpr int kTabPad = 2 * kLChunk;        // coefficients past the last row: up to two rounds
 constexpr double kBig = 0x1p600;            // rescaling threshold
 constexpr double kInvBig = 0x1p-600;
 constexpr double kLnBig = 415.88830833596718565;  // 600 ln 2
@@ -511,12 +512,16 @@ __global__ void __launch_bounds__(256) fold_analysis(RingArgs R, const double2* 
 // two operations a step instead of three; s_l multiplies the a_lm instead
 // (before a synthesis, after an analysis).  alpha comes from the rounded s, so
 // every step is exact to a few ulp of its own whatever the rounding of the
-// product behind s_l.  alpha and s per (l, m), in a_lm order; alpha_m is 0.
+// product behind s_l.  alpha and s per (l, m), in a_lm order; alpha_m is 0, and
+// so are the entries past the last row that the analysis steps over: what a step
+// past lmax gives is added, times 0, to the sums of its round.
 __global__ void __launch_bounds__(64) rec_coefs(int lmax, double* __restrict__ alpha,
                                                 double* __restrict__ scl) {
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m > lmax) return;
   const int64_t i0 = alm_idx(lmax, m, m) - m;
+  if (m == lmax)
+    for (int i = 1; i <= kTabPad; ++i) alpha[i0 + lmax + i] = 0.0;
   const double M = m;
   double s = 1.0;
   alpha[i0 + m] = 0.0;
@@ -1155,13 +1160,16 @@ struct PolArgs {
 // Y_l / t_l with t_l t_{l-1} = a_l, t = 1 at l = max(m, 2):
 //   X_l = (alpha z + beta) X_{l-1} - X_{l-2},  alpha = t_{l-1}^2, beta = alpha b/a
 // (t is applied to a_E, a_B as s is to a_lm).  alpha, beta and t per (l, m), in
-// a_lm order, 0 below l = max(m, 2), where t is 1 and alpha, beta still 0.  The
-// integer products stay below 2^53 for l <= 8191.
+// a_lm order, 0 below l = max(m, 2), where t is 1 and alpha, beta still 0, and 0
+// past the last row as in rec_coefs.  The integer products stay below 2^53 for
+// l <= 8191.
 __global__ void __launch_bounds__(64) rec_coefs_s2(int lmax, double2* __restrict__ ab,
                                                    double* __restrict__ scl) {
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m > lmax) return;
   const int64_t i0 = alm_idx(lmax, m, m) - m;
+  if (m == lmax)
+    for (int i = 1; i <= kTabPad; ++i) ab[i0 + lmax + i] = make_double2(0.0, 0.0);
   const int ls = m > 2 ? m : 2;
   const double M = m;
   double t = 1.0;
@@ -1674,8 +1682,7 @@ void build_pol_tables(Ctx* c, ShtPlan* P) {
   }
   P->domz = (double*)ctx_alloc(c, sizeof(double) * R.nr);
   P->dlogc2 = (double*)ctx_alloc(c, sizeof(double) * (lmax + 1));
-  // (the analysis reads up to two rounds past the last row)
-  P->dab2 = (double2*)ctx_alloc(c, sizeof(double2) * (P->nalm + 2 * kLChunk2));
+  P->dab2 = (double2*)ctx_alloc(c, sizeof(double2) * (P->nalm + kTabPad));
   P->dscl2 = (double*)ctx_alloc(c, sizeof(double) * P->nalm);
   PSX_HIP(hipMemcpy(P->domz, omz.data(), sizeof(double) * R.nr, hipMemcpyHostToDevice));
   PSX_HIP(hipMemcpy(P->dlogc2, logc2.data(), sizeof(double) * (lmax + 1), hipMemcpyHostToDevice));
@@ -1712,9 +1719,9 @@ ShtPlan* get_plan(Ctx* c, int nside, int lmax, bool pol = false) {
   P->dlogsin = (double*)ctx_alloc(c, sizeof(double) * R.nr);
   P->dphi0 = (double*)ctx_alloc(c, sizeof(double) * R.nr);
   P->dlogc = (double*)ctx_alloc(c, sizeof(double) * (lmax + 1));
-  // alpha, then s (the analysis reads up to two rounds past the last row)
-  P->dalpha = (double*)ctx_alloc(c, sizeof(double) * (2 * P->nalm + 2 * kLChunk));
-  P->dscl = P->dalpha + P->nalm;
+  // alpha and its padding, then s
+  P->dalpha = (double*)ctx_alloc(c, sizeof(double) * (2 * P->nalm + kTabPad));
+  P->dscl = P->dalpha + P->nalm + kTabPad;
   PSX_HIP(hipMemcpy(P->dn, R.n.data(), sizeof(int) * R.nr, hipMemcpyHostToDevice));
   PSX_HIP(hipMemcpy(P->dfirst, R.first.data(), sizeof(int64_t) * R.nr, hipMemcpyHostToDevice));
   PSX_HIP(hipMemcpy(P->dxoff, R.xoff.data(), sizeof(int64_t) * R.nr, hipMemcpyHostToDevice));

@@ -405,3 +405,41 @@ def test_values_that_are_not_finite_stay_in_their_map(pkg, ctx, nside, lmax, bad
     s = ctx.alm2map(a, nside, lmax)
     assert np.array_equal(s[1], ctx.alm2map(a[1:], nside, lmax)[0])
     assert np.isfinite(s[0]).all() if np.isfinite(bad) else not np.isfinite(s[0]).any()
+
+
+def _recycled_memory(pkg, sizes, value):
+    """Freed device blocks of the given sizes, filled with value."""
+    c = pkg.Context(0)
+    try:
+        held = []
+        for b in sizes:
+            for _ in range(48):
+                held.append(c.alloc(b))
+                c.h2d(held[-1], np.full(b // 8, value))
+        for p in held:
+            c.free(p)
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("nside,lmax", [(1, 0), (1, 1), (1, 2), (1, 3), (2, 8), (16, 40), (64, 129)])
+def test_transforms_do_not_depend_on_memory_left_by_others(pkg, nside, lmax):
+    # the passes step past lmax on what follows a plan's tables, which may be
+    # memory that held anything
+    rng = np.random.default_rng(nside + lmax)
+    npix, na = 12 * nside * nside, (lmax + 1) * (lmax + 2) // 2
+    m = rng.standard_normal((3, npix))
+    sizes = [16 * (na + 8), 16 * (na + 16), 8 * (2 * na + 16)]
+    outs = []
+    for value in (0.0, np.nan, np.inf, 1e308):
+        _recycled_memory(pkg, sizes, value)
+        c = pkg.Context(0)
+        try:
+            outs.append([c.map2alm(m[:1], nside, lmax, 0), c.map2alm(m[:2], nside, lmax, 0)]
+                        + ([c.map2alm_pol(m, nside, lmax, 0)] if lmax >= 2 else []))
+        finally:
+            c.close()
+    for o in outs[1:]:
+        for a, b in zip(o, outs[0]):
+            assert np.isfinite(np.asarray(a).view(float)).all()
+            assert np.array_equal(a, b)
