@@ -681,9 +681,12 @@ struct RoundSums {
     }
   }
 };
-// Coefficients up to this keep every sum of an analysis finite: |L_lm| < 2^14 and
-// 2^13 ring pairs.
-constexpr double kHuge = 0x1p960;
+// Coefficients up to this keep every sum of an analysis finite, those of the up to
+// seven steps past lmax on the next rows' coefficients too, since they reach the
+// others times 0: |L_lm| < 2^14; two steps in a row grow by at most 2^16 (the
+// product of their alphas is A^2 <= 2m + 3, or smaller where a row begins), seven by
+// 2^63; 2^13 ring pairs.
+constexpr double kHuge = 0x1p920;
 
 // The waves' sums of kSumRounds rounds gather in LDS and are added up and stored
 // together: one barrier and one run of stores per block of rounds.  The round's

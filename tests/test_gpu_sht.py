@@ -443,3 +443,17 @@ def test_transforms_do_not_depend_on_memory_left_by_others(pkg, nside, lmax):
         for a, b in zip(o, outs[0]):
             assert np.isfinite(np.asarray(a).view(float)).all()
             assert np.array_equal(a, b)
+
+
+# on either side of the line above which the lanes of an analysis are summed apart
+@pytest.mark.parametrize("k", [880, 912, 922, 958])
+@pytest.mark.parametrize("nside,lmax", [(8, 13), (256, 603)])
+def test_analysis_of_very_large_maps_scales(pkg, ctx, nside, lmax, k):
+    # the two sides sum in different orders: relative L2 errors below 5e-14 each
+    rng = np.random.default_rng(k)
+    m = rng.standard_normal((3, 12 * nside * nside))
+    for f in (lambda x: ctx.map2alm(x[:2], nside, lmax, 0),
+              lambda x: np.asarray(ctx.map2alm_pol(x, nside, lmax, 0)).reshape(3, -1)):
+        t, u = f(m), f(m * 2.0 ** k) * 2.0 ** -k
+        for q in range(len(t)):
+            assert np.linalg.norm(u[q] - t[q]) <= 1e-13 * np.linalg.norm(t[q])
