@@ -1645,6 +1645,7 @@ struct ShtPlan {
   // spin 2, built on first use
   double *domz = nullptr, *dlogc2 = nullptr, *dscl2 = nullptr;
   double2* dab2 = nullptr;
+  bool pol = false;
   rocfft_plan fwd = nullptr, inv = nullptr;
   rocfft_execution_info info = nullptr;
   void* work = nullptr;
@@ -1683,16 +1684,18 @@ void build_pol_tables(Ctx* c, ShtPlan* P) {
     logc2[m] = (double)(0.5L * logl((2.0L * m + 1.0L) / (4.0L * (long double)kPi)) + lk -
                         (long double)(m - 2) * logl(2.0L));
   }
-  P->domz = (double*)ctx_alloc(c, sizeof(double) * R.nr);
-  P->dlogc2 = (double*)ctx_alloc(c, sizeof(double) * (lmax + 1));
-  P->dab2 = (double2*)ctx_alloc(c, sizeof(double2) * (P->nalm + kTabPad));
-  P->dscl2 = (double*)ctx_alloc(c, sizeof(double) * P->nalm);
+  // an allocation that fails leaves the others to the next call
+  if (!P->domz) P->domz = (double*)ctx_alloc(c, sizeof(double) * R.nr);
+  if (!P->dlogc2) P->dlogc2 = (double*)ctx_alloc(c, sizeof(double) * (lmax + 1));
+  if (!P->dab2) P->dab2 = (double2*)ctx_alloc(c, sizeof(double2) * (P->nalm + kTabPad));
+  if (!P->dscl2) P->dscl2 = (double*)ctx_alloc(c, sizeof(double) * P->nalm);
   PSX_HIP(hipMemcpy(P->domz, omz.data(), sizeof(double) * R.nr, hipMemcpyHostToDevice));
   PSX_HIP(hipMemcpy(P->dlogc2, logc2.data(), sizeof(double) * (lmax + 1), hipMemcpyHostToDevice));
   hipLaunchKernelGGL(rec_coefs_s2, dim3((unsigned)((lmax + 64) / 64)), dim3(64), 0, c->stream, lmax,
                      P->dab2, P->dscl2);
   PSX_HIP(hipGetLastError());
   PSX_HIP(hipStreamSynchronize(c->stream));
+  P->pol = true;
 }
 
 ShtPlan* get_plan(Ctx* c, int nside, int lmax, bool pol = false) {
@@ -1700,7 +1703,7 @@ ShtPlan* get_plan(Ctx* c, int nside, int lmax, bool pol = false) {
   auto key = std::make_tuple((void*)c, nside, lmax);
   auto it = g_plans.find(key);
   if (it != g_plans.end()) {
-    if (pol && !it->second->dab2) build_pol_tables(c, it->second);
+    if (pol && !it->second->pol) build_pol_tables(c, it->second);
     return it->second;
   }
   if (!g_fft_ready) {

@@ -457,3 +457,37 @@ def test_analysis_of_very_large_maps_scales(pkg, ctx, nside, lmax, k):
         t, u = f(m), f(m * 2.0 ** k) * 2.0 ** -k
         for q in range(len(t)):
             assert np.linalg.norm(u[q] - t[q]) <= 1e-13 * np.linalg.norm(t[q])
+
+
+def test_transform_after_a_refused_allocation(pkg):
+    # the budget ends at each of a polarised transform's device allocations in
+    # turn; with the space back, the same context gives what a fresh one gives
+    nside, lmax = 16, 40
+    na = (lmax + 1) * (lmax + 2) // 2
+    rng = np.random.default_rng(9)
+    teb = rng.standard_normal((3, na)) + 1j * rng.standard_normal((3, na))
+    teb[:, :lmax + 1] = teb[:, :lmax + 1].real
+    total = 1 << 26
+
+    def attempt(room):
+        c = pkg.Context(0, hbm_budget=total)
+        try:
+            hold = c.alloc(total - c.bytes_in_use() - room)
+            try:
+                c.alm2map_pol(teb, nside, lmax)
+            except pkg.BudgetError:
+                c.free(hold)
+                return False, np.asarray(c.alm2map_pol(teb, nside, lmax))
+            return True, np.asarray(c.alm2map_pol(teb, nside, lmax))
+        finally:
+            c.close()
+
+    ref = attempt(total // 2)[1]
+    step, refused = 8 * na - 256, 0     # less than the last table's size
+    for room in range(8, total // 2, step):
+        done, out = attempt(room)
+        assert np.array_equal(out, ref)
+        if done:
+            break
+        refused += 1
+    assert done and refused > 10
