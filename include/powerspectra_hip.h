@@ -232,7 +232,8 @@ int psx_decouple_covmat(psx_ctx* ctx, int n, const double* Y, const double* B1,
 int psx_lu_solve(psx_ctx* ctx, int n, const double* A, int64_t lda,
                  double* B, int64_t ldb, int nrhs);
 /* The same on device buffers: dA is overwritten by its LU factors and dB by
- * the solution; enqueued on the context stream, returns when done. */
+ * the solution; enqueued on the context stream, returns when done.  A zero
+ * pivot returns PSX_ERR_SINGULAR and leaves dB as it was. */
 int psx_lu_solve_d(psx_ctx* ctx, int n, double* dA, int64_t lda, double* dB, int64_t ldb,
                    int nrhs);
 /* The joint EE/BB (sign = +1) or EB/BE (sign = -1) decoupling solve

@@ -1236,6 +1236,24 @@ __global__ void __launch_bounds__(256) lu_permute_cols(const int* __restrict__ p
   for (int i = threadIdx.x; i < n; i += 256) b[i] = col[perm[i]];
 }
 
+// The row order of B before LAPACK's interchanges, one thread per column (after a
+// zero pivot only).
+__global__ void __launch_bounds__(64) lu_undo_swaps(const int* __restrict__ ipiv, int n,
+                                                    double* __restrict__ B, int64_t ldb,
+                                                    int nrhs) {
+  const int col = (int)(blockIdx.x * 64 + threadIdx.x);
+  if (col >= nrhs) return;
+  double* b = B + (int64_t)col * ldb;
+  for (int i = n - 1; i >= 0; --i) {
+    const int q = ipiv[i] - 1;
+    if (q > i && q < n) {
+      const double t = b[i];
+      b[i] = b[q];
+      b[q] = t;
+    }
+  }
+}
+
 // A device array for LAPACK's interchanges: n entries, the info slot at n + 32.
 static size_t pivot_bytes(int n) {
   return (sizeof(int) * ((size_t)n + 64) + 255) & ~size_t(255);
@@ -1252,20 +1270,36 @@ static void check_pivots(Ctx* c, int n, const int* ipiv) {
                   " (Julia SingularException)");
 }
 
-// dA (n x n, lda) becomes its LU factors, dB (n x nrhs) A^{-1} dB.
+// dA (n x n, lda) becomes its LU factors, dB (n x nrhs) A^{-1} dB.  With keep_b a
+// singular matrix leaves dB as it was: the pivots are looked at before the
+// substitution (a wait, which callers with a copy of their own do without) and the
+// rows moved with the panels go back.
 void lu_solve_dev(Ctx* c, int n, double* dA, int64_t lda, double* dB, int64_t ldb,
-                  int nrhs) {
+                  int nrhs, bool keep_b) {
   const size_t wb = (lu_work_bytes(n) + 255) & ~size_t(255);
   char* work = (char*)ctx_scratch(c, wb + pivot_bytes(n));
   int* ipiv = (int*)(work + wb);
   lu_factor_on(LuLane{c->stream, blas(c), work}, n, dA, lda, ipiv, ipiv + n + 32, dB, ldb, nrhs);
+  if (keep_b) {
+    try {
+      check_pivots(c, n, ipiv);
+    } catch (const Error& e) {
+      if (e.code == PSX_ERR_SINGULAR && nrhs > 0) {
+        hipLaunchKernelGGL(lu_undo_swaps, dim3((unsigned)((nrhs + 63) / 64)), dim3(64), 0,
+                           c->stream, (const int*)ipiv, n, dB, ldb, nrhs);
+        (void)hipStreamSynchronize(c->stream);
+      }
+      throw;
+    }
+  }
   if (nrhs <= kTrsMaxRhs) {
     for (int j = 0; j < nrhs; ++j) lu_trs_dev(c, n, dA, lda, dB + (int64_t)j * ldb);
   } else {
     trsm_left_dev(c, false, n, dA, lda, dB, ldb, nrhs);
     trsm_left_dev(c, true, n, dA, lda, dB, ldb, nrhs);
   }
-  check_pivots(c, n, ipiv);
+  if (keep_b) PSX_HIP(hipStreamSynchronize(c->stream));
+  else check_pivots(c, n, ipiv);
 }
 
 // Independent systems side by side.  System i runs on lane i: lane 0 is the
@@ -1500,7 +1534,7 @@ int psx_lu_solve_d(psx_ctx* hctx, int n, double* dA, int64_t lda, double* dB, in
                 "bad sizes for lu_solve");
     PSX_REQUIRE(dA && (dB || nrhs == 0), PSX_ERR_ARGUMENT, "null pointer");
     PSX_HIP(hipSetDevice(c->device));
-    lu_solve_dev(c, n, dA, lda, dB, ldb, nrhs);
+    lu_solve_dev(c, n, dA, lda, dB, ldb, nrhs, true);
   });
 }
 

@@ -351,8 +351,9 @@ void cov_layout(int kind, ContractRequest& rq, const double* const* W);
 // stream
 void dgemm_dev(Ctx* c, int m, int n, int k, const double* dA, int64_t lda, const double* dB,
                int64_t ldb, double* dC, int64_t ldc);
+// dA overwritten by LU; with keep_b a singular dA leaves dB as it was
 void lu_solve_dev(Ctx* c, int n, double* dA, int64_t lda, double* dB,
-                  int64_t ldb, int nrhs);  // dA overwritten by LU
+                  int64_t ldb, int nrhs, bool keep_b = false);
 void decouple_dev(Ctx* c, int n, double* dY, double* dB1, double* dB2, double* dT,
                   const std::function<void()>& b2);
 // One of several independent systems A X = B on the device (A overwritten by

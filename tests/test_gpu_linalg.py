@@ -378,3 +378,27 @@ def test_solve_many_right_hand_sides_at_block_edges(ctx, n, m):
     if n > 1 and m == n:
         Y = rng.uniform(-1, 1, (n, n))
         assert np.array_equal(ctx.decouple_covmat(Y, A, A), ctx.decouple_covmat(Y, A, A.copy()))
+
+
+@pytest.mark.parametrize("n,nrhs", [(5, 1), (40, 1), (300, 4), (700, 6), (6200, 2)])
+def test_lu_solve_d_leaves_the_right_hand_sides_of_a_singular_system(ctx, pkg, n, nrhs):
+    # a zero pivot is found before the right-hand sides change; padded leading
+    # dimensions, and sizes on either side of every row movement
+    rng = np.random.default_rng(n)
+    lda, ldb = n + 3, n + 5
+    A = np.zeros((lda, n), order="F")
+    A[:n] = rng.uniform(-1, 1, (n, n))
+    A[:n, n // 2] = 0.0
+    B = np.asfortranarray(rng.uniform(-1, 1, (ldb, nrhs)))
+    dA, dB = ctx.alloc(A.nbytes), ctx.alloc(B.nbytes)
+    try:
+        ctx.h2d(dA, A)
+        ctx.h2d(dB, B)
+        with pytest.raises(pkg.SingularException, match=f"position {n // 2 + 1} "):
+            ctx.check(ctx.lib.psx_lu_solve_d(ctx.handle, n, dA, lda, dB, ldb, nrhs), "lu_solve_d")
+        got = np.empty_like(B)
+        ctx.d2h(got, dB)
+        assert np.array_equal(got, B)
+    finally:
+        ctx.free(dA)
+        ctx.free(dB)
