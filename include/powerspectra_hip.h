@@ -179,7 +179,10 @@ int psx_mcm_set_d(psx_ctx* ctx, int lmin, int lmax, int64_t LW,
  * gives their counts.  Spectra and ratios are 0-based with length >= lmax+1,
  * W has length LW (reference: workspace.lmax+1).  Fills C[l1,l2] = C[l2,l1]
  * for lmin <= l1 <= l2 <= lmax.  `precision`: PSX_FP64, or PSX_MIXED /
- * PSX_FP64_MFMA through the matrix-core pass of psx_cov_batch (not TETE). */
+ * PSX_FP64_MFMA through the matrix-core pass of psx_cov_batch (not TETE).
+ * A negative product under a square root returns PSX_ERR_DOMAIN; C is then as
+ * it was, except that blocks of more than 32 MB in PSX_FP64, and those of
+ * psx_cov_d, are unspecified. */
 int psx_cov(psx_ctx* ctx, int kind, int lmin, int lmax,
             const double* const* spectra, const double* const* ratios,
             const double* const* W, int64_t LW, int precision,

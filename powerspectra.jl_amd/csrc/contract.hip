@@ -1163,8 +1163,8 @@ void run_contraction_to_host(Ctx* c, const ContractRequest& rq, double* const* h
     if (err) fetch_cov_flag(c, err);
     std::vector<D2HMatrix> whole;
     for (int k = 0; k < nout; ++k) whole.push_back({host[k], ldh, rq.dout[k], n, n, n});
-    d2h_matrices(c, whole.data(), nout);
-    if (err) check_cov_flag(c);
+    const std::function<void()> check = [&] { check_cov_flag(c); };
+    d2h_matrices(c, whole.data(), nout, err ? &check : nullptr);
     return;
   }
   // columns [j0, j1) of every output once the band completing them is done

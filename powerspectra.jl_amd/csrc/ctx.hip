@@ -534,7 +534,8 @@ bool small(const std::vector<Chunk>& ch) {
   return ch.size() == 1 && ch[0].bytes() <= kInlineBytes;
 }
 
-void d2h_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chunk>& ch) {
+void d2h_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chunk>& ch,
+                const std::function<void()>* landed) {
   const size_t n = ch.size();
   if (n == 0) return;
   st.grow((int)std::min<size_t>(n, Stage::kSlots));
@@ -566,6 +567,7 @@ void d2h_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chun
     }
     Stage::Slot& sl = at(k);
     PSX_HIP(hipEventSynchronize(sl.ev));
+    if (k == 0 && landed) (*landed)();
     const Chunk& x = ch[k];
     start_copy(sl, pool, inlined, x, true);
   }
@@ -609,7 +611,7 @@ void h2d_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chun
 }  // namespace
 
 void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatrix* m, int nm,
-                     int parts) {
+                     int parts, const std::function<void()>* landed) {
   std::vector<Chunk> ch;
   int64_t total = 0;
   for (int i = 0; i < nm; ++i)
@@ -618,12 +620,12 @@ void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatri
   for (int i = 0; i < nm; ++i)
     cut(ch, most, m[i].host, m[i].ldh, const_cast<double*>(m[i].dev), m[i].ldd, m[i].rows, m[i].cols,
         m[i].after);
-  d2h_chunks(s, stage, pool, ch);
+  d2h_chunks(s, stage, pool, ch, landed);
 }
 
-void d2h_matrices(Ctx* c, const D2HMatrix* m, int nm) {
+void d2h_matrices(Ctx* c, const D2HMatrix* m, int nm, const std::function<void()>* landed) {
   ensure_stage(c);
-  d2h_matrices_on(c->stream, c->stage, *c->pool, m, nm, kParts);
+  d2h_matrices_on(c->stream, c->stage, *c->pool, m, nm, kParts, landed);
 }
 
 void d2h_matrix(Ctx* c, double* host, int64_t ldh, const double* dev, int64_t ldd,

@@ -227,13 +227,16 @@ struct D2HMatrix {
   int64_t rows, cols;
   hipEvent_t after = nullptr;  // the copy waits for this event when set
 };
-void d2h_matrices(Ctx* c, const D2HMatrix* m, int nm);
+// (`landed`, if given, is called before the host memory is first written, when
+// everything enqueued on the context stream before the call is done)
+void d2h_matrices(Ctx* c, const D2HMatrix* m, int nm,
+                  const std::function<void()>* landed = nullptr);
 // the same on the context's copy stream, so that the pieces waiting for
 // events of the context stream copy out while later work there still runs
 void d2h_matrices_overlapped(Ctx* c, const D2HMatrix* m, int nm);
 // the same on stream s through the caller's slots, in about `parts` chunks
 void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatrix* m, int nm,
-                     int parts);
+                     int parts, const std::function<void()>* landed = nullptr);
 void h2d_matrix(Ctx* c, double* dev, int64_t ldd, const double* host, int64_t ldh,
                 int64_t rows, int64_t cols);
 // The same copy through the slots on the context's copy stream, behind earlier
@@ -338,8 +341,9 @@ size_t contraction_scratch_bytes(const ContractRequest& rq);
 // A contraction into packed device outputs (rq.ldo = n) followed by their
 // copy to the host blocks host[k] (leading dimension ldh).  Large outputs run
 // in l1 bands: the columns each band completes are copied out while the
-// later bands compute.  Returns with the host blocks complete; raises the
-// covariance domain error after the copy.
+// later bands compute.  Returns with the host blocks complete.  A covariance
+// domain error is raised before the host block is written, or after it where it
+// ran in bands.
 void run_contraction_to_host(Ctx* c, const ContractRequest& rq, double* const* host,
                              int64_t ldh);
 // request building shared by the entry points and the server

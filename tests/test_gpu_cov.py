@@ -91,3 +91,29 @@ def test_bad_arity(ctx, pkg):
     spec, rat, W = _inputs(0, lmax, lmax + 1)
     with pytest.raises(pkg.ArgumentError):
         ctx.cov(0, 0, lmax, spec, rat, W[:7])
+
+
+# results of one copied piece, of several chunks of a few slots, and of the
+# largest size that is computed in one launch
+@pytest.mark.parametrize("n", [7, 96, 700, 2047])
+def test_domain_error_leaves_the_result_untouched(ctx, pkg, n):
+    import ctypes
+    from importlib import import_module
+    abi = import_module(pkg.__name__ + "._abi")
+    lmax = n - 1
+    spec, rat, W = _inputs(0, lmax, lmax + 1)
+    spec[0] = spec[0].copy()
+    spec[0][lmax // 2] = -1.0
+    ptrs = lambda a, m: (abi._dp * m)(*([abi.dptr(x) for x in a]
+                                        + [ctypes.cast(None, abi._dp)] * (m - len(a))))
+    out = np.full((n, n), 7.25, order="F")
+    before = out.copy(order="F")
+    call = lambda s: ctx.lib.psx_cov(ctx.handle, 0, 0, lmax, ptrs(s, 4), ptrs(rat, 4), ptrs(W, 8),
+                                     W[0].size, 0, abi.dptr(out), n)
+    with pytest.raises(pkg.DomainError):
+        ctx.check(call(spec), "psx_cov")
+    assert np.array_equal(out, before)
+    # and the context goes on: the same call on good spectra
+    spec, rat, W = _inputs(0, lmax, lmax + 1)
+    ctx.check(call(spec), "psx_cov")
+    assert np.array_equal(out, ctx.cov(0, 0, lmax, spec, rat, W))
