@@ -338,7 +338,8 @@ contract_kernel(KArgs A) {
             e += (v - (sum - z)) + (x - z);
             v = sum;
           }
-          v += e;
+          // (infinite sums have no rounding error, only Inf - Inf)
+          v = isfinite(e) ? v + e : v;
           fin[k][rr] = v;
         }
       __syncthreads();

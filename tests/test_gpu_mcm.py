@@ -185,3 +185,20 @@ def test_cov_rows_at_split_edges(ctx, oracle, kind, n):
         ref = oracle.cov(kind, lmin, lmax, S[:nS], R[:nR], W, rows=(l1, l1))[l1 - lmin]
         e = rel_err(C[l1 - lmin], ref)
         assert e <= RTOL_FP64, (kind, n, l1, e)
+
+
+# on either side of the size where a tile's sum over c stops being split
+@pytest.mark.parametrize("n", [60, 300, 1600, 1601])
+@pytest.mark.parametrize("value", [np.inf, -np.inf])
+def test_infinite_W_reaches_its_pairs(ctx, n, value):
+    # every pair that the multipole l3 couples (|l1 - l2| <= l3 <= l1 + l2, even
+    # sum, so a nonzero 3j symbol) is infinite, in a block alone and in a set
+    l3 = 20
+    W = mask_like_W(n, seed=n)
+    W[l3] = value
+    l = np.arange(n)
+    l1, l2 = l[:, None], l[None, :]
+    hit = (np.abs(l1 - l2) <= l3) & (l1 + l2 >= l3) & ((l1 + l2 + l3) % 2 == 0)
+    assert (ctx.mcm(0, 0, n - 1, W)[hit] == value).all()
+    assert (ctx.mcm_set(0, n - 1, W, W, W, W)[0][hit] == value).all()
+    assert (ctx.mcm_batch(0, 0, n - 1, [W, W])[1][hit] == value).all()
