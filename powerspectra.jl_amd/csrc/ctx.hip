@@ -483,11 +483,15 @@ void wait_copied(const Stage::Slot& sl) {
 }
 
 // waits for every host copy of the stage, also when an error unwinds: they use
-// the caller's memory
+// the caller's memory.  An error leaves nothing in flight on the stream either,
+// since the device side may be the next call's.
 struct CopiesDone {
   Stage& st;
+  hipStream_t s;
+  const int errors = std::uncaught_exceptions();
   ~CopiesDone() {
     for (int i = 0; i < st.have; ++i) wait_copied(st.slot[i]);
+    if (std::uncaught_exceptions() > errors) (void)hipStreamSynchronize(s);
   }
 };
 
@@ -539,7 +543,7 @@ void d2h_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chun
   const size_t n = ch.size();
   if (n == 0) return;
   st.grow((int)std::min<size_t>(n, Stage::kSlots));
-  CopiesDone done{st};
+  CopiesDone done{st, s};
   const int ring = st.have, base = st.next;
   const bool inlined = small(ch);
   auto at = [&](size_t k) -> Stage::Slot& { return st.slot[(base + k) % ring]; };
@@ -578,7 +582,7 @@ void h2d_chunks(hipStream_t s, Stage& st, CopyPool& pool, const std::vector<Chun
   const size_t n = ch.size();
   if (n == 0) return;
   st.grow((int)std::min<size_t>(n, Stage::kSlots));
-  CopiesDone done{st};
+  CopiesDone done{st, s};
   const int ring = st.have, base = st.next;
   const bool inlined = small(ch);
   auto at = [&](size_t k) -> Stage::Slot& { return st.slot[(base + k) % ring]; };
