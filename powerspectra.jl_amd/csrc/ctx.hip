@@ -339,8 +339,8 @@ constexpr size_t kDirectBytes = size_t(16) << 10;
 CopyPool::CopyPool(int threads) {
   try {
     for (int i = 0; i < threads; ++i) threads_.emplace_back([this] { work(); });
-  } catch (const std::system_error&) {
-    // (as many as the process may have; with none, submit runs the tasks)
+  } catch (const std::exception&) {
+    // (as many as the process or its memory allow; with none, submit runs the tasks)
   }
 }
 

@@ -2,6 +2,17 @@
 // named by the first argument; 0 if it holds.
 #include "../../powerspectra.jl_amd/csrc/psx_internal.h"
 
+#include <new>
+
+static thread_local int new_fails_at = -1;   // the n-th allocation from now fails
+void* operator new(size_t n) {
+  if (new_fails_at >= 0 && new_fails_at-- == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 namespace psx {
 void release_blas(Ctx*) {}
 void release_tile_cache(Ctx*) {}
@@ -79,10 +90,32 @@ static bool nothing_in_flight_after_an_error() {
   return ok;
 }
 
+// a pool that cannot have all its threads works with those it has; one that
+// cannot be made at all is an error, not the end of the process
+static bool pool_without_memory() {
+  int made = 0;
+  for (int at = 0; at < 40; ++at) {
+    std::unique_ptr<CopyPool> p;
+    try {
+      new_fails_at = at;
+      p = std::make_unique<CopyPool>(8);
+    } catch (const std::bad_alloc&) {
+    }
+    new_fails_at = -1;
+    if (!p) continue;
+    ++made;
+    std::atomic<int> done{0};
+    for (int i = 0; i < 20; ++i) p->submit([&] { ++done; });
+    while (done < 20) std::this_thread::yield();
+  }
+  return made > 30;
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "round_trips") return round_trips() ? 0 : 1;
   if (which == "nothing_in_flight_after_an_error")
     return nothing_in_flight_after_an_error() ? 0 : 1;
+  if (which == "pool_without_memory") return pool_without_memory() ? 0 : 1;
   return 2;
 }

@@ -23,6 +23,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["round_trips", "nothing_in_flight_after_an_error"])
+@pytest.mark.parametrize("case", ["round_trips", "nothing_in_flight_after_an_error",
+                                  "pool_without_memory"])
 def test_host_copies(program, case):
     assert subprocess.run([program, case], timeout=120).returncode == 0
