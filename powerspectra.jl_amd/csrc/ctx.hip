@@ -74,7 +74,15 @@ HeldBuf::HeldBuf(Ctx* cc, CachedSlot& s, size_t bytes) : c(cc), slot(&s) {
   cap = bytes;
 }
 
-HeldBuf::~HeldBuf() { slot->busy = false; }
+HeldBuf::~HeldBuf() {
+  // after an error nothing may still be queued on the buffer, the next call's, or
+  // on host memory that the failed call was given
+  if (std::uncaught_exceptions() > errors) {
+    (void)hipStreamSynchronize(c->stream);
+    if (c->xstream) (void)hipStreamSynchronize(c->xstream);
+  }
+  slot->busy = false;
+}
 
 double* HeldBuf::take(size_t bytes) {
   const size_t at = (used + 255) & ~size_t(255);

@@ -7,6 +7,7 @@
 #include <condition_variable>
 #include <cstdint>
 #include <deque>
+#include <exception>
 #include <functional>
 #include <initializer_list>
 #include <map>
@@ -163,6 +164,7 @@ struct HeldBuf {
   Ctx* c;
   CachedSlot* slot;
   size_t cap = 0, used = 0;
+  const int errors = std::uncaught_exceptions();
   HeldBuf(Ctx* cc, CachedSlot& s, size_t bytes);
   ~HeldBuf();
   HeldBuf(const HeldBuf&) = delete;

@@ -90,6 +90,28 @@ static bool nothing_in_flight_after_an_error() {
   return ok;
 }
 
+// nor does an error in a call that has its device buffer filled: what is queued
+// reads the caller's memory and writes the buffer
+static bool nothing_in_flight_when_a_buffer_is_given_back() {
+  bool ok = true;
+  for (int x = 0; x < 2; ++x) {
+    Ctx* c = context();
+    ensure_stage(c);
+    const std::vector<double> a = numbers(1000, 1.0);
+    try {
+      XferBuf buf(c, sizeof(double) * a.size());
+      double* d = buf.take(sizeof(double) * a.size());
+      PSX_HIP(hipMemcpyAsync(d, a.data(), sizeof(double) * a.size(), hipMemcpyHostToDevice,
+                             x ? c->xstream : c->stream));
+      PSX_REQUIRE(false, PSX_ERR_ARGUMENT, "an error");
+    } catch (const Error&) {
+    }
+    ok = ok && c->stream->ops.empty() && c->xstream->ops.empty();
+    ok = ok && psx_ctx_destroy((psx_ctx*)c) == PSX_OK;
+  }
+  return ok;
+}
+
 // a pool that cannot have all its threads works with those it has; one that
 // cannot be made at all is an error, not the end of the process
 static bool pool_without_memory() {
@@ -116,6 +138,8 @@ int main(int argc, char** argv) {
   if (which == "round_trips") return round_trips() ? 0 : 1;
   if (which == "nothing_in_flight_after_an_error")
     return nothing_in_flight_after_an_error() ? 0 : 1;
+  if (which == "nothing_in_flight_when_a_buffer_is_given_back")
+    return nothing_in_flight_when_a_buffer_is_given_back() ? 0 : 1;
   if (which == "pool_without_memory") return pool_without_memory() ? 0 : 1;
   return 2;
 }

@@ -24,6 +24,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["round_trips", "nothing_in_flight_after_an_error",
+                                  "nothing_in_flight_when_a_buffer_is_given_back",
                                   "pool_without_memory"])
 def test_host_copies(program, case):
     assert subprocess.run([program, case], timeout=120).returncode == 0
