@@ -324,8 +324,8 @@ int psx_memcpy_d2h(psx_ctx* h, void* dst, const void* src, size_t bytes) {
 
 // ---- staged host copies ---------------------------------------------------
 // Copies between device memory and pageable host memory run far below PCIe
-// speed (a 2-D one goes row by row: 660 us for a 96 x 96 block), so all go
-// through a ring of pinned slots: the DMA runs ahead in some while host threads
+// speed (a 2-D one goes row by row: 660 us for a 96 x 96 block), so all but short
+// ranges go through a ring of pinned slots: the DMA runs ahead in some while host threads
 // copy others, a chunk split between several threads, which also fault in a
 // fresh destination's pages.  Chunks are an eighth of the transfer, at most a
 // slot (12 MB, 220 us at 57 GB/s: 2 MB chunks lost 20 % of that rate between
@@ -339,9 +339,14 @@ constexpr size_t kChunkBytes = size_t(1) << 20;
 constexpr int kParts = 8;                           // chunks of a transfer, where they fit
 constexpr size_t kTaskBytes = size_t(768) << 10;    // of a chunk, per task
 constexpr size_t kInlineBytes = size_t(256) << 10;  // copied by the caller itself
-// one piece up to this goes to the runtime as it is, which copies it at once: a slot,
-// its event and the pinned copy take 6 us more
-constexpr size_t kDirectBytes = size_t(16) << 10;
+// One range up to kDirectBytes goes to the runtime as it is, out of the device from
+// kDirectOutBytes on: a slot, its event and the pinned copy take 10 us more in (the
+// alms of alm2map and alm2cl, 160 bytes to 730 KB: 58 -> 40, 111 -> 86, 152 -> 118 and
+// 211 -> 160 us a call) and a pool thread's wake-up and copy up to 40 out (maps of 98
+// and 393 KB: 77 -> 62, 133 -> 93 us).  Smaller results measure alike or better from a
+// slot; above 1 MB the slots' copies overlap their DMAs.
+constexpr size_t kDirectBytes = size_t(1) << 20;
+constexpr size_t kDirectOutBytes = size_t(64) << 10;
 }  // namespace
 
 CopyPool::CopyPool(int threads) {
@@ -632,6 +637,12 @@ void d2h_matrices_on(hipStream_t s, Stage& stage, CopyPool& pool, const D2HMatri
   for (int i = 0; i < nm; ++i)
     cut(ch, most, m[i].host, m[i].ldh, const_cast<double*>(m[i].dev), m[i].ldd, m[i].rows, m[i].cols,
         m[i].after);
+  if (ch.size() == 1 && ch[0].nc == 1 && !ch[0].after && !landed &&
+      ch[0].bytes() > kDirectOutBytes && ch[0].bytes() <= kDirectBytes) {
+    PSX_HIP(hipMemcpyAsync(ch[0].host, ch[0].dev, ch[0].bytes(), hipMemcpyDeviceToHost, s));
+    PSX_HIP(hipStreamSynchronize(s));
+    return;
+  }
   d2h_chunks(s, stage, pool, ch, landed);
 }
 
@@ -657,6 +668,10 @@ void h2d_matrix_on(Ctx* c, hipStream_t s, double* dev, int64_t ldd, const double
   std::vector<Chunk> ch;
   cut(ch, chunk_doubles(std::max<int64_t>(rows, 0) * std::max<int64_t>(cols, 0)),
       const_cast<double*>(host), ldh, dev, ldd, rows, cols, nullptr);
+  if (ch.size() == 1 && ch[0].nc == 1 && ch[0].bytes() <= kDirectBytes) {
+    PSX_HIP(hipMemcpyAsync(dev, host, ch[0].bytes(), hipMemcpyHostToDevice, s));
+    return;
+  }
   h2d_chunks(s, c->stage, *c->pool, ch);
 }
 }  // namespace

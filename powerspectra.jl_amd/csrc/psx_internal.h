@@ -215,9 +215,11 @@ void alm2map_pol_dev(Ctx* c, int nside, int lmax, int nmaps, const double* dteb,
 
 // Column-major matrix copies between host memory (any pageable buffer,
 // leading dimension ldh) and device memory (leading dimension ldd), in
-// stream order on the context stream, through the context's pinned slots.
-// d2h returns when the host side is complete; h2d returns when the host
-// buffer has been read (the device side is complete in stream order).
+// stream order on the context stream, through the context's pinned slots (short
+// ranges by the runtime's own copy).  d2h returns when the host side is
+// complete; h2d returns when the host buffer has been read, or for a short
+// range in pinned memory is read in stream order (the device side is complete
+// in stream order).
 void d2h_matrix(Ctx* c, double* host, int64_t ldh, const double* dev, int64_t ldd,
                 int64_t rows, int64_t cols);
 // several matrices through one pipeline (the DMA does not drain between them)

@@ -39,6 +39,7 @@ static bool round_trips() {
   Ctx* c = context();
   bool ok = true;
   const int64_t shapes[][3] = {{1, 1, 1}, {7, 5, 9}, {300, 300, 300}, {1000, 900, 1001},
+                               {8192, 1, 8192}, {8193, 1, 8193}, {512, 256, 512}, {131073, 1, 131073},
                                {5000000, 1, 5000000}, {2000000, 4, 2000003}};
   for (auto& s : shapes)
     for (int x = 0; x < 4; ++x) {

@@ -257,3 +257,32 @@ def test_work_buffer_yields_to_allocations(pkg):
         assert np.array_equal(ctx.mask_spectra(maps, nside, lmax), cl)
     finally:
         ctx.close()
+
+
+# either side of the sizes from which (64 KB) and up to which (1 MB) a single
+# range is the runtime's own copy: n^2 doubles out, (lmax + 1)(lmax + 2) in
+@pytest.mark.parametrize("n,lmax", [(90, 89), (91, 90), (362, 360), (363, 361)])
+def test_ranges_at_the_edges_of_the_direct_copies(ctx, n, lmax):
+    W = mask_like_W(n, seed=n)
+    dW, dM = ctx.alloc(W.nbytes), ctx.alloc(8 * n * n)
+    try:
+        ctx.h2d(dW, W)
+        ctx.check(ctx.lib.psx_mcm_d(ctx.handle, 0, 0, n - 1, dW, W.size, dM, n), "mcm_d")
+        ref = np.empty((n, n), order="F")
+        ctx.d2h(ref, dM)
+    finally:
+        ctx.free(dW)
+        ctx.free(dM)
+    out = np.full((n, n), np.nan, order="F")
+    assert np.array_equal(ctx.mcm(0, 0, n - 1, W, out), ref) and np.array_equal(out, ref)
+    # small whole numbers, whose products and sums are exact in any order
+    na = (lmax + 1) * (lmax + 2) // 2
+    rng = np.random.default_rng(n)
+    a = rng.integers(-9, 10, (2, na)) + 1j * rng.integers(-9, 10, (2, na))
+    got = np.asarray(ctx.alm2cl([a[0], a[1]], lmax)).reshape(2, 2, lmax + 1)
+    m = np.concatenate([np.full(lmax + 1 - k, k) for k in range(lmax + 1)])
+    l = np.concatenate([np.arange(k, lmax + 1) for k in range(lmax + 1)])
+    p = (a[0].real * a[1].real + a[0].imag * a[1].imag) * np.where(m == 0, 1, 2)
+    s = np.bincount(l, weights=p, minlength=lmax + 1)
+    ref = s / (2 * np.arange(lmax + 1) + 1)
+    assert np.abs(got[0, 1] - ref).max() <= 4 * np.finfo(float).eps * np.abs(ref).max()
