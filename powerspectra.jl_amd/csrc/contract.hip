@@ -339,7 +339,7 @@ contract_kernel(KArgs A) {
             v = sum;
           }
           // (infinite sums have no rounding error, only Inf - Inf)
-          v = isfinite(e) ? v + e : v;
+          v += e == e ? e : 0.0;
           fin[k][rr] = v;
         }
       __syncthreads();
