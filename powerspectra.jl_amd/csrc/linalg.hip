@@ -266,8 +266,8 @@ __global__ void __launch_bounds__(kLuRows) lu_leaf_col(double* A, int64_t lda, i
 // to 34 us a 16-column one of 2048 to 3072, 19 to 25 us an 8-column one of 4096
 // to 6144: 1.4 to 3.1 us a column, against 2.6 to 3.7 with 1024 threads and all
 // columns unrolled, and 5.7 for a launch per column above 3072 rows.  Bound by the
-// instructions a row takes, 31 vector and 29 scalar ones with a mask for the rows
-// still live (28 us at 6144 rows), and by a column's chain of steps below that.
+// instructions a row takes (28 us at 6144 rows with a mask for the rows still live,
+// 25 with zeros in their place), and by a column's chain of steps below that.
 // Device solves: n = 2509 13.7 -> 7 ms, n = 6144 45.9 -> 26 ms.
 constexpr int kLuWgThreads = 512;
 constexpr int kLuWgWaves = kLuWgThreads / 64;
@@ -432,10 +432,12 @@ __device__ __forceinline__ void lu_wg_stage(double (&vals)[NR][W], unsigned& gon
         }
     }
     double* a = A + (int64_t)(c + j) * lda + c + t;
-    // quotients by the rounded reciprocal with one residual correction: the
-    // correctly rounded quotient (|value| <= |pivot|); pivots whose reciprocal
-    // could leave the normal range are divided by, and under a zero pivot the
-    // column (all zeros) is left as it is
+    // quotients by the rounded reciprocal with one residual correction (|value| <=
+    // |pivot|): the first is off by 2^-52 of itself at most, the correction's own
+    // error is 2^-52 of that, so the sum before its rounding is the quotient to some
+    // 2^-103 and the result is within half an ulp and a little; pivots whose
+    // reciprocal could leave the normal range are divided by, and under a zero pivot
+    // the column (all zeros) is left as it is
     double l[NR];
     if (__builtin_amdgcn_ballot_w64(fabs(piv) > 0x1p-1000 && fabs(piv) < 0x1p1000)) {
       const double rp = 1.0 / piv;
@@ -823,7 +825,7 @@ __global__ void __launch_bounds__(64 * kTsmWaves) trsm_block(const double* __res
     plain &= fabs(d[s]) > 0x1p-1000 && fabs(d[s]) < 0x1p1000;
   }
   // every pivot's reciprocal in the normal range: quotients by it, with one
-  // residual correction (the correctly rounded quotient)
+  // residual correction (good to half an ulp and a little, as in lu_wg_stage)
   const bool fast = __builtin_amdgcn_ballot_w64(!plain) == 0;
   // sets of kTsmAhead columns, from the first (lower) or last (upper) that
   // holds one of the block; a thread stages kTsmStage of a set's entries in

@@ -12,9 +12,9 @@
 //      combined over the north/south ring pair into F+ = F_N + F_S and
 //      F- = F_N - F_S (lambda_lm(-z) = (-1)^{l+m} lambda_lm(z)).
 //   3. Legendre sums a_lm = (4 pi / Npix) sum_pairs lambda_lm(z) F+-(m), one
-//      workgroup per (m, chunk of 1024 ring pairs), the sum over rings
-//      reduced through LDS in rounds of 8 l, partial sums per chunk added by
-//      a second kernel.
+//      workgroup per (m, chunk of up to 2048 ring pairs), the sum over a wave's
+//      rings formed on the matrix cores in rounds of 8 values of l and map, the
+//      waves' sums added through LDS, partial sums per chunk by a second kernel.
 // Synthesis runs the same steps backwards (one thread per ring pair
 // accumulating over l, no reduction), and map2alm refines with `niter` Jacobi
 // iterations a += A(map - S(a)) as Healpix.jl does.
@@ -720,9 +720,9 @@ __device__ __forceinline__ void lds_barrier() {
 // P independent recurrences; per round of LC l values the 16 sums of every (l,
 // map, re/im) over the pairs are formed in the same order whatever the group size
 // (one map alone gives the same sums).  Bound by latency at two waves a SIMD (the
-// coefficients of P pairs fill the registers) and by the FP64 units, half busy:
-// nside 1024, lmax 3071, 2 maps 4.15 -> 3.7 ms against sums through LDS with weights
-// on every step, nside 512, lmax 1535 645 -> 595 us; with P = 4 4.4 ms.
+// coefficients of P pairs fill the registers) and by the FP64 units, 58 % busy:
+// nside 1024, lmax 3071, 2 maps 4.2 -> 3.5 ms against sums through LDS with weights
+// on every step, nside 512, lmax 1535 675 -> 600 us; P = 4 takes 1.2 times as long.
 template <int NM, int P, int T>
 __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(2)))
 legendre_analysis(LegArgs A, MapPtrs<NM> M) {
@@ -901,7 +901,7 @@ inline int64_t g_elems(int lmax, int nr) {
 }
 
 // ring pairs per synthesis thread: fewer for larger groups (per pair and map, four
-// accumulators; 4 maps of 2048 pairs, lmax 3071: 4.1 ms with 2, 4.7 with 4)
+// accumulators; 4 maps of 2048 pairs, lmax 3071: 3.9 ms with 2, 1.15 times that with 4)
 __host__ __device__ constexpr int syn_pairs(int nm) { return nm <= 2 ? 4 : 2; }
 
 // Synthesis: G_q[m][k] = sum_l a_q,lm lambda_lm(z_k) for SP ring pairs per
@@ -909,9 +909,9 @@ __host__ __device__ constexpr int syn_pairs(int nm) { return nm <= 2 ? 4 : 2; }
 // even - odd); a_lm s_lm and the recurrence coefficients are uniform across the
 // workgroup and read with scalar loads, kSynChunk at a time ahead of the
 // steps that use them.  Bound by the FP64 units (70 % busy at a clock that falls to
-// 2.06 GHz under them): nside 1024, lmax 3071, 4 maps 5.8 -> 4.1 ms against the
+// 2.06 GHz under them): nside 1024, lmax 3071, 4 maps 5.8 -> 3.9 ms against the
 // unnormalised recurrence with weights on every step; a second set of scalars,
-// loaded a round ahead, gave 4.3 ms.
+// loaded a round ahead, took 5 % longer.
 template <int NM>
 __global__ void __launch_bounds__(256)
 legendre_synthesis(LegArgs A, const double2* __restrict__ coef, const int* __restrict__ odd,
@@ -1145,7 +1145,7 @@ void launch_fold_synthesis(const Rings& R, hipStream_t s, RingArgs ra, const dou
 // of the m m' = -+2m term); run separately, each keeps full relative
 // precision, while a recurrence on lambda+- directly loses the small one near
 // the pole.
-constexpr int kLChunk2 = 4;                 // l values per LDS round, spin 2
+constexpr int kLChunk2 = 4;                 // l values per round, spin 2
 
 struct PolArgs {
   RingArgs R;
@@ -1392,7 +1392,7 @@ legendre_analysis_s2(PolArgs A, const double2* __restrict__ F, int64_t fs,
 
 // Ring pairs per spin-2 analysis thread: 4, fewer where 256 threads of 4 would
 // outnumber the pairs (512 pairs, lmax 767: 228 us with 4, 177 with 2); with 2 at
-// 2048 pairs, lmax 3071 it takes 7.8 ms instead of 6.7.
+// 2048 pairs, lmax 3071 it takes 1.16 times the 6.1 ms of 4.
 inline int an2_pairs(int npairs) { return npairs > 512 ? 4 : npairs > 256 ? 2 : 1; }
 
 // Spin-2 synthesis: GQ[m][k], GU[m][k] = Q_m, U_m of every ring, kSyn2Pairs
@@ -1918,7 +1918,7 @@ void launch_synthesis(ShtPlan& P, hipStream_t s, const ShtBufs* B, const double2
 }
 
 // maps per analysis pass (the analysis holds each map's F+- of its ring pairs
-// in registers and reduces 2 values per map and l through LDS)
+// in registers; a round of 16 sums is 8 l of one map or 4 l of two)
 constexpr int kAnGroup = 2;
 
 // alms[q] (+)= A(maps[q]) for a group of nm <= kMaxGroup maps: Legendre passes
