@@ -281,7 +281,8 @@ int psx_lu_factor(psx_ctx* ctx, int n, const double* A, int64_t lda, double* LU,
  * Replaces Healpix.jl's map2alm as called by mcm(spec, mask1, mask2) and the
  * covariance workspace (reference src/modecoupling.jl:250-251,
  * src/workspace.jl:155,163).  nside a power of two <= 2048,
- * lmax <= min(4 nside, 8191). */
+ * lmax <= min(4 nside, 8191).  Values within a factor 128 of the largest
+ * double may overflow inside a transform, here and below. */
 int psx_map2alm(psx_ctx* ctx, int nside, int lmax, int niter, int nmaps,
                 const double* maps, double* alms);
 /* Synthesis (Healpix.jl alm2map): the inverse of one analysis step. */

@@ -181,8 +181,10 @@ void execute(Server* S, Slot* sl, Job& j) {
   if (j.host_out) {
     D2HMatrix m[5];
     for (int k = 0; k < j.nout; ++k) m[k] = {j.rq.out[k], j.rq.ld, outs[k], n, n, n};
-    // (few chunks: the slots' copies already overlap each other; a burst of 24
-    // requests of lmax 511 to 1535 takes 4.2 ms with 4 chunks each, 4.45 with 8)
+    // (few chunks: one slot's DMA overlaps the others' host copies already, so a
+    // result need only be cut enough for its own, and each chunk costs an event and
+    // a wake-up; a burst of 24 requests of lmax 511 to 1535 takes 4.2 ms with 4
+    // chunks each, 4.45 with 8)
     d2h_matrices_on(sl->stream, sl->stage, *S->ctx->pool, m, j.nout, 4);
   }
 }
